@@ -46,11 +46,14 @@ const char* const kKernelNames[] = {
     "fs_local_deferred_k64", "fs_onesweep_loop_k64", "fs_local_deferred_k32", "fs_local_k32_w",
     "fs_local_deferred_k32_w", "fs_local_k64_w", "fs_local_deferred_k64_w", "fs_onesweep_k32_s",
     "fs_onesweep_any_k32_s", "fs_onesweep_k32_vs", "fs_onesweep_k64_s", "fs_onesweep_any_k64_s", "fs_onesweep_k64_vs",
+    "fs_split_k32", "fs_split_k64", "fs_part_k32", "fs_part_k32_v", "fs_part_k64", "fs_part_k64_v", "fs_bucket_k32",
+    "fs_bucket_k32_v", "fs_bucket_k64", "fs_bucket_k64_v",
 };
 enum {
     K_UP32, K_UP64, K_OS32, K_OS32V, K_OS64, K_OS64V, K_IOTA, K_ANY32, K_ANY64, K_SCRATCH_ADDR, K_FIRST32, K_FIRST64,
     K_SAMPLE32, K_SAMPLE64, K_LOCAL32, K_RESCATTER32, K_RESCATTER64, K_LOCAL64, K_DEFER64, K_LOOP64, K_DEFER32,
     K_LOCAL32W, K_DEFER32W, K_LOCAL64W, K_DEFER64W, K_OS32S, K_ANY32S, K_OS32VS, K_OS64S, K_ANY64S, K_OS64VS,
+    K_SPLIT32, K_SPLIT64, K_PART32, K_PART32V, K_PART64, K_PART64V, K_BUCKET32, K_BUCKET32V, K_BUCKET64, K_BUCKET64V,
     K_COUNT
 };
 // the stable digit-pass kernel and the keys-only first-pass kernel of each variant (FS_VAR_*)
@@ -71,6 +74,10 @@ struct fs_sorter {
     // [wide][64-bit keys] (fs_local_k32, fs_local_k64, fs_local_k32_w, fs_local_k64_w)
     uint32_t local_keys[2][2] = {};
     uint32_t local_block[2][2] = {};
+    // bucket path: threads per block, keys per tile of the partition by
+    // [64-bit keys], keys a block sorts by [64-bit keys][values], most samples
+    // and most buckets
+    uint32_t bk_block = 0, bk_part_block = 0, bk_split_block = 0, bk_tile[2] = {}, bk_cap[2][2] = {}, bk_samples = 0, bk_max = 0;
     uint32_t local_min_bits32 = 8;  // fewest segment bits whose 32-bit segments fs_local_k32 sorts itself
     int num_cus = 256;
 
@@ -82,6 +89,7 @@ struct fs_sorter {
     uint32_t* rtable = nullptr;     // [FS_RTABLE_WORDS] region bases, total and caps of the fused pass
     uint32_t* plan = nullptr;       // u32[FS_PLAN_WORDS] device-side schedule
     uint32_t* segc = nullptr;       // u32[FS_SEGC_WORDS] segment counters and deferred-segment list of the top-16 path
+    uint32_t* bk_tab = nullptr;     // u32[FS_BK_TAB_WORDS] bucket table
     uint32_t* status = nullptr;     // pinned host word written by kernels on device errors
     unsigned long long* stats = nullptr;   // device u64[FS_STAT_COUNT]
     bool stats_on = false;
@@ -101,6 +109,8 @@ struct fs_sorter {
     uint32_t fused_mode = 0;             // FS_TEST_FUSED: 0 by size, 1 never, 2 always
     uint32_t top16_mode = 0;             // FS_TEST_TOP16: 0 by size, 1 never, 2 always (even skewed), 3 sampled
     uint32_t seg_bits = 0;               // FS_TEST_SEG_BITS: 0 by size, else the segment bits
+    uint32_t bucket_mode = 0;            // FS_TEST_BUCKETS: 0 by size, 1 never, 2 always one block, 3 always buckets
+    uint32_t bucket_lnb = 0;             // ... log2 of the buckets (0: by size)
     uint32_t local_wide_mode = 0;        // FS_TEST_LOCAL_WIDE: 0 by size, 1 wide local-sort blocks
     // the last sort's schedule (the sorter's, or the static scratch's) and
     // whether it began with the fused first pass
@@ -361,6 +371,67 @@ static bool top16_path(const fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) 
     return n >= (key64(t) ? FS_TOP16_MIN_KEYS64 : FS_TOP16_MIN_KEYS32) && n <= (local_mean_max(s, t, true) << 16);
 }
 
+// The bucket path (bucket_sort.h): sorts that one block does by itself in one
+// launch, and those that a sample, a partition and a block per bucket do in
+// three, where the digit passes take one launch per digit and one more.
+enum BucketPath { BK_NONE, BK_ONE_BLOCK, BK_BUCKETS };
+struct BucketLimit {
+    uint64_t one_block, buckets;
+};
+static BucketLimit bucket_limit(fs_op op, fs_key_type t) {
+    const bool v = op != FS_OP_SORT;
+    if (key64(t))
+        return v ? BucketLimit{FS_BK_ONE_64V, FS_BK_MAX_64V} : BucketLimit{FS_BK_ONE_64, FS_BK_MAX_64};
+    return v ? BucketLimit{FS_BK_ONE_32V, FS_BK_MAX_32V} : BucketLimit{FS_BK_ONE_32, FS_BK_MAX_32};
+}
+static BucketPath bucket_path(const fs_sorter* s, fs_op op, fs_key_type t, uint64_t n, bool no_alloc) {
+    if (n < 2 || n >= (1ull << 31)) return BK_NONE;
+    const uint32_t cap = s->bk_cap[key64(t) ? 1 : 0][op != FS_OP_SORT ? 1 : 0];
+    if (s->bucket_mode == 2u) return n <= cap ? BK_ONE_BLOCK : BK_NONE;
+    if (s->bucket_mode == 3u) return no_alloc || n < 64 ? BK_NONE : BK_BUCKETS;
+    // (the other test options ask for the paths that they are about)
+    if (s->bucket_mode == 1u || s->fused_mode || s->top16_mode || s->force_wide || s->up_blocks_per_cu || s->stats_on ||
+        s->fault != FS_FAULT_NONE)
+        return BK_NONE;
+    const BucketLimit lim = bucket_limit(op, t);
+    if (n <= lim.one_block && n <= cap) return BK_ONE_BLOCK;
+    return !no_alloc && n <= lim.buckets ? BK_BUCKETS : BK_NONE;
+}
+
+// log2 of the buckets (about FS_BK_MEAN keys each) and of the samples (16 to a
+// bucket), and the keys S1 holds for the buckets' regions: the sample's
+// estimate plus its room, largest when every bucket has the same share.
+struct BucketShape {
+    uint32_t lnb, lm, tile, tiles;
+    uint64_t s1_keys;
+};
+static BucketShape bucket_shape(const fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
+    BucketShape b;
+    b.lnb = 3;
+    while ((1u << (b.lnb + 1)) <= s->bk_max && n > ((uint64_t)FS_BK_MEAN << b.lnb)) ++b.lnb;
+    if (s->bucket_lnb) b.lnb = s->bucket_lnb;
+    while ((1u << b.lnb) > s->bk_max) --b.lnb;
+    // samples per bucket: with s of them a bucket outgrows r times its mean
+    // with probability P(Poisson(r s) < s), below 2e-6 for 4 samples and r =
+    // 5.3, 8 and 3.6, 16 and 2.7 (the block of such a bucket then takes long,
+    // but the sort stays exact)
+    const uint32_t cap = s->bk_cap[key64(t) ? 1 : 0][op != FS_OP_SORT ? 1 : 0];
+    const double ratio = (double)cap * (double)(1u << b.lnb) / (double)n;
+    b.lm = b.lnb + (ratio >= 5.3 ? 2 : ratio >= 3.6 ? 3 : ratio >= 2.7 ? 4 : 5);
+    if (b.lm < 9) b.lm = 9;
+    while ((1u << b.lm) > s->bk_samples) --b.lm;
+    // a tile per CU where the keys suffice, of 1 to all of the partition's keys per thread
+    const uint32_t most = s->bk_tile[key64(t) ? 1 : 0] / s->bk_part_block;
+    uint64_t rows = n / ((uint64_t)s->bk_part_block * (uint64_t)s->num_cus) + 1;
+    if (rows > most) rows = most;
+    b.tile = (uint32_t)rows * s->bk_part_block;
+    b.tiles = (uint32_t)((n + b.tile - 1) / b.tile);
+    const double nb = (double)(1u << b.lnb), m = (double)(1u << b.lm);
+    b.s1_keys = (uint64_t)((double)n / m * (m + 6.0 * __builtin_sqrt(m * nb) + (double)FS_BK_ROOM * nb) * 1.01 + 32.0 * nb);
+    if (b.s1_keys < n) b.s1_keys = n;
+    return b;
+}
+
 // The digit-pass variant a sort runs: by key width and op, and its small
 // tiles (FS_VAR_K32S ... FS_VAR_K64VS) below FS_SMALL_TILE_KEYS (32-bit keys)
 // or FS_SMALL_TILE_KEYS64 (64-bit keys) keys on the LSD passes (the fused and
@@ -397,6 +468,18 @@ static uint32_t seg_bits_for(uint64_t n, uint64_t mean_max) {
 static fs_status reserve(fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
     if (n <= 1) return FS_OK;
     const size_t kb = key_bytes(t);
+    const BucketPath bp = bucket_path(s, op, t, n, false);
+    if (bp == BK_ONE_BLOCK) return FS_OK;
+    if (bp == BK_BUCKETS) {
+        const BucketShape b = bucket_shape(s, op, t, n);
+        fs_status r;
+        if ((r = ensure(s, s->s1k, b.s1_keys * kb)) != FS_OK) return r;
+        if ((r = ensure(s, s->s2k, n * kb)) != FS_OK) return r;
+        if (op == FS_OP_SORT) return FS_OK;
+        if ((r = ensure(s, s->s1v, b.s1_keys * 4)) != FS_OK) return r;
+        if ((r = ensure(s, s->s2v, n * 4)) != FS_OK) return r;
+        return ensure(s, s->lb0, ((size_t)b.tiles + (b.tiles + FS_LB_GROUP - 1) / FS_LB_GROUP) * s->bk_max * 4);
+    }
     const uint32_t tile = s->tile[sort_variant(s, op, t, n, false)];
     const uint64_t num_tiles = (n + tile - 1) / tile;
     fs_status r;
@@ -438,6 +521,57 @@ static ScratchSet static_scratch(const fs_sorter* s) {
                       p + FS_NA_OFF_RTABLE, 0};   // (no top-16 path on the static scratch)
 }
 
+// The launches of the bucket path.
+static fs_status enqueue_buckets(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint32_t* vals, uint64_t n,
+                                 hipStream_t st, BucketPath bp, bool no_alloc) {
+    fs_status r;
+    if (bp == BK_BUCKETS && (r = reserve(s, op, t, n)) != FS_OK) return r;
+    const ScratchSet sc = no_alloc ? static_scratch(s) : sorter_scratch(s);
+    const bool v = op != FS_OP_SORT, k64 = key64(t);
+    FsArgs a;
+    memset(&a, 0, sizeof a);
+    a.n = n;
+    a.key64 = k64 ? 1u : 0u;
+    a.xform = xform_of(t);
+    a.op = op == FS_OP_SORT ? FSK_OP_KEYS : (op == FS_OP_ARGSORT ? FSK_OP_ARGSORT : FSK_OP_PAIRS);
+    a.digits = k64 ? 8u : 4u;
+    a.keys = (uint64_t)(uintptr_t)keys;
+    a.vals = (uint64_t)(uintptr_t)vals;
+    a.plan = sc.plan;
+    a.status = (uint64_t)(uintptr_t)s->status;
+    a.bk_tab = (uint64_t)(uintptr_t)s->bk_tab;
+    void* args[] = {&a};
+    const int kbucket = k64 ? (v ? K_BUCKET64V : K_BUCKET64) : (v ? K_BUCKET32V : K_BUCKET32);
+    if (bp == BK_ONE_BLOCK) {
+        if ((r = launch(s, kbucket, 1, s->bk_block, args, st, no_alloc)) != FS_OK) return r;
+    } else {
+        const BucketShape b = bucket_shape(s, op, t, n);
+        a.s1k = sc.s1k;
+        a.s1v = sc.s1v;
+        a.s2k = sc.s2k;
+        a.s2v = sc.s2v;
+        a.lookback0 = sc.lb0;
+        a.num_tiles = b.tiles;
+        a.tile = b.tile;
+        a.s1_keys = (uint32_t)b.s1_keys;
+        a.bk_lnb = b.lnb;
+        a.bk_lm = b.lm;
+#ifdef FS_FAULT_INJECTION
+        a.fault = s->fault;
+#endif
+        const int kpart = k64 ? (v ? K_PART64V : K_PART64) : (v ? K_PART32V : K_PART32);
+        if ((r = launch(s, k64 ? K_SPLIT64 : K_SPLIT32, 1, s->bk_split_block, args, st)) != FS_OK) return r;
+        if ((r = launch(s, kpart, b.tiles, s->bk_part_block, args, st)) != FS_OK) return r;
+        if ((r = launch(s, kbucket, 1u << b.lnb, s->bk_block, args, st)) != FS_OK) return r;
+    }
+    s->last_stream = st;
+    s->pending = true;
+    s->last_plan = (uint32_t*)(uintptr_t)sc.plan;
+    s->last_fused = false;
+    s->last_top16 = false;
+    return FS_OK;
+}
+
 // no_alloc: the sort runs on the static scratch (fs_encode_no_alloc): nothing
 // is allocated, the scratch is not grown and no profiling events are created.
 static fs_status enqueue(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint32_t* vals,
@@ -464,6 +598,8 @@ static fs_status enqueue(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint
     const size_t kb = key_bytes(t);
     if ((uintptr_t)keys % kb != 0 || (vals && (uintptr_t)vals % 4 != 0))
         return set_err(s, FS_ERR_INVALID_ARGUMENT, "misaligned key or value pointer");
+    const BucketPath bp = bucket_path(s, op, t, n, no_alloc);
+    if (bp != BK_NONE) return enqueue_buckets(s, op, t, keys, vals, n, st, bp, no_alloc);
     const int var = sort_variant(s, op, t, n, no_alloc);
     const uint32_t tile = s->tile[var];
     const uint32_t num_tiles = (uint32_t)((n + tile - 1) / tile);
@@ -745,6 +881,20 @@ static fs_status create(int device, hipStream_t stream, bool own, fs_sorter** ou
                 s->local_block[w][i] = threads;
             }
         s->local_min_bits32 = lg[4];
+        hipDeviceptr_t kp = nullptr;
+        size_t ksz = 0;
+        uint32_t bg[11] = {};
+        if (hipModuleGetGlobal(&kp, &ksz, s->module, "fs_kernel_bucket_geometry") != hipSuccess ||
+            ksz != sizeof(bg) || hipMemcpyDtoH(bg, kp, sizeof(bg)) != hipSuccess || bg[0] < FS_RADIX || bg[8] != FS_BK_NB)
+            return create_failed(s, FS_ERR_SHADER_COMPILATION, "code object lacks a valid fs_kernel_bucket_geometry");
+        s->bk_block = bg[0];
+        s->bk_tile[0] = bg[1];
+        s->bk_tile[1] = bg[2];
+        for (int i = 0; i < 4; ++i) s->bk_cap[i / 2][i % 2] = bg[3 + i];
+        s->bk_samples = bg[7];
+        s->bk_max = bg[8];
+        s->bk_part_block = bg[9];
+        s->bk_split_block = bg[10];
     }
     const size_t tab = (size_t)FS_MAX_DIGITS * FS_RADIX * 4;
     if (hipMalloc(&s->hist, (size_t)FS_HIST_WORDS * 4) != hipSuccess || hipMalloc(&s->binbase, tab) != hipSuccess ||
@@ -752,6 +902,7 @@ static fs_status create(int device, hipStream_t stream, bool own, fs_sorter** ou
         hipMalloc(&s->rtable, FS_RTABLE_WORDS * 4) != hipSuccess ||
         hipMalloc(&s->plan, FS_PLAN_WORDS * sizeof(uint32_t)) != hipSuccess ||
         hipMalloc(&s->segc, FS_SEGC_WORDS * sizeof(uint32_t)) != hipSuccess ||
+        hipMalloc(&s->bk_tab, FS_BK_TAB_WORDS * sizeof(uint32_t)) != hipSuccess ||
         hipMalloc(&s->stats, FS_STAT_SLOTS * FS_STAT_COUNT * sizeof(unsigned long long)) != hipSuccess ||
         hipHostMalloc(&s->status, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess)
         return create_failed(s, FS_ERR_OUT_OF_MEMORY, "device tables of the sorter");
@@ -808,6 +959,7 @@ void fs_sorter_free(fs_sorter* s) {
     if (s->binbase) (void)hipFree(s->binbase);
     if (s->plan) (void)hipFree(s->plan);
     if (s->segc) (void)hipFree(s->segc);
+    if (s->bk_tab) (void)hipFree(s->bk_tab);
     if (s->stats) (void)hipFree(s->stats);
     if (s->status) (void)hipHostFree(s->status);
     for (int b = 0; b < 2; ++b) {
@@ -960,6 +1112,12 @@ fs_status fs_sorter_set_test_option(fs_sorter* s, fs_test_option opt, uint64_t v
                                           (unsigned long long)value);
             s->local_wide_mode = (uint32_t)value;
             return FS_OK;
+        case FS_TEST_BUCKETS:
+            if ((value & 0xFFu) > 3u || (value >> 8) > 16u)
+                return set_err(s, FS_ERR_INVALID_ARGUMENT, "bucket choice %llu", (unsigned long long)value);
+            s->bucket_mode = (uint32_t)(value & 0xFFu);
+            s->bucket_lnb = (uint32_t)(value >> 8);
+            return FS_OK;
         case FS_TEST_SEG_BITS:
             if (value != 0 && (value < 8 || value > 16))
                 return set_err(s, FS_ERR_INVALID_ARGUMENT, "segment bits %llu outside 8..16", (unsigned long long)value);
@@ -972,7 +1130,7 @@ fs_status fs_sorter_set_test_option(fs_sorter* s, fs_test_option opt, uint64_t v
             return FS_OK;
         case FS_TEST_INJECT_FAULT:
 #ifdef FS_FAULT_INJECTION
-            if (value > FS_FAULT_SMALL_S1) return set_err(s, FS_ERR_INVALID_ARGUMENT, "unknown fault %llu",
+            if (value > FS_FAULT_SMALL_REGIONS) return set_err(s, FS_ERR_INVALID_ARGUMENT, "unknown fault %llu",
                                                            (unsigned long long)value);
             s->fault = (uint32_t)value;
             return FS_OK;

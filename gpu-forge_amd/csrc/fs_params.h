@@ -360,6 +360,84 @@
 #define FS_LOOP_SLOT64 4u
 #endif
 
+// Bucket path (bucket_sort.h): threads per block; keys per thread of the
+// partition's tiles, of the blocks that sort a bucket (or a small input) in
+// LDS, and of the sample; most buckets.
+#ifndef FS_BK_BLOCK
+#define FS_BK_BLOCK 512
+#endif
+#ifndef FS_BP_BLOCK
+#define FS_BP_BLOCK 1024
+#endif
+#ifndef FS_BS_BLOCK
+#define FS_BS_BLOCK 1024
+#endif
+#define FS_BK32_WAVES 6
+#define FS_BK32V_WAVES 4
+#define FS_BK64_WAVES 4
+#define FS_BK64V_WAVES 4
+#ifndef FS_BP32_ITEMS
+#define FS_BP32_ITEMS 8
+#endif
+#ifndef FS_BP64_ITEMS
+#define FS_BP64_ITEMS 5
+#endif
+#ifndef FS_BK32_ITEMS
+#define FS_BK32_ITEMS 16
+#endif
+#ifndef FS_BK32V_ITEMS
+#define FS_BK32V_ITEMS 16
+#endif
+#ifndef FS_BK64_ITEMS
+#define FS_BK64_ITEMS 16
+#endif
+#ifndef FS_BK64V_ITEMS
+#define FS_BK64V_ITEMS 12
+#endif
+#ifndef FS_BS_ITEMS
+#define FS_BS_ITEMS 8
+#endif
+#ifndef FS_BK_LNB
+#define FS_BK_LNB 9
+#endif
+#define FS_BK_NB (1u << FS_BK_LNB)
+// block sort: bits that name a group, and the most keys of a group that is
+// ranked by comparison
+#ifndef FS_BK_GBITS
+#define FS_BK_GBITS 12
+#endif
+#define FS_BK_GLIM(wide, vals) ((wide) ? ((vals) ? 32u : 40u) : ((vals) ? 16u : 24u))
+// Largest sorts that one block does alone, and that buckets do, by key width
+// and values (V); keys a bucket is meant to hold
+#ifndef FS_BK_ONE_32
+#define FS_BK_ONE_32 8192u
+#define FS_BK_ONE_32V 8192u
+#define FS_BK_ONE_64 8192u
+#define FS_BK_ONE_64V 6144u
+#define FS_BK_MAX_32 1500000u
+#define FS_BK_MAX_32V 1500000u
+#define FS_BK_MAX_64 1500000u
+#define FS_BK_MAX_64V 1100000u
+#endif
+#ifndef FS_BK_MEAN
+#define FS_BK_MEAN 2048u
+#endif
+// bits of 64-bit samples sorted first (all of them when these leave two out of order)
+#define FS_BK_SAMPLE_BITS 40u
+// Room of a bucket's region, in samples beyond its own and six standard
+// deviations of them; the most sample-widths the regions of nb buckets of m
+// samples can take (every bucket the same share, the rounding to 16 keys apart)
+#define FS_BK_ROOM 18.0f
+// Table words: bucket counts, region bases, region capacities, the bits set
+// and clear in some key (low, high word each), the splitters
+#define FS_BK_CNT 0u
+#define FS_BK_BASE (FS_BK_CNT + FS_BK_NB)
+#define FS_BK_CAPS (FS_BK_BASE + FS_BK_NB)
+#define FS_BK_BITS (FS_BK_CAPS + FS_BK_NB)
+#define FS_BK_BIT_SLOTS 16u
+#define FS_BK_LB (FS_BK_BITS + 4u * FS_BK_BIT_SLOTS)
+#define FS_BK_TAB_WORDS (FS_BK_LB + 2u * FS_BK_NB)
+
 // Error bits additionally reported through the status word.
 #define FS_DEVERR_BAD_TILE 2u        // a digit pass block mapped to a tile >= num_tiles
 #define FS_DEVERR_BAD_PLAN 4u        // a schedule named a buffer the call does not have
@@ -375,6 +453,9 @@
 #define FS_FAULT_STALL_TILE 4u     // tile 1 of the first pass never publishes -> LOOKBACK_TIMEOUT
 #define FS_FAULT_SMALL_S1 5u       // the region sample's S1 budget halved: its layout does not fit and
                                    // the regions split the budget evenly (no error; the sort stays exact)
+
+#define FS_FAULT_SMALL_REGIONS 6u  // the bucket path's region of bucket 1 gets one row's room (no error; the sort
+                                   // stays exact, done by one block)
 
 // Scratch of the entry point that allocates nothing (fs_encode_no_alloc): a
 // file-scope static device array of FS_NA_SCRATCH_BYTES in the code object,
@@ -446,6 +527,9 @@ typedef struct FsArgs {
                                 // sort leaves to its second launch
     uint32_t seg_bits;          // top-16 launch sequence: bits that name a segment of the local sort
                                 // (8..16), else 0
+    uint32_t bk_lnb;            // bucket path: log2 of the buckets (0: one block sorts everything)
+    uint64_t bk_tab;            // u32[FS_BK_TAB_WORDS] bucket table
+    uint32_t bk_lm;             // log2 of the samples
     uint32_t reserved0;
 } FsArgs;
 

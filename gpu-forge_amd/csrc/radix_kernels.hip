@@ -680,7 +680,7 @@ DEV void rank_wave(const uint32_t (&x)[ITEMS], uint32_t xshift, uint16_t* wb, Ra
 // that is published; it stops at the first INC or at tile 0 (which publishes
 // INC).  Then it publishes this tile's INC.  Every wait is bounded
 // (FS_SPIN_LIMIT).  WIDE selects the 64-bit tile entries.
-template <bool WIDE>
+template <bool WIDE, uint32_t RADIX = FS_RADIX>
 DEV uint32_t lookback(GLOBAL uint32_t* lb, const GLOBAL uint32_t* grp, uint32_t tile, uint32_t d,
                       uint32_t valid, uint64_t status, uint32_t& rounds, uint32_t& stalls, uint32_t& entries) {
     typedef LbEntry<WIDE> E;
@@ -707,7 +707,7 @@ DEV uint32_t lookback(GLOBAL uint32_t* lb, const GLOBAL uint32_t* grp, uint32_t 
         typename E::type e[FS_LB_WINDOW];
 #pragma unroll
         for (int j = 0; j < FS_LB_WINDOW; ++j)
-            e[j] = (j < (int)avail) ? E::load(lb, (uint64_t)(t - 1 - j) * FS_RADIX + d) : 0u;
+            e[j] = (j < (int)avail) ? E::load(lb, (uint64_t)(t - 1 - j) * RADIX + d) : 0u;
         uint32_t used = 0;
         bool stalled = false;
 #pragma unroll
@@ -735,8 +735,8 @@ DEV uint32_t lookback(GLOBAL uint32_t* lb, const GLOBAL uint32_t* grp, uint32_t 
 #pragma unroll
         for (int j = 0; j < FS_LB_GWIN; ++j) {
             const uint64_t gg = g - 1 - j;
-            ei[j] = (j < (int)avail) ? E::load(lb, (gg * FS_LB_GROUP + FS_LB_GROUP - 1) * FS_RADIX + d) : 0u;
-            eg[j] = (j < (int)avail) ? ld_agent(&grp[gg * FS_RADIX + d]) : 0u;
+            ei[j] = (j < (int)avail) ? E::load(lb, (gg * FS_LB_GROUP + FS_LB_GROUP - 1) * RADIX + d) : 0u;
+            eg[j] = (j < (int)avail) ? ld_agent(&grp[gg * RADIX + d]) : 0u;
         }
         uint32_t used = 0;
         bool stalled = false;
@@ -759,7 +759,7 @@ DEV uint32_t lookback(GLOBAL uint32_t* lb, const GLOBAL uint32_t* grp, uint32_t 
         entries += used;
         if (!done && stalled) stall();
     }
-    E::store(lb, (uint64_t)tile * FS_RADIX + d, FS_LB_INC, excl + valid);
+    E::store(lb, (uint64_t)tile * RADIX + d, FS_LB_INC, excl + valid);
     return excl;
 }
 
@@ -3151,6 +3151,8 @@ extern "C" __global__ void __launch_bounds__(FS_K64_BLOCK) FS_OCC(FS_K64_BLOCK /
     }
 }
 
+#include "bucket_sort.h"
+
 // Tile sizes of the digit-pass variants (FS_VAR_*), read by the host runtime.
 extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_tile_keys[FS_VARIANTS] = {
     FS_K32_BLOCK * FS_K32_ITEMS, FS_K32V_BLOCK * FS_K32V_ITEMS,
@@ -3163,6 +3165,13 @@ extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_tile_keys[FS_VA
 extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_local_geometry[9] = {
     FS_L32_BLOCK * FS_L32_ITEMS, FS_L32_BLOCK, FS_L64_BLOCK * FS_L64_ITEMS, FS_L64_BLOCK, 32u - (FS_LOCAL_UBITS + 8u),
     FS_LW_BLOCK * FS_L32_ITEMS, FS_LW_BLOCK, FS_LW_BLOCK * FS_L64_ITEMS, FS_LW_BLOCK};
+// Bucket path: threads per block, keys per tile of the partition (32-bit keys,
+// 64-bit), keys a block sorts in LDS (32-bit, with values, 64-bit, with
+// values), most samples, most buckets, threads per block of the partition and of the sample.
+extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_bucket_geometry[11] = {
+    FS_BK_BLOCK, FS_BP_BLOCK * FS_BP32_ITEMS, FS_BP_BLOCK * FS_BP64_ITEMS, FS_BK_BLOCK * FS_BK32_ITEMS,
+    FS_BK_BLOCK * FS_BK32V_ITEMS, FS_BK_BLOCK * FS_BK64_ITEMS, FS_BK_BLOCK * FS_BK64V_ITEMS,
+    FS_BS_BLOCK * FS_BS_ITEMS, FS_BK_NB, FS_BP_BLOCK, FS_BS_BLOCK};
 // Threads per block of the same variants.
 extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_block_threads[FS_VARIANTS] = {
     FS_K32_BLOCK, FS_K32V_BLOCK, FS_K64_BLOCK, FS_K64V_BLOCK, FS_K32S_BLOCK, FS_KS_BLOCK, FS_KS_BLOCK, FS_KS_BLOCK};

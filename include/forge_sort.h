@@ -250,9 +250,12 @@ typedef enum fs_test_option {
                                            the sample choosing as by default */
     FS_TEST_SEG_BITS = 5,               /* top-16 path: 0 = segment bits by size (the default),
                                            8..16 = segments named by that many top bits */
-    FS_TEST_LOCAL_WIDE = 6              /* top-16 path: 0 = wide local-sort blocks by size (the
+    FS_TEST_LOCAL_WIDE = 6,             /* top-16 path: 0 = wide local-sort blocks by size (the
                                            default: beyond the other blocks' size limit),
                                            1 = wide blocks at every size */
+    FS_TEST_BUCKETS = 7                 /* bucket path: 0 = by size (the default), 1 = never, 2 = one
+                                           block for every sort that fits it, 3 = buckets for every
+                                           sort of at least 64 keys; + (b << 8): 2^b buckets */
 } fs_test_option;
 fs_status fs_sorter_set_test_option(fs_sorter *s, fs_test_option opt, uint64_t value);
 

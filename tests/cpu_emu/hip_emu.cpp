@@ -389,6 +389,17 @@ void fs_gather_elems(uint64_t, uint64_t, uint64_t, uint64_t, uint64_t, uint32_t,
 extern uint32_t fs_kernel_tile_keys[FS_VARIANTS];
 extern uint32_t fs_kernel_block_threads[FS_VARIANTS];
 extern uint32_t fs_kernel_local_geometry[9];
+extern uint32_t fs_kernel_bucket_geometry[11];
+void fs_split_k32(FsArgs);
+void fs_split_k64(FsArgs);
+void fs_part_k32(FsArgs);
+void fs_part_k32_v(FsArgs);
+void fs_part_k64(FsArgs);
+void fs_part_k64_v(FsArgs);
+void fs_bucket_k32(FsArgs);
+void fs_bucket_k32_v(FsArgs);
+void fs_bucket_k64(FsArgs);
+void fs_bucket_k64_v(FsArgs);
 }
 
 struct emu_function {
@@ -399,6 +410,16 @@ struct emu_function {
 #define A0 (*(FsArgs*)p[0])
 #define D1 (*(uint32_t*)p[1])
 static emu_function g_funcs[] = {
+    {"fs_split_k32", [](void** p) { fs_split_k32(A0); }},
+    {"fs_split_k64", [](void** p) { fs_split_k64(A0); }},
+    {"fs_part_k32", [](void** p) { fs_part_k32(A0); }},
+    {"fs_part_k32_v", [](void** p) { fs_part_k32_v(A0); }},
+    {"fs_part_k64", [](void** p) { fs_part_k64(A0); }},
+    {"fs_part_k64_v", [](void** p) { fs_part_k64_v(A0); }},
+    {"fs_bucket_k32", [](void** p) { fs_bucket_k32(A0); }},
+    {"fs_bucket_k32_v", [](void** p) { fs_bucket_k32_v(A0); }},
+    {"fs_bucket_k64", [](void** p) { fs_bucket_k64(A0); }},
+    {"fs_bucket_k64_v", [](void** p) { fs_bucket_k64_v(A0); }},
     {"fs_upsweep_k32", [](void** p) { fs_upsweep_k32(A0); }},
     {"fs_upsweep_k64", [](void** p) { fs_upsweep_k64(A0); }},
     {"fs_onesweep_k32", [](void** p) { fs_onesweep_k32(A0, D1); }},
@@ -566,6 +587,7 @@ hipError_t hipModuleGetFunction(hipFunction_t* f, hipModule_t, const char* name)
 hipError_t hipModuleGetGlobal(hipDeviceptr_t* p, size_t* sz, hipModule_t, const char* name) {
     if (!strcmp(name, "fs_kernel_tile_keys")) { *p = fs_kernel_tile_keys; *sz = sizeof fs_kernel_tile_keys; return hipSuccess; }
     if (!strcmp(name, "fs_kernel_block_threads")) { *p = fs_kernel_block_threads; *sz = sizeof fs_kernel_block_threads; return hipSuccess; }
+    if (!strcmp(name, "fs_kernel_bucket_geometry")) { *p = fs_kernel_bucket_geometry; *sz = sizeof fs_kernel_bucket_geometry; return hipSuccess; }
     if (!strcmp(name, "fs_kernel_local_geometry")) { *p = fs_kernel_local_geometry; *sz = sizeof fs_kernel_local_geometry; return hipSuccess; }
     return hipErrorNotFound;
 }

@@ -8,6 +8,7 @@ package is pointed at the emulation library only inside this process.
 """
 import ctypes
 import os
+import re
 import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -325,6 +326,22 @@ def check_first_pass(sorter, op, kind, n, dist, seed):
 
 
 def check(sorter, op, kind, n, dist, seed):
+    # one_<op>: one block sorts everything; bk_<op>, bk<b>_<op>: the bucket
+    # path (2^b buckets); bkover_<op>: with a region that overflows (fault build)
+    bucket = re.fullmatch(r"(one|bk|bkover)(\d*)_(sort|argsort|pairs|offset)", op)
+    if bucket:
+        one, b, rest = bucket.groups()
+        sorter.set_test_option(forge_sort.TEST_BUCKETS,
+                               forge_sort.BUCKETS_ONE_BLOCK if one == "one"
+                               else forge_sort.BUCKETS_ALWAYS + (int(b or 0) << 8))
+        if one == "bkover":
+            sorter.set_test_option(forge_sort.TEST_INJECT_FAULT, forge_sort.FAULT_SMALL_REGIONS)
+        try:
+            return check(sorter, rest, kind, n, dist, seed)
+        finally:
+            sorter.set_test_option(forge_sort.TEST_BUCKETS, forge_sort.BUCKETS_BY_SIZE)
+            if one == "bkover":
+                sorter.set_test_option(forge_sort.TEST_INJECT_FAULT, forge_sort.FAULT_NONE)
     if op in FIRST_PASS or op.startswith(("top16s", "top16w")):
         return check_first_pass(sorter, op, kind, n, dist, seed)
     if op == "noalloc":

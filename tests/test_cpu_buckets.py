@@ -1,0 +1,50 @@
+"""The bucket path's kernels on the CPU emulator against the oracle: small blocks
+and tiles, so that a few thousand keys fill many buckets; one wave at a time,
+which turns a missing barrier into a wrong result; the sanitizers; a region
+that overflows."""
+import os
+import subprocess
+
+import pytest
+
+from test_cpu_emulation import emulator, pytestmark, run_cases  # noqa: F401
+
+CASES = [
+    # one block: every op and key width, one key more than the rows of a wave,
+    # few values, quantised and special floats, every key equal
+    "one_sort:u32:500:uniform:1", "one_sort:f32:768:few:2", "one_argsort:u32:300:few:3", "one_pairs:f64:512:uniform:4",
+    "one_sort:i64:511:uniform:5", "one_sort:u32:2:uniform:6", "one_sort:u64:400:low12:7", "one_argsort:i32:65:same:8",
+    # buckets: uniform, few values (buckets of one value larger than a block),
+    # skewed, narrow, equal keys; look-back over many tiles
+    "bk_sort:u32:3000:uniform:9", "bk_sort:u32:3000:few:10", "bk_sort:i64:2000:uniform:11", "bk_argsort:f32:2000:few:12",
+    "bk_pairs:u64:1500:uniform:13", "bk_pairs:u32:3000:zipf:14", "bk_argsort:f64:3000:low12:15", "bk_sort:f64:3000:same:16",
+    "bk_argsort:u32:5000:same:17", "bk_sort:u32:64:uniform:18", "bk_offset:f32:3001:uniform:19",
+    # few buckets of many keys: blocks that sort theirs through device memory
+    "bk2_sort:u32:5000:uniform:20", "bk2_pairs:f64:4000:few:21", "bk2_argsort:u32:4000:uniform:22",
+]
+
+
+def test_emulated_buckets(emulator):  # noqa: F811
+    run_cases("small", CASES, parallel=4)
+    run_cases("prod", ["one_sort:u32:8192:uniform:1", "one_pairs:f64:6144:few:2", "bk_sort:u32:40000:uniform:3",
+                       "bk_argsort:f32:30000:few:4", "bk_pairs:u64:20000:zipf:5"], parallel=3, env={"EMU_CUS": "8"})
+
+
+@pytest.mark.parametrize("order", ["wave", "wave_rev"])
+def test_emulated_buckets_wave_serial(emulator, order):  # noqa: F811
+    run_cases("small", CASES, timeout=900, env={"EMU_SCHED": order}, parallel=4)
+
+
+def test_emulated_buckets_overflow(emulator):  # noqa: F811
+    """A region with room for one row only: its keys do not fit, and one block
+    sorts the caller's keys instead (the fault-injection build)."""
+    run_cases("faults", ["bkover_sort:u32:3000:uniform:1", "bkover_pairs:u64:2000:few:2", "bkover_argsort:f32:3000:uniform:3",
+                         "bkover_sort:i64:2000:uniform:4"])
+
+
+def test_emulated_buckets_sanitizers(emulator):  # noqa: F811
+    libasan = subprocess.run(["g++", "-print-file-name=libasan.so"], capture_output=True, text=True).stdout.strip()
+    if not os.path.isabs(libasan):
+        pytest.skip("libasan not found")
+    run_cases("san", CASES[::2], timeout=600, env={"LD_PRELOAD": libasan, "EMU_NO_SEGV_HANDLER": "1", "EMU_CUS": "4",
+                                                  "ASAN_OPTIONS": "detect_leaks=0:detect_stack_use_after_return=0"}, parallel=3)

@@ -12,12 +12,27 @@
 //                   own, so that copies of one key never crowd a bucket with
 //                   other keys
 //     fs_part_*     every key to its bucket's region of scratch S1: the bucket
-//                   by binary search in the splitters (LDS), its place by one
-//                   atomic per tile and bucket (keys only) or, for values,
-//                   whose order among equal keys must hold, by the decoupled
-//                   look-back of the digit passes
+//                   from a table of the keys' groups or by binary search in
+//                   the splitters (LDS), its place by one atomic per tile and
+//                   bucket (keys only) or, for values, whose order among
+//                   equal keys must hold, by the decoupled look-back of the
+//                   digit passes
 //     fs_bucket_*   one block per bucket: read once, sorted in LDS, written
 //                   once to its place in the output
+//   two levels (larger sorts of 64-bit keys: three passes over them instead
+//   of eight digits')
+//     fs_split_*, fs_part1_*   as above, 256 buckets
+//     fs_split2_*   one block per bucket samples it, in S1, for its children
+//     fs_part2_*    every bucket's keys to its children's regions of S2
+//     fs_child_*    one block per child, as fs_bucket_*
+//     fs_rest_*     children larger than a block and buckets of an overflowed
+//                   child, from a list, on a small grid
+//   The digit passes run before these and sort keys of few varying digits
+//   (FS_BK2_FEW_DIGITS); f64, 128M keys: 4,567 -> 2,496 us (part1 623, part2
+//   554, child 648, rest 96), u64 pairs, 16M: 906 -> 542 (143, 107, 143, 20).
+//   The partitions move 1 GB of reads and 1 GB of scattered writes of
+//   f64 128M at 3.3 and 3.7 TB/s (a copy here: 4.75), the children's blocks
+//   are bound by their LDS passes.
 //
 // The block sort groups the keys by the top bits of their range and ranks each
 // within its group by comparison; blocks with large groups (many copies of a
@@ -26,24 +41,27 @@
 // block (16 bits) and the values follow by one gather at the end.
 //
 // Buckets are sized by the sample, so a bucket can outgrow its region or a
-// block's LDS (16 samples a bucket and regions of FS_BK_ROOM times the
-// estimate: not once in 10^6 sorts).  Such a sort stays exact: the block of an
-// oversized bucket, or block 0 for every key after an overflowed region, sorts
-// it alone through device memory (slow_sort).
+// block's LDS (a region has room for its samples, six standard deviations of
+// them and FS_BK_ROOM more: below 10^-9 a bucket).  Such a sort stays exact:
+// the block of an oversized bucket, or block 0 for every key after an
+// overflowed region, sorts it alone through device memory (slow_sort).
 
 // Elements of the LDS block sort of WAVES waves: rows of 64 keys, `per` rows
 // to each wave (wave w: rows w * per ...), so that a small segment still uses
 // every wave.
-template <bool K64, bool VALS, int BLOCK, int ITEMS>
+template <bool K64, bool VALS, int BLOCK, int ITEMS, int GB = FS_BK_GBITS>
 struct BlockSortLds {
     typedef typename KeyT<K64>::type K;
     static constexpr uint32_t CAP = BLOCK * ITEMS;
     static constexpr int WAVES = BLOCK / 64;
     alignas(16) K keys[CAP];
     uint16_t pos[VALS ? CAP : 1];                // with values: each key's position in the block
-    alignas(16) uint16_t wcnt[WAVES][FS_RADIX];  // per-wave digit counts, then bases
-    uint32_t dbase[FS_RADIX];
-    uint16_t starts[(1u << FS_BK_GBITS) + 2u];   // group starts
+    // stable passes (not in the children's blocks, which leave those to fs_rest_*):
+    // per-wave digit counts, then bases
+    static constexpr bool LSD = GB == FS_BK_GBITS;
+    alignas(16) uint16_t wcnt[LSD ? WAVES : 1][LSD ? FS_RADIX : 2];
+    uint32_t dbase[LSD ? FS_RADIX : 1];
+    uint16_t starts[(1u << GB) + 2u];   // group starts
     uint32_t wsum[WAVES];
     uint32_t flag;
     K red[2][WAVES];
@@ -122,7 +140,7 @@ DEV void block_sort_pass(typename KeyT<K64>::type (&k)[ITEMS], Ranks<VALS ? ITEM
 // order) to 2^FS_BK_GBITS groups: by the top bits of k, or (floats) by value,
 // linear between the least and greatest finite values of the block; keys
 // beyond those, the infinities and NaNs among them, fall into the outer groups.
-template <bool K64>
+template <bool K64, int GB = FS_BK_GBITS>
 struct GroupMap {
     typedef typename KeyT<K64>::type K;
     bool by_value;
@@ -148,12 +166,19 @@ struct GroupMap {
         else f = __builtin_bit_cast(uint32_t, (float)v);
         return xf_fwd<K64>(f, FS_XF_FLOAT);
     }
+    // The group of any key of the input (not less `base`), also one outside the
+    // range the map was made for.
+    DEV uint32_t of_key(K u) const {
+        if (by_value) return (*this)(u - base);
+        const K t = u < base ? (K)0 : u - base;
+        return (uint32_t)((t < span ? t : span) >> shift) & ((1u << GB) - 1u);
+    }
     DEV uint32_t operator()(K k) const {
-        if (!by_value) return (uint32_t)(k >> shift) & ((1u << FS_BK_GBITS) - 1u);
+        if (!by_value) return (uint32_t)(k >> shift) & ((1u << GB) - 1u);
         K u = k + base;
         u = u > FINITE ? FINITE : u < ~FINITE ? ~FINITE : u;
         const double t = (value(u) - low) * scale;
-        const double top = (double)((1u << FS_BK_GBITS) - 1u);
+        const double top = (double)((1u << GB) - 1u);
         return (uint32_t)(t > top ? top : t > 0.0 ? t : 0.0);
     }
 };
@@ -165,13 +190,13 @@ struct GroupMap {
 // 64 bits.  False, the rows untouched in registers, when a group holds more
 // than FS_BK_GLIM keys (keys crowded in a small part of the range, or, with
 // values, many copies of a key).
-template <bool K64, bool VALS, int BLOCK, int ITEMS>
-DEV bool group_sort(const typename KeyT<K64>::type (&k)[ITEMS], uint32_t len, const GroupMap<K64>& map, uint32_t per,
-                    BlockSortLds<K64, VALS, BLOCK, ITEMS>& L) {
+template <bool K64, bool VALS, int BLOCK, int ITEMS, int GB>
+DEV bool group_sort(const typename KeyT<K64>::type (&k)[ITEMS], uint32_t len, const GroupMap<K64, GB>& map, uint32_t per,
+                    BlockSortLds<K64, VALS, BLOCK, ITEMS, GB>& L) {
     typedef typename KeyT<K64>::type K;
-    constexpr uint32_t CAP = BLOCK * ITEMS, NG = 1u << FS_BK_GBITS;
+    constexpr uint32_t CAP = BLOCK * ITEMS, NG = 1u << GB;
     constexpr uint32_t GPT = NG / BLOCK, GLIM = FS_BK_GLIM(K64, VALS);
-    static_assert(NG % BLOCK == 0 && sizeof(L.keys) >= (NG + 1u) * 4u, "group counters in the keys' words");
+    static_assert(NG % BLOCK == 0 && sizeof(L.keys) >= NG * 4u, "group counters in the keys' words");
     const uint32_t tid = threadIdx.x;
     const uint32_t row0 = (tid >> 6) * per * 64u + (tid & 63u);
     uint32_t* cnt = reinterpret_cast<uint32_t*>(L.keys);
@@ -333,9 +358,9 @@ DEV void block_sort(typename KeyT<K64>::type (&k)[ITEMS], Ranks<VALS ? ITEMS : 1
 // Two folds of the block's valid keys, to every thread: the least and the
 // greatest (BITS false), or the bits set in some key and those clear in some
 // key.
-template <bool K64, bool VALS, int BLOCK, int ITEMS, bool BITS>
+template <bool K64, bool VALS, int BLOCK, int ITEMS, bool BITS, int GB>
 DEV void block_fold(const typename KeyT<K64>::type (&k)[ITEMS], uint32_t len, uint32_t per,
-                    BlockSortLds<K64, VALS, BLOCK, ITEMS>& L, typename KeyT<K64>::type& r0,
+                    BlockSortLds<K64, VALS, BLOCK, ITEMS, GB>& L, typename KeyT<K64>::type& r0,
                     typename KeyT<K64>::type& r1) {
     typedef typename KeyT<K64>::type K;
     constexpr int WAVES = BLOCK / 64;
@@ -378,18 +403,18 @@ DEV uint32_t bit_length(K v) {
 
 // The map of a block whose keys run from `least` to `most`: by value (floats),
 // or by the top bits of the range.
-template <bool K64>
-DEV GroupMap<K64> group_map(typename KeyT<K64>::type least, typename KeyT<K64>::type most, bool by_value) {
+template <bool K64, int GB = FS_BK_GBITS>
+DEV GroupMap<K64, GB> group_map(typename KeyT<K64>::type least, typename KeyT<K64>::type most, bool by_value) {
     typedef typename KeyT<K64>::type K;
-    typedef GroupMap<K64> Map;
+    typedef GroupMap<K64, GB> Map;
     const uint32_t bits = bit_length<K>(most - least);
-    Map map{by_value, bits > FS_BK_GBITS ? bits - FS_BK_GBITS : 0u, least, (K)(most - least), 0.0, 0.0};
+    Map map{by_value, bits > GB ? bits - GB : 0u, least, (K)(most - least), 0.0, 0.0};
     if (by_value) {
         const K lo = least < (K)~Map::FINITE ? (K)~Map::FINITE : least > Map::FINITE ? Map::FINITE : least;
         const K hi = most > Map::FINITE ? Map::FINITE : most < (K)~Map::FINITE ? (K)~Map::FINITE : most;
         map.low = Map::value(lo);
         const double span = Map::value(hi) - map.low;
-        map.scale = span > 0.0 ? (double)(1u << FS_BK_GBITS) / span : 0.0;
+        map.scale = span > 0.0 ? (double)(1u << GB) / span : 0.0;
     }
     return map;
 }
@@ -479,24 +504,104 @@ DEV void bucket_pass_info(const FsArgs& a, uint64_t varying) {
 // fs_split_*: the splitters
 // ---------------------------------------------------------------------------
 
-template <bool K64, int BLOCK, int ITEMS>
+// L2 false: one block, the caller's keys (further blocks only clear look-back
+// entries); L2 true: block p samples bucket p of the first level, in S1, for
+// its children in S2, and writes the bucket's description (FS_BK2_*).
+// What bounds it: one block's chain of loads, counts and scans (8,192 single
+// keys of 1.5M: 23 us, of which the loads of as many cache lines are 6; taking
+// neighbours together was that much faster, but runs of equal keys then made
+// regions overflow).
+
+// (two levels) whether the digit passes have done the sort
+DEV bool digits_sort(const FsArgs& a) {
+    return a.bk2_tab && ((const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab)[FS_BK2_MODE] != 0u;
+}
+
+template <bool K64, int BLOCK, int ITEMS, bool L2>
 DEV void split_body(const FsArgs& a) {
     typedef typename KeyT<K64>::type K;
-    constexpr uint32_t CAP = BLOCK * ITEMS;
+    constexpr uint32_t CAP = BLOCK * ITEMS, NB = L2 ? FS_BK2_NB : FS_BK_NB;
     __shared__ BlockSortLds<K64, false, BLOCK, ITEMS> L;
-    __shared__ K lbs[FS_BK_NB];
-    static_assert(BLOCK >= FS_BK_NB, "a bucket per thread");
+    __shared__ K lbs[NB];
+    __shared__ uint32_t s_par[4];
+    static_assert(BLOCK >= FS_BK_NB && FS_BK_NB >= FS_BK2_NB, "a bucket per thread");
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-    const uint32_t nb = 1u << a.bk_lnb, m = 1u << a.bk_lm;
-    if (nb > FS_BK_NB || m > CAP || m < nb) {
+    const uint32_t nb = 1u << (L2 ? a.bk2_lnb : a.bk_lnb), lm = L2 ? a.bk2_lm : a.bk_lm, m = 1u << lm;
+    const uint32_t par = L2 ? blockIdx.x : 0u;
+    if (nb > NB || m > CAP || m < nb || (L2 && gridDim.x != 1u << a.bk_lnb)) {
         if (tid == 0) report(a, FS_DEVERR_BAD_PLAN);
         return;
     }
-    GLOBAL uint32_t* tab = gptr<uint32_t>(a.bk_tab);
-
-    // samples 4i .. 4i + 3: consecutive keys (one line of memory) at a hashed
-    // position within the i-th of m / 4 equal parts of the input
+    if (digits_sort(a)) return;                          // (uniform)
+    GLOBAL uint32_t* tab1 = gptr<uint32_t>(a.bk_tab);
+    GLOBAL uint32_t* tab2 = gptr<uint32_t>(a.bk2_tab);
+    GLOBAL uint32_t* cnt = L2 ? tab2 + FS_BK2_CNT + par * NB : tab1 + FS_BK_CNT;
+    GLOBAL uint32_t* bases = L2 ? tab2 + FS_BK2_BASE + par * NB : tab1 + FS_BK_BASE;
+    GLOBAL uint32_t* caps = L2 ? tab2 + FS_BK2_CAPS + par * NB : tab1 + FS_BK_CAPS;
+    GLOBAL K* glb = L2 ? reinterpret_cast<GLOBAL K*>(tab2 + FS_BK2_LB) + par * NB : reinterpret_cast<GLOBAL K*>(tab1 + FS_BK_LB);
+    GLOBAL uint32_t* gmap = L2 ? tab2 + FS_BK2_MAP + par * FS_BK_MAP_WORDS : tab1 + FS_BK_MAP;
+    uint32_t n = (uint32_t)a.n, origin = 0;              // keys sampled; first S2 key of the children's regions
     const GLOBAL K* src = gptr<const K>(a.keys);
+    if constexpr (L2) {
+        const uint32_t nb1 = 1u << a.bk_lnb;
+        const uint32_t c = tid < nb1 ? tab1[FS_BK_CNT + tid] : 0u, t = (c + a.tile - 1u) / a.tile;
+        const GLOBAL K* lb1 = reinterpret_cast<const GLOBAL K*>(tab1 + FS_BK_LB);
+        // a bucket of one value has no children: its tiles copy it to its place
+        const bool one = tid < nb1 && (tid + 1u < nb1 ? lb1[tid + 1u] - lb1[tid] == (K)1 : lb1[tid] == ~(K)0);
+        if (tid == 0) L.flag = 0u;
+        const uint32_t start = block_exclusive_scan<BLOCK>(c, L.wsum), tstart = block_exclusive_scan<BLOCK>(t, L.wsum);
+        if (tid < nb1 && c > tab1[FS_BK_CAPS + tid]) L.flag = 1u;
+        if (tid == par) {
+            s_par[0] = c;
+            s_par[1] = start;
+            s_par[2] = tstart;
+            s_par[3] = one ? 1u : 0u;
+        }
+        __syncthreads();
+        if (L.flag) {                                    // (uniform) a region overflowed: fs_rest_* sorts the caller's keys
+            if (tid == 0 && par == 0u) st_agent(&tab2[FS_BK2_OVER], 1u);
+            return;
+        }
+        n = s_par[0];
+        origin = (uint32_t)(((uint64_t)s_par[1] * a.bk2_room) >> 8) + par * (32u * nb + 64u);
+        origin = (origin + 15u) & ~15u;
+        const uint32_t rbase = tab1[FS_BK_BASE + par], ts = s_par[2], tn = (n + a.tile - 1u) / a.tile;
+        if (tid < FS_BK2_INFO_WORDS) {
+            const uint32_t v = tid == 0u ? n : tid == 1u ? rbase : tid == 2u ? s_par[1] : tid == 3u ? ts : tid == 4u ? s_par[3] : 0u;
+            tab2[FS_BK2_INFO + par * FS_BK2_INFO_WORDS + tid] = v;
+        }
+        GLOBAL uint32_t* tmap = gptr<uint32_t>(a.tilemap);
+        for (uint32_t i = tid; i < tn; i += BLOCK)
+            if (ts + i < a.tiles2) tmap[ts + i] = par;
+        if (par + 1u == nb1)                             // (tiles the grid has to spare)
+            for (uint32_t i = ts + tn + tid; i < a.tiles2; i += BLOCK) tmap[i] = 0xFFFFFFFFu;
+        for (uint32_t i = tid; i < nb; i += BLOCK) st_agent(&cnt[i], 0u);
+        if (a.op != FSK_OP_KEYS) {
+            GLOBAL uint32_t* lb = gptr<uint32_t>(a.lookback0);
+            for (uint32_t i = tid; i < tn * nb; i += BLOCK) lb[(uint64_t)ts * nb + i] = 0u;
+            GLOBAL uint32_t* grp = lb + (uint64_t)a.tiles2 * nb + (uint64_t)(ts / FS_LB_GROUP + par) * nb;
+            for (uint32_t i = tid; i < (tn + FS_LB_GROUP - 1u) / FS_LB_GROUP * nb; i += BLOCK) grp[i] = 0u;
+        }
+        if (n == 0u || s_par[3]) return;                 // (uniform)
+        src = gptr<const K>(a.s1k) + rbase;
+    } else {
+        // counters of the partition and (values) its look-back entries start at zero
+        if (a.op != FSK_OP_KEYS) {
+            GLOBAL uint32_t* lb = gptr<uint32_t>(a.lookback0);
+            const uint32_t words = (a.num_tiles + (a.num_tiles + FS_LB_GROUP - 1u) / FS_LB_GROUP) * nb;
+            const uint32_t from = gridDim.x > 1u ? blockIdx.x - 1u : 0u, by = gridDim.x > 1u ? gridDim.x - 1u : 1u;
+            if (gridDim.x == 1u || blockIdx.x)
+                for (uint32_t i = from * BLOCK + tid; i < words; i += by * BLOCK) lb[i] = 0u;
+        }
+        if (blockIdx.x) return;                          // (uniform)
+        for (uint32_t i = tid; i < nb; i += BLOCK) st_agent(&cnt[i], 0u);
+        for (uint32_t i = tid; i < 4u * FS_BK_BIT_SLOTS; i += BLOCK) st_agent(&tab1[FS_BK_BITS + i], 0u);
+        if (a.bk2_tab && tid < 2u) st_agent(&tab2[FS_BK2_OVER + tid], 0u);
+    }
+
+    // sample i: the key at a hashed position within the i-th of m equal parts
+    // of the input.  (Single keys: neighbours often belong together, in runs of
+    // one value or one file's records, and tell little more than one of them.)
     const uint32_t per = (m + BLOCK - 1u) / BLOCK;
     const uint32_t row0 = w * per * 64u + lane;
     K k[ITEMS];
@@ -507,20 +612,9 @@ DEV void split_body(const FsArgs& a) {
         const uint32_t s = row0 + (uint32_t)i * 64u;
         k[i] = ~(K)0;
         if ((uint32_t)i < per && s < m) {
-            const uint32_t c = s >> 2;
-            const uint64_t p0 = ((uint64_t)c * a.n) >> (a.bk_lm - 2u), p1 = ((uint64_t)(c + 1u) * a.n) >> (a.bk_lm - 2u);
-            const uint32_t h = (c * 0x9E3779B9u) ^ ((c * 0x85EBCA6Bu) >> 13);
-            const uint64_t p = p0 + (((uint64_t)h * (p1 > p0 + 4u ? p1 - p0 - 4u : 1u)) >> 32) + (s & 3u);
-            k[i] = xf_fwd<K64>(src[p < a.n ? p : a.n - 1u], a.xform);
+            k[i] = src[sample_position(s, lm, n)];
+            if (!L2) k[i] = xf_fwd<K64>(k[i], a.xform);
         }
-    }
-    // counters of the partition and (values) its look-back entries start at zero
-    for (uint32_t i = tid; i < FS_BK_NB; i += BLOCK) st_agent(&tab[FS_BK_CNT + i], 0u);
-    for (uint32_t i = tid; i < 4u * FS_BK_BIT_SLOTS; i += BLOCK) st_agent(&tab[FS_BK_BITS + i], 0u);
-    if (a.op != FSK_OP_KEYS) {
-        GLOBAL uint4* lb = gptr<uint4>(a.lookback0);
-        const uint32_t words = (a.num_tiles + (a.num_tiles + FS_LB_GROUP - 1u) / FS_LB_GROUP) * FS_BK_NB;
-        for (uint32_t i = tid; i < words / 4u; i += BLOCK) lb[i] = uint4{0u, 0u, 0u, 0u};
     }
 
     const uint32_t stride = m / nb;
@@ -542,7 +636,7 @@ DEV void split_body(const FsArgs& a) {
         spread = count_groups<K64, false, BLOCK, ITEMS>(k, m, map, per, 2u * stride, L);
     }
     if (spread) {
-        for (uint32_t i = tid; i < FS_BK_NB; i += BLOCK) lbs[i] = i ? ~(K)0 : (K)0;
+        for (uint32_t i = tid; i < NB; i += BLOCK) lbs[i] = i ? ~(K)0 : (K)0;
         __syncthreads();
         s0 = tid * stride;
         s1 = s0 + stride;
@@ -555,7 +649,39 @@ DEV void split_body(const FsArgs& a) {
             lbs[tid] = map.inside(g, gn ? (float)(s0 - g0) / (float)gn : 0.0f);
         }
         __syncthreads();
+        // The partition finds a key's bucket from its group: the splitters in
+        // smaller groups, all below the key, then the few in its own.
+        constexpr uint32_t TG = 1u << (FS_BK_GBITS - 1), TPT = (TG + BLOCK - 1) / BLOCK;
+        uint32_t* tc = reinterpret_cast<uint32_t*>(L.keys);
+        for (uint32_t i = tid; i < TG; i += BLOCK) tc[i] = 0u;
+        __syncthreads();
+        if (tid >= 1u && tid < nb) atomicAdd(&tc[map.of_key(lbs[tid]) >> 1], 1u);
+        __syncthreads();
+        uint32_t tsum = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < TPT; ++j) tsum += tid * TPT + j < TG ? tc[tid * TPT + j] : 0u;
+        uint32_t tx = block_exclusive_scan<BLOCK>(tsum, L.wsum);
+        GLOBAL uint16_t* gt = reinterpret_cast<GLOBAL uint16_t*>(gmap + FS_BK_MAP_HEAD);
+#pragma unroll
+        for (uint32_t j = 0; j < TPT; ++j) {
+            if (tid * TPT + j >= TG) continue;
+            gt[tid * TPT + j] = (uint16_t)tx;
+            tx += tc[tid * TPT + j];
+        }
+        if (tid == 0) {
+            const uint64_t w64[4] = {(uint64_t)map.base, (uint64_t)map.span, __builtin_bit_cast(uint64_t, map.low),
+                                     __builtin_bit_cast(uint64_t, map.scale)};
+            gmap[0] = 1u;
+            gmap[1] = map.by_value ? 1u : 0u;
+            gmap[2] = map.shift;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                gmap[4 + 2 * i] = (uint32_t)w64[i];
+                gmap[5 + 2 * i] = (uint32_t)(w64[i] >> 32);
+            }
+        }
     } else {
+        if (tid == 0) gmap[0] = 0u;
         // Keys crowded in parts of the range, or many copies of some: the
         // sample sorted, by groups where those hold copies of one key each,
         // else by stable passes.  64-bit keys take the top FS_BK_SAMPLE_BITS
@@ -599,7 +725,7 @@ DEV void split_body(const FsArgs& a) {
             const bool dup = tid + 1u < nb && q == L.keys[(tid + 1u) * stride] && (K)(q + base) != ~(K)0;
             emit = rep ? 0u : dup ? 2u : 1u;
         }
-        for (uint32_t i = tid; i < FS_BK_NB; i += BLOCK) lbs[i] = i ? ~(K)0 : (K)0;
+        for (uint32_t i = tid; i < NB; i += BLOCK) lbs[i] = i ? ~(K)0 : (K)0;
         const uint32_t at = block_exclusive_scan<BLOCK>(emit, L.wsum) + 1u;
         if (emit && at < nb) lbs[at] = q + base;
         if (emit == 2u && at + 1u < nb) lbs[at + 1u] = q + base + 1u;
@@ -619,25 +745,25 @@ DEV void split_body(const FsArgs& a) {
     }
 
     // Region of bucket j: room for its share of the sample plus six standard
-    // deviations, scaled to n.
+    // deviations, scaled to n.  (Should the regions not fit the S1 or S2 that
+    // the host sized for the largest layout, a bug, their buckets overflow:
+    // the sort stays exact.)
     uint32_t cap = 0;
     if (tid < nb) {
         const float c = (float)(s1 > s0 ? s1 - s0 : 0u);
         const float room = c + 6.0f * __builtin_sqrtf(c) + FS_BK_ROOM;
-        cap = ((uint32_t)(room * ((float)a.n / (float)m)) + 16u) & ~15u;
-        if (cap > (uint32_t)a.n) cap = ((uint32_t)a.n + 15u) & ~15u;
+        cap = ((uint32_t)(room * ((float)n / (float)m)) + 16u) & ~15u;
+        if (cap > n) cap = (n + 15u) & ~15u;
     }
 #ifdef FS_FAULT_INJECTION
-    if (a.fault == FS_FAULT_SMALL_REGIONS && tid == 1u) cap = 64u;
+    if (a.fault == (L2 ? FS_FAULT_SMALL_REGIONS2 : FS_FAULT_SMALL_REGIONS) && tid == 1u) cap = 16u;
 #endif
-    const uint32_t rbase = block_exclusive_scan<BLOCK>(cap, L.wsum);
+    const uint32_t rbase = block_exclusive_scan<BLOCK>(cap, L.wsum) + origin;
     if (tid < nb) {
-        // (a layout beyond S1 cannot be: the host sized it for the largest)
-        const bool fits = (uint64_t)rbase + cap <= a.s1_keys;
-        if (!fits) report(a, FS_DEVERR_BAD_PLAN);
-        tab[FS_BK_BASE + tid] = fits ? rbase : 0u;
-        tab[FS_BK_CAPS + tid] = fits ? cap : 0u;
-        reinterpret_cast<GLOBAL K*>(tab + FS_BK_LB)[tid] = lbs[tid];
+        const bool fits = (uint64_t)rbase + cap <= (L2 ? a.s2_keys : a.s1_keys);
+        bases[tid] = fits ? rbase : 0u;
+        caps[tid] = fits ? cap : 0u;
+        glb[tid] = lbs[tid];
     }
 }
 
@@ -645,20 +771,24 @@ DEV void split_body(const FsArgs& a) {
 // fs_part_*: keys (and values) to their buckets' regions
 // ---------------------------------------------------------------------------
 
-template <bool K64, bool VALS, int BLOCK, int ITEMS>
+// LEVEL 0: one level; 1, 2: the levels of two.  2: tiles of the first level's buckets, in S1, to their children's regions in
+// S2; a tile of a bucket of one value goes to its place in the output.
+template <bool K64, bool VALS, int BLOCK, int ITEMS, int LEVEL>
 DEV void part_body(const FsArgs& a) {
     typedef typename KeyT<K64>::type K;
+    constexpr bool L2 = LEVEL == 2;
     constexpr int WAVES = BLOCK / 64;
     constexpr uint32_t TILE = BLOCK * ITEMS;
-    constexpr uint32_t NB = FS_BK_NB;
+    constexpr uint32_t NB = LEVEL ? FS_BK2_NB : FS_BK_NB;
     constexpr uint32_t DROP = 0xFFFFFFFFu;
-    static_assert(BLOCK >= FS_BK_NB && TILE <= 0xFFFFu, "a bucket per thread, 16-bit tile positions");
+    static_assert(BLOCK >= NB && TILE <= 0xFFFFu, "a bucket per thread, 16-bit tile positions");
     static_assert((uint64_t)FS_LB_GROUP * TILE < (1ull << FS_LB_GCOUNT_SHIFT), "group sums must fit their field");
     __shared__ union {
         K keys[TILE];
         uint32_t vals[TILE];
     } stage;
     __shared__ uint16_t bid[TILE];                     // bucket of every staged position
+    __shared__ uint32_t table[VALS ? 1 : FS_BK_MAP_WORDS - FS_BK_MAP_HEAD];   // two pairs of groups to a word
     __shared__ uint16_t wcnt[VALS ? WAVES : 1][NB];    // values: per-wave bucket counts, then bases
     __shared__ K lbs[NB];
     __shared__ uint32_t cnt[NB];                       // the tile's bucket counts, then starts
@@ -666,25 +796,72 @@ DEV void part_body(const FsArgs& a) {
     __shared__ uint32_t wsum[WAVES];
     __shared__ uint32_t bits[4];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-    const uint32_t lnb = a.bk_lnb, nb = 1u << lnb;
-    const uint32_t tile = blockIdx.x, n32 = (uint32_t)a.n;
+    const uint32_t nb = 1u << (L2 ? a.bk2_lnb : a.bk_lnb);
     const uint32_t rows = a.tile / BLOCK;               // keys per thread of this sort's tiles (at most ITEMS)
-    if (tile >= a.num_tiles || nb > NB || rows > (uint32_t)ITEMS || rows == 0u) {
+    if (blockIdx.x >= (L2 ? a.tiles2 : a.num_tiles) || nb > NB || rows > (uint32_t)ITEMS || rows == 0u) {
         if (tid == 0) report(a, FS_DEVERR_BAD_TILE);
         return;
     }
-    GLOBAL uint32_t* tab = gptr<uint32_t>(a.bk_tab);
+    if (LEVEL && digits_sort(a)) return;                 // (uniform)
+    GLOBAL uint32_t* tab1 = gptr<uint32_t>(a.bk_tab);
+    GLOBAL uint32_t* tab2 = gptr<uint32_t>(a.bk2_tab);
+    uint32_t par = 0, tile = blockIdx.x, n32 = (uint32_t)a.n;   // the bucket, the tile of it, its keys
+    uint64_t src_k = a.keys, src_v = a.vals;
+    uint64_t lb_at = 0, grp_at = (uint64_t)a.num_tiles * nb;
+    if constexpr (L2) {
+        if (((const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab)[FS_BK2_OVER]) return;   // (uniform)
+        par = ((const CONSTANT uint32_t*)(uintptr_t)a.tilemap)[blockIdx.x];
+        if (par >= 1u << a.bk_lnb) return;              // no tile for this block
+        const CONSTANT uint32_t* info = (const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab + FS_BK2_INFO + par * FS_BK2_INFO_WORDS;
+        n32 = info[0];
+        const uint32_t rbase = info[1], start = info[2], ts = info[3];
+        tile = blockIdx.x - ts;
+        if (tile * a.tile >= n32) return;
+        src_k = a.s1k + (uint64_t)rbase * sizeof(K);
+        src_v = a.s1v + (uint64_t)rbase * 4u;
+        lb_at = (uint64_t)ts * nb;
+        grp_at = (uint64_t)a.tiles2 * nb + (uint64_t)(ts / FS_LB_GROUP + par) * nb;
+        if (info[4]) {                                   // one value
+            const uint32_t t0 = tile * a.tile, t1 = min(t0 + a.tile, n32);
+            K xa, xb;
+            xf_inv_masks<K64>(a.xform, xa, xb);
+            const K v = xf_inv_apply<K64>(reinterpret_cast<const GLOBAL K*>(tab1 + FS_BK_LB)[par], xa, xb);
+            const GLOBAL uint32_t* sv = gptr<const uint32_t>(src_v);
+            for (uint32_t i = t0 + tid; i < t1; i += BLOCK) {
+                if (a.op != FSK_OP_ARGSORT) gptr<K>(a.keys)[start + i] = v;
+                if (VALS) gptr<uint32_t>(a.vals)[start + i] = sv[i];
+            }
+            return;
+        }
+    }
+    GLOBAL uint32_t* counts = L2 ? tab2 + FS_BK2_CNT + par * NB : tab1 + FS_BK_CNT;
+    const GLOBAL uint32_t* bases = L2 ? tab2 + FS_BK2_BASE + par * NB : tab1 + FS_BK_BASE;
+    const GLOBAL uint32_t* caps = L2 ? tab2 + FS_BK2_CAPS + par * NB : tab1 + FS_BK_CAPS;
+    const GLOBAL K* glb = L2 ? reinterpret_cast<const GLOBAL K*>(tab2 + FS_BK2_LB) + par * NB
+                             : reinterpret_cast<const GLOBAL K*>(tab1 + FS_BK_LB);
+    const uint32_t tiles = L2 ? (n32 + a.tile - 1u) / a.tile : a.num_tiles;
+    const uint32_t dst_keys = L2 ? a.s2_keys : a.s1_keys;
     const uint32_t begin = tile * a.tile, wbegin = begin + w * 64u * rows + lane;
     const uint32_t tv = n32 - begin < a.tile ? n32 - begin : a.tile;  // the tile's keys
-    const GLOBAL K* src = gptr<const K>(a.keys);
+    const GLOBAL K* src = gptr<const K>(src_k);
     auto valid = [&](int i) -> bool { return (uint32_t)i < rows && wbegin + (uint32_t)i * 64u < n32; };
     K k[ITEMS];
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) k[i] = valid(i) ? src[wbegin + (uint32_t)i * 64u] : (K)0;
     for (uint32_t i = tid; i < NB; i += BLOCK) {
-        lbs[i] = i < nb ? reinterpret_cast<const GLOBAL K*>(tab + FS_BK_LB)[i] : ~(K)0;
+        lbs[i] = i < nb ? glb[i] : ~(K)0;
         cnt[i] = 0u;
     }
+    const CONSTANT uint32_t* gmap = L2 ? (const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab + FS_BK2_MAP + par * FS_BK_MAP_WORDS
+                                       : (const CONSTANT uint32_t*)(uintptr_t)a.bk_tab + FS_BK_MAP;
+    // (the stable partition waits on its look-back, not on the search: it
+    // measured 4% faster without the table)
+    const bool mapped = !VALS && gmap[0] != 0u;         // (uniform)
+    if (mapped) {
+        const GLOBAL uint32_t* gt = (L2 ? tab2 + FS_BK2_MAP + par * FS_BK_MAP_WORDS : tab1 + FS_BK_MAP) + FS_BK_MAP_HEAD;
+        for (uint32_t i = tid; i < (uint32_t)(sizeof(table) / 4u); i += BLOCK) table[i] = gt[i];
+    }
+    const uint32_t my_cap = tid < nb ? caps[tid] : 0u, my_base = tid < nb ? bases[tid] : 0u;
     if (tid < 4u) bits[tid] = 0u;
     if (VALS)
         for (uint32_t i = tid; i < WAVES * NB / 2u; i += BLOCK) reinterpret_cast<uint32_t*>(&wcnt[0][0])[i] = 0u;
@@ -693,25 +870,52 @@ DEV void part_body(const FsArgs& a) {
     uint32_t b[ITEMS];
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
-        k[i] = xf_fwd<K64>(k[i], a.xform);
-        if (valid(i)) {
+        if (!L2) k[i] = xf_fwd<K64>(k[i], a.xform);
+        if (!L2 && valid(i)) {
             on |= k[i];
             off |= ~k[i];
         }
         b[i] = 0u;
     }
-    // bucket: the number of splitters at or below the key (every item's
-    // search advances together: the reads of a step are independent)
-    for (uint32_t step = nb >> 1; step; step >>= 1) {
+    // bucket: the number of splitters at or below the key.  Where the sample
+    // spread over its groups: those in smaller groups from the table, then the
+    // few of the key's own (1.1 LDS reads a key more, where a binary search
+    // takes 8 or 9); else by search (every item's search advances together:
+    // the reads of a step are independent).
+    if (mapped) {
+        GroupMap<K64> map;
+        map.by_value = gmap[1] != 0u;
+        map.shift = gmap[2];
+        uint64_t w64[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w64[i] = ((uint64_t)gmap[5 + 2 * i] << 32) | gmap[4 + 2 * i];
+        map.base = (K)w64[0];
+        map.span = (K)w64[1];
+        map.low = __builtin_bit_cast(double, w64[2]);
+        map.scale = __builtin_bit_cast(double, w64[3]);
+        const uint16_t* tb = reinterpret_cast<const uint16_t*>(table);
 #pragma unroll
         for (int g = 0; g < ITEMS; g += 4) {
             if ((uint32_t)g >= rows) continue;
 #pragma unroll
-            for (int i = g; i < g + 4 && i < ITEMS; ++i) b[i] += lbs[b[i] + step] <= k[i] ? step : 0u;
+            for (int i = g; i < g + 4 && i < ITEMS; ++i) b[i] = tb[map.of_key(k[i]) >> 1];
+#pragma unroll
+            for (int i = g; i < g + 4 && i < ITEMS; ++i)
+                while (b[i] + 1u < nb && lbs[b[i] + 1u] <= k[i]) ++b[i];
+        }
+    } else {
+        for (uint32_t step = nb >> 1; step; step >>= 1) {
+#pragma unroll
+            for (int g = 0; g < ITEMS; g += 4) {
+                if ((uint32_t)g >= rows) continue;
+#pragma unroll
+                for (int i = g; i < g + 4 && i < ITEMS; ++i) b[i] += lbs[b[i] + step] <= k[i] ? step : 0u;
+            }
         }
     }
     // the tile's bits to one of several slots (every tile on one word would
     // queue there)
+    if constexpr (!L2) {
     on = wave_fold<K>(on, [](K x, K y) { return (K)(x | y); });
     off = wave_fold<K>(off, [](K x, K y) { return (K)(x | y); });
     if (lane == 63u) {
@@ -721,6 +925,7 @@ DEV void part_body(const FsArgs& a) {
             atomicOr(&bits[1], (uint32_t)((uint64_t)on >> 32));
             atomicOr(&bits[3], (uint32_t)((uint64_t)off >> 32));
         }
+    }
     }
     // (every lane takes part in the counting; the lanes past n count nothing)
     Ranks<ITEMS> rank;
@@ -743,15 +948,15 @@ DEV void part_body(const FsArgs& a) {
         }
     }
     __syncthreads();
-    if (tid < 4u && bits[tid])
-        __hip_atomic_fetch_or(&tab[FS_BK_BITS + 4u * (tile % FS_BK_BIT_SLOTS) + tid], bits[tid], __ATOMIC_RELAXED,
+    if (!L2 && tid < 4u && bits[tid])
+        __hip_atomic_fetch_or(&tab1[FS_BK_BITS + 4u * (tile % FS_BK_BIT_SLOTS) + tid], bits[tid], __ATOMIC_RELAXED,
                               __HIP_MEMORY_SCOPE_AGENT);
-    GLOBAL uint32_t* lb = gptr<uint32_t>(a.lookback0);
-    GLOBAL uint32_t* grp = lb + (uint64_t)a.num_tiles * NB;
+    GLOBAL uint32_t* lb = gptr<uint32_t>(a.lookback0) + lb_at;
+    GLOBAL uint32_t* grp = gptr<uint32_t>(a.lookback0) + grp_at;
     const uint32_t count = tid < nb ? cnt[tid] : 0u;
     if (VALS && tid < nb) {
-        LbEntry<false>::store(lb, (uint64_t)tile * NB + tid, tile == 0u ? FS_LB_INC : FS_LB_AGG, count);
-        __hip_atomic_fetch_add(&grp[(uint64_t)(tile / FS_LB_GROUP) * NB + tid], (1u << FS_LB_GCOUNT_SHIFT) | count,
+        LbEntry<false>::store(lb, (uint64_t)tile * nb + tid, tile == 0u ? FS_LB_INC : FS_LB_AGG, count);
+        __hip_atomic_fetch_add(&grp[(uint64_t)(tile / FS_LB_GROUP) * nb + tid], (1u << FS_LB_GCOUNT_SHIFT) | count,
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     const uint32_t ex = block_exclusive_scan<BLOCK>(count, wsum);
@@ -759,17 +964,16 @@ DEV void part_body(const FsArgs& a) {
         uint32_t at = 0;
         if (VALS) {
             uint32_t r0 = 0, r1 = 0, r2 = 0;
-            at = tile == 0u ? 0u : lookback<false, NB>(lb, grp, tile, tid, count, a.status, r0, r1, r2);
-            if (tile + 1u == a.num_tiles) st_agent(&tab[FS_BK_CNT + tid], at + count);
+            at = tile == 0u ? 0u : lookback<false>(lb, grp, tile, tid, count, a.status, r0, r1, r2, nb);
+            if (tile + 1u == tiles) st_agent(&counts[tid], at + count);
         } else if (count) {
-            at = __hip_atomic_fetch_add(&tab[FS_BK_CNT + tid], count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            at = __hip_atomic_fetch_add(&counts[tid], count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        const uint32_t cap = tab[FS_BK_CAPS + tid];
         // (a run that does not fit is dropped: the bucket launch sees the count)
-        gbase[tid] = (at <= cap && count <= cap - at) ? tab[FS_BK_BASE + tid] + at - ex : DROP;
+        gbase[tid] = (at <= my_cap && count <= my_cap - at) ? my_base + at - ex : DROP;
         cnt[tid] = ex;
     }
-    if (VALS) rank_wave<true, ITEMS, FS_BK_LNB>(b, 0u, wcnt[w], rank, rows);
+    if (VALS) rank_wave<true, ITEMS, LEVEL ? FS_BK2_LNB : FS_BK_LNB>(b, 0u, wcnt[w], rank, rows);
     __syncthreads();
     if (VALS) {
         if (tid < nb) {
@@ -798,7 +1002,7 @@ DEV void part_body(const FsArgs& a) {
         }
     }
     __syncthreads();
-    GLOBAL K* dst = gptr<K>(a.s1k);
+    GLOBAL K* dst = gptr<K>(L2 ? a.s2k : a.s1k);
     uint32_t gp[ITEMS];
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
@@ -806,7 +1010,7 @@ DEV void part_body(const FsArgs& a) {
         gp[i] = DROP;
         if (p < tv) {
             const uint32_t g = gbase[bid[p] & (NB - 1u)];
-            if (g != DROP && g + p < a.s1_keys) {
+            if (g != DROP && g + p < dst_keys) {
                 gp[i] = g + p;
                 dst[g + p] = stage.keys[p];
             }
@@ -814,18 +1018,18 @@ DEV void part_body(const FsArgs& a) {
     }
     if (VALS) {
         uint32_t v[ITEMS];
-        const GLOBAL uint32_t* sv = gptr<const uint32_t>(a.vals);
+        const GLOBAL uint32_t* sv = gptr<const uint32_t>(src_v);
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
             const uint32_t p = wbegin + (uint32_t)i * 64u;
-            v[i] = a.op == FSK_OP_ARGSORT ? p : valid(i) ? sv[p] : 0u;
+            v[i] = !L2 && a.op == FSK_OP_ARGSORT ? p : valid(i) ? sv[p] : 0u;
         }
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i)
             if (valid(i)) stage.vals[pos.get(i)] = v[i];
         __syncthreads();
-        GLOBAL uint32_t* dv = gptr<uint32_t>(a.s1v);
+        GLOBAL uint32_t* dv = gptr<uint32_t>(L2 ? a.s2v : a.s1v);
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i)
             if (gp[i] != DROP) dv[gp[i]] = stage.vals[(uint32_t)i * BLOCK + tid];
@@ -907,6 +1111,68 @@ DEV void slow_sort(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool fwd, ui
     }
 }
 
+// One block sorts len keys (at most its LDS's) at src_k, with their values at
+// src_v (0: their positions, argsort), into the caller's keys and values from
+// `start` on.  whole: the source is the caller's (transformed on load).
+template <bool K64, bool VALS, int BLOCK, int ITEMS>
+DEV void block_range_sort(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool whole, uint32_t start, uint32_t len,
+                          BlockSortLds<K64, VALS, BLOCK, ITEMS>& L) {
+    typedef typename KeyT<K64>::type K;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+    const bool put_keys = a.op != FSK_OP_ARGSORT;
+    K xa, xb;
+    xf_inv_masks<K64>(a.xform, xa, xb);
+    GLOBAL K* dk = gptr<K>(a.keys);
+    GLOBAL uint32_t* dv = gptr<uint32_t>(a.vals);
+    const uint32_t per = (len + BLOCK - 1u) / BLOCK;     // rows per wave
+    const uint32_t row0 = w * per * 64u + lane;
+    const GLOBAL K* src = gptr<const K>(src_k);
+    K k[ITEMS];
+    Ranks<VALS ? ITEMS : 1> p;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t x = row0 + (uint32_t)i * 64u;
+        k[i] = (uint32_t)i < per && x < len ? src[x] : ~(K)0;
+        if (VALS) p.set_in_order(i, x & 0xFFFFu);
+    }
+    if (whole) {
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i)
+            if (row0 + (uint32_t)i * 64u < len) k[i] = xf_fwd<K64>(k[i], a.xform);
+    }
+    if (whole) {
+        K on = 0, off = 0;
+        block_fold<K64, VALS, BLOCK, ITEMS, true>(k, len, per, L, on, off);
+        if (tid == 0) bucket_pass_info<K64>(a, (uint64_t)(on & off));
+    }
+    K base = 0;
+    sort_rows<K64, VALS, BLOCK, ITEMS>(k, p, len, per, a.xform == FS_XF_FLOAT, L, base);
+
+    // consecutive positions per thread index; values by the position their key had
+    if constexpr (VALS) {
+        uint32_t v[ITEMS];
+        const GLOBAL uint32_t* sv = gptr<const uint32_t>(src_v);
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t x = (uint32_t)i * BLOCK + tid;
+            v[i] = x < len ? (src_v ? sv[L.pos[x]] : L.pos[x]) : 0u;
+        }
+        if (whole) __syncthreads();                     // in place: every value read before any is written
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t x = (uint32_t)i * BLOCK + tid;
+            if (x < len) dv[start + x] = v[i];
+        }
+    }
+    if (put_keys) {
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t x = (uint32_t)i * BLOCK + tid;
+            if (x < len) dk[start + x] = xf_inv_apply<K64>((K)(L.keys[x] + base), xa, xb);
+        }
+    }
+}
+
 template <bool K64, bool VALS, int BLOCK, int ITEMS>
 DEV void bucket_body(const FsArgs& a) {
     typedef typename KeyT<K64>::type K;
@@ -917,7 +1183,7 @@ DEV void bucket_body(const FsArgs& a) {
     __shared__ uint32_t s_over, s_giants;
     __shared__ uint16_t giant[FS_BK_NB];
     static_assert(CAP <= 0x10000u, "16-bit positions");
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+    const uint32_t tid = threadIdx.x;
     const uint32_t lnb = a.bk_lnb, nb = 1u << lnb;
     const bool whole = lnb == 0u;                       // (uniform) one block, the caller's keys
     const GLOBAL uint32_t* tab = gptr<const uint32_t>(a.bk_tab);
@@ -999,59 +1265,210 @@ DEV void bucket_body(const FsArgs& a) {
         return;
     }
 
-    const uint32_t per = (len + BLOCK - 1u) / BLOCK;     // rows per wave
-    const uint32_t row0 = w * per * 64u + lane;
-    const GLOBAL K* src = gptr<const K>(src_k);
+    block_range_sort<K64, VALS, BLOCK, ITEMS>(a, src_k, src_v, whole, start, len, L);
+}
+
+// ---------------------------------------------------------------------------
+// fs_child_*, fs_rest_*: two levels of buckets
+// ---------------------------------------------------------------------------
+
+// Work for fs_rest_*: the two words of an entry.
+DEV void push_rest(const FsArgs& a, uint32_t id, uint32_t what) {
+    GLOBAL uint32_t* tab2 = gptr<uint32_t>(a.bk2_tab);
+    const uint32_t at = __hip_atomic_fetch_add(&tab2[FS_BK2_RESTS], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (at < a.rest_cap) {
+        GLOBAL uint32_t* e = gptr<uint32_t>(a.rest) + 2u * (uint64_t)at;
+        e[0] = id;
+        e[1] = what;
+    } else {
+        report(a, FS_DEVERR_BAD_PLAN);                   // (the host sized the list for every entry there can be)
+    }
+}
+
+// The place of child `id`: its region in S2 and its keys' place in the output.
+// false when there is nothing to do.  over: some child of its bucket outgrew
+// its region (the bucket is then sorted from S1 instead).
+struct ChildPlace {
+    uint32_t start, len, base;
+    bool over, one;
+};
+template <bool K64, int BLOCK>
+DEV bool child_place(const FsArgs& a, uint32_t id, uint32_t* wsum, uint32_t* s_seg, ChildPlace& c) {
+    typedef typename KeyT<K64>::type K;
+    static_assert(BLOCK >= FS_BK2_NB, "a child per thread");
+    const uint32_t tid = threadIdx.x, nb = 1u << a.bk2_lnb;
+    const uint32_t par = id >> a.bk2_lnb, j = id & (nb - 1u);
+    const CONSTANT uint32_t* tab2 = (const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab;
+    const CONSTANT uint32_t* info = tab2 + FS_BK2_INFO + par * FS_BK2_INFO_WORDS;
+    if (tab2[FS_BK2_OVER] || info[0] == 0u || info[4]) return false;          // (uniform)
+    const GLOBAL uint32_t* t = gptr<const uint32_t>(a.bk2_tab);
+    const uint32_t n = tid < nb ? t[FS_BK2_CNT + par * FS_BK2_NB + tid] : 0u;
+    const uint32_t cap = tid < nb ? t[FS_BK2_CAPS + par * FS_BK2_NB + tid] : 0u;
+    if (tid == 0) s_seg[2] = 0u;
+    const uint32_t ex = block_exclusive_scan<BLOCK>(n, wsum);
+    if (n > cap) s_seg[2] = 1u;
+    if (tid == j) {
+        s_seg[0] = ex;
+        s_seg[1] = n;
+    }
+    __syncthreads();
+    const GLOBAL K* lb = reinterpret_cast<const GLOBAL K*>(t + FS_BK2_LB) + par * FS_BK2_NB;
+    c.start = info[2] + s_seg[0];
+    c.len = s_seg[1];
+    c.base = tab2[FS_BK2_BASE + par * FS_BK2_NB + j];
+    c.over = s_seg[2] != 0u;
+    c.one = j + 1u < nb ? lb[j + 1u] - lb[j] == (K)1 && j != 0u : lb[j] == ~(K)0;
+    return true;
+}
+
+// First launch: a small block per child (many to a CU) sorts it where the
+// groups spread it; copies of one value are copied; the others (larger than
+// the block, crowded) go to the rest list.
+template <bool K64, bool VALS, int BLOCK, int ITEMS, int GB>
+DEV void child_body(const FsArgs& a) {
+    typedef typename KeyT<K64>::type K;
+    constexpr uint32_t CAP = BLOCK * ITEMS;
+    __shared__ BlockSortLds<K64, VALS, BLOCK, ITEMS, GB> L;
+    __shared__ uint32_t s_seg[3];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+    const uint32_t id = tile_of_block(blockIdx.x, gridDim.x);
+    if (gridDim.x != 1u << (a.bk_lnb + a.bk2_lnb)) {
+        if (tid == 0) report(a, FS_DEVERR_BAD_PLAN);
+        return;
+    }
+    // The keys' region and their number are known at once; their loads are in
+    // flight while the scan finds their place in the output.
+    const CONSTANT uint32_t* ctab = (const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab;
+    const uint32_t child = (id >> a.bk2_lnb) * FS_BK2_NB + (id & ((1u << a.bk2_lnb) - 1u));
+    const CONSTANT uint32_t* cinfo = ctab + FS_BK2_INFO + (id >> a.bk2_lnb) * FS_BK2_INFO_WORDS;
+    if (ctab[FS_BK2_OVER] || ctab[FS_BK2_MODE] || cinfo[0] == 0u || cinfo[4]) return;   // (uniform)
+    const uint32_t len0 = ctab[FS_BK2_CNT + child] <= CAP ? ctab[FS_BK2_CNT + child] : 0u;
+    const uint32_t per = (len0 + BLOCK - 1u) / BLOCK, row0 = w * per * 64u + lane;
+    const GLOBAL K* src = gptr<const K>(a.s2k) + ctab[FS_BK2_BASE + child];
     K k[ITEMS];
-    Ranks<VALS ? ITEMS : 1> p;
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
         const uint32_t x = row0 + (uint32_t)i * 64u;
-        k[i] = (uint32_t)i < per && x < len ? src[x] : ~(K)0;
-        if (VALS) p.set_in_order(i, x & 0xFFFFu);
+        k[i] = (uint32_t)i < per && x < len0 ? src[x] : ~(K)0;
     }
-    if (whole) {
+    ChildPlace c;
+    if (!child_place<K64, BLOCK>(a, id, L.wsum, s_seg, c)) return;
+    if (c.over) {                                        // (uniform)
+        if (tid == 0 && (id & ((1u << a.bk2_lnb) - 1u)) == 0u) push_rest(a, id, FS_REST_BUCKET);
+        return;
+    }
+    if (c.len == 0u) return;
+    if (c.len > CAP) {
+        // copies of one value a few thousand at a time, anything else whole
+        const uint32_t parts = c.one ? (c.len + FS_REST_KEYS - 1u) / FS_REST_KEYS : 1u;
+        for (uint32_t i = tid; i < parts; i += BLOCK) push_rest(a, id, c.one ? i : FS_REST_SORT);
+        return;
+    }
+    K least = 0, most = 0;
+    block_fold<K64, VALS, BLOCK, ITEMS, false, GB>(k, c.len, per, L, least, most);
+    const uint32_t bits = bit_length<K>(most - least);
+    if (bits == 0u) {                                    // (uniform) one value: in order as it is
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t x = row0 + (uint32_t)i * 64u;
+            if ((uint32_t)i >= per || x >= c.len) continue;
+            L.keys[x] = 0;
+            if constexpr (VALS) L.pos[x] = (uint16_t)x;
+        }
+        __syncthreads();
+    } else {
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i)
-            if (row0 + (uint32_t)i * 64u < len) k[i] = xf_fwd<K64>(k[i], a.xform);
+            if ((uint32_t)i < per && row0 + (uint32_t)i * 64u < c.len) k[i] -= least;
+        if (!group_sort<K64, VALS, BLOCK, ITEMS, GB>(k, c.len, group_map<K64, GB>(least, most, false), per, L)) {
+            if (tid == 0) push_rest(a, id, FS_REST_SORT);
+            return;
+        }
     }
-    if (whole) {
-        K on = 0, off = 0;
-        block_fold<K64, VALS, BLOCK, ITEMS, true>(k, len, per, L, on, off);
-        if (tid == 0) bucket_pass_info<K64>(a, (uint64_t)(on & off));
+    const GLOBAL uint32_t* sv = gptr<const uint32_t>(a.s2v) + c.base;
+    K xa, xb;
+    xf_inv_masks<K64>(a.xform, xa, xb);
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t x = (uint32_t)i * BLOCK + tid;
+        if (x >= c.len) continue;
+        if constexpr (VALS) gptr<uint32_t>(a.vals)[c.start + x] = sv[L.pos[x]];
+        if (!VALS || a.op != FSK_OP_ARGSORT) gptr<K>(a.keys)[c.start + x] = xf_inv_apply<K64>((K)(L.keys[x] + least), xa, xb);
     }
-    K base = 0;
-    sort_rows<K64, VALS, BLOCK, ITEMS>(k, p, len, per, a.xform == FS_XF_FLOAT, L, base);
+}
 
-    // consecutive positions per thread index; values by the position their key had
-    if constexpr (VALS) {
-        uint32_t v[ITEMS];
-        const GLOBAL uint32_t* sv = gptr<const uint32_t>(src_v);
+// Second launch: a small grid takes the rest list in turn: children on the
+// one-level path's block sort (or through device memory when that is too
+// small), pieces of a child of one value, whole buckets whose children
+// outgrew their regions; everything, by one block, when a first-level region
+// did.
+template <bool K64, bool VALS, int BLOCK, int ITEMS>
+DEV void rest_body(const FsArgs& a) {
+    typedef typename KeyT<K64>::type K;
+    __shared__ BlockSortLds<K64, VALS, BLOCK, ITEMS> L;
+    __shared__ uint32_t s_seg[3];
+    const uint32_t tid = threadIdx.x;
+    const CONSTANT uint32_t* tab1 = (const CONSTANT uint32_t*)(uintptr_t)a.bk_tab;
+    const CONSTANT uint32_t* tab2 = (const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab;
+    if (tab2[FS_BK2_MODE]) return;                       // (uniform)
+    if (blockIdx.x == 0 && tid == 0) {
+        uint32_t b[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t x = (uint32_t)i * BLOCK + tid;
-            v[i] = x < len ? (src_v ? sv[L.pos[x]] : L.pos[x]) : 0u;
-        }
-        if (whole) __syncthreads();                     // in place: every value read before any is written
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t x = (uint32_t)i * BLOCK + tid;
-            if (x < len) dv[start + x] = v[i];
-        }
+        for (uint32_t i = 0; i < 4u * FS_BK_BIT_SLOTS; ++i) b[i % 4u] |= tab1[FS_BK_BITS + i];
+        bucket_pass_info<K64>(a, ((uint64_t)(b[1] & b[3]) << 32) | (b[0] & b[2]));
     }
-    if (put_keys) {
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t x = (uint32_t)i * BLOCK + tid;
-            if (x < len) dk[start + x] = xf_inv_apply<K64>((K)(L.keys[x] + base), xa, xb);
+    if (tab2[FS_BK2_OVER]) {                             // (uniform)
+        if (blockIdx.x == 0)
+            slow_sort<K64, VALS, BLOCK, ITEMS>(a, a.keys, a.op == FSK_OP_PAIRS ? a.vals : 0u, true, a.s2k, a.s2v, a.s1k,
+                                               a.s1v, a.keys, a.vals, (uint32_t)a.n, L);
+        return;
+    }
+    const uint32_t count = min(tab2[FS_BK2_RESTS], a.rest_cap);
+    for (uint32_t e = blockIdx.x; e < count; e += gridDim.x) {
+        const CONSTANT uint32_t* ent = (const CONSTANT uint32_t*)(uintptr_t)a.rest + 2u * (uint64_t)e;
+        const uint32_t id = ent[0], what = ent[1];
+        const uint32_t par = id >> a.bk2_lnb, nb = 1u << a.bk2_lnb;
+        if (par >= 1u << a.bk_lnb) return;
+        const CONSTANT uint32_t* info = tab2 + FS_BK2_INFO + par * FS_BK2_INFO_WORDS;
+        ChildPlace c{0u, 0u, 0u, false, false};
+        const bool bucket = what == FS_REST_BUCKET;      // (uniform, as every branch here)
+        if (bucket || child_place<K64, BLOCK>(a, id, L.wsum, s_seg, c)) {
+            __syncthreads();                             // (s_seg read by every thread)
+            // a bucket from its region in S1 through its children's in S2; a
+            // child the other way round (its bucket's keys in S1 are dead)
+            const uint64_t in2 = bucket ? ((((uint64_t)info[2] * a.bk2_room) >> 8) + par * (32u * nb + 64u) + 15u) & ~15ull
+                                        : (uint64_t)c.base;
+            const uint64_t in1 = bucket ? (uint64_t)info[1] : (uint64_t)info[1] + (c.start - info[2]);
+            const uint32_t start = bucket ? info[2] : c.start, len = bucket ? info[0] : c.len;
+            const uint64_t k1 = a.s1k + in1 * sizeof(K), v1 = a.s1v + in1 * 4u;
+            const uint64_t k2 = a.s2k + in2 * sizeof(K), v2 = a.s2v + in2 * 4u;
+            const uint64_t sk = bucket ? k1 : k2, sv = bucket ? v1 : v2;
+            if (bucket || what == FS_REST_SORT) {
+                if (!bucket && len <= (uint32_t)(BLOCK * ITEMS))
+                    block_range_sort<K64, VALS, BLOCK, ITEMS>(a, sk, VALS ? sv : 0u, false, start, len, L);
+                else
+                    slow_sort<K64, VALS, BLOCK, ITEMS>(a, sk, sv, false, bucket ? k2 : k1, bucket ? v2 : v1, sk, sv,
+                                                       a.keys + (uint64_t)start * sizeof(K),
+                                                       a.vals + (uint64_t)start * 4u, len, L);
+            } else {
+                const uint32_t p0 = what * FS_REST_KEYS, p1 = min(p0 + FS_REST_KEYS, c.len);
+                K xa, xb;
+                xf_inv_masks<K64>(a.xform, xa, xb);
+                const K v = xf_inv_apply<K64>(gptr<const K>(sk)[0], xa, xb);
+                for (uint32_t p = p0 + tid; p < p1; p += BLOCK) {
+                    if (a.op != FSK_OP_ARGSORT) gptr<K>(a.keys)[c.start + p] = v;
+                    if (VALS) gptr<uint32_t>(a.vals)[c.start + p] = gptr<const uint32_t>(sv)[p];
+                }
+            }
         }
+        __syncthreads();                                // the entry's LDS is the next one's
     }
 }
 
 // Blocks per CU by LDS: the bucket kernels' registers leave room for them.
 #define FS_BK_KERNELS(sfx, K64, VALS, PITEMS, BITEMS, WAVES)                                                      \
     extern "C" __global__ void __launch_bounds__(FS_BP_BLOCK) fs_part_##sfx(FsArgs a) {                           \
-        part_body<K64, VALS, FS_BP_BLOCK, PITEMS>(a);                                                             \
+        part_body<K64, VALS, FS_BP_BLOCK, PITEMS, 0>(a);                                                          \
     }                                                                                                             \
     extern "C" __global__ void __launch_bounds__(FS_BK_BLOCK) FS_OCC(WAVES) fs_bucket_##sfx(FsArgs a) {           \
         bucket_body<K64, VALS, FS_BK_BLOCK, BITEMS>(a);                                                           \
@@ -1061,9 +1478,31 @@ FS_BK_KERNELS(k32_v, false, true, FS_BP32_ITEMS, FS_BK32V_ITEMS, FS_BK32V_WAVES)
 FS_BK_KERNELS(k64, true, false, FS_BP64_ITEMS, FS_BK64_ITEMS, FS_BK64_WAVES)
 FS_BK_KERNELS(k64_v, true, true, FS_BP64_ITEMS, FS_BK64V_ITEMS, FS_BK64V_WAVES)
 
+// Two levels.  The partition of the first has at most 256 buckets and larger
+// tiles than one level's, so that a tile's runs of a bucket are long (f64
+// 128M keys: 885 -> 659 us against 512 buckets of 5,120-key tiles).
+#define FS_BK2_KERNELS(sfx, VALS, PITEMS, BITEMS, CITEMS, CWAVES, CGBITS)                                         \
+    extern "C" __global__ void __launch_bounds__(FS_BP_BLOCK) fs_part1_##sfx(FsArgs a) {                          \
+        part_body<true, VALS, FS_BP_BLOCK, PITEMS, 1>(a);                                                         \
+    }                                                                                                             \
+    extern "C" __global__ void __launch_bounds__(FS_BP_BLOCK) fs_part2_##sfx(FsArgs a) {                          \
+        part_body<true, VALS, FS_BP_BLOCK, PITEMS, 2>(a);                                                         \
+    }                                                                                                             \
+    extern "C" __global__ void __launch_bounds__(FS_BC_BLOCK) FS_OCC(CWAVES) fs_child_##sfx(FsArgs a) {           \
+        child_body<true, VALS, FS_BC_BLOCK, CITEMS, CGBITS>(a);                                                   \
+    }                                                                                                             \
+    extern "C" __global__ void __launch_bounds__(FS_BK_BLOCK) FS_OCC(2) fs_rest_##sfx(FsArgs a) {                 \
+        rest_body<true, VALS, FS_BK_BLOCK, BITEMS>(a);                                                            \
+    }
+FS_BK2_KERNELS(k64, false, FS_BP2_64_ITEMS, FS_BK64_ITEMS, FS_BC64_ITEMS, FS_BC64_WAVES, FS_BC_GBITS)
+FS_BK2_KERNELS(k64_v, true, FS_BP2_64V_ITEMS, FS_BK64V_ITEMS, FS_BC64V_ITEMS, FS_BC64V_WAVES, FS_BCV_GBITS)
+
 extern "C" __global__ void __launch_bounds__(FS_BS_BLOCK) fs_split_k32(FsArgs a) {
-    split_body<false, FS_BS_BLOCK, FS_BS_ITEMS>(a);
+    split_body<false, FS_BS_BLOCK, FS_BS_ITEMS, false>(a);
 }
 extern "C" __global__ void __launch_bounds__(FS_BS_BLOCK) fs_split_k64(FsArgs a) {
-    split_body<true, FS_BS_BLOCK, FS_BS_ITEMS>(a);
+    split_body<true, FS_BS_BLOCK, FS_BS_ITEMS, false>(a);
+}
+extern "C" __global__ void __launch_bounds__(FS_BS_BLOCK) fs_split2_k64(FsArgs a) {
+    split_body<true, FS_BS_BLOCK, FS_BS2_ITEMS, true>(a);
 }

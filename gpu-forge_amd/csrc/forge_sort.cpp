@@ -47,13 +47,15 @@ const char* const kKernelNames[] = {
     "fs_local_deferred_k32_w", "fs_local_k64_w", "fs_local_deferred_k64_w", "fs_onesweep_k32_s",
     "fs_onesweep_any_k32_s", "fs_onesweep_k32_vs", "fs_onesweep_k64_s", "fs_onesweep_any_k64_s", "fs_onesweep_k64_vs",
     "fs_split_k32", "fs_split_k64", "fs_part_k32", "fs_part_k32_v", "fs_part_k64", "fs_part_k64_v", "fs_bucket_k32",
-    "fs_bucket_k32_v", "fs_bucket_k64", "fs_bucket_k64_v",
+    "fs_bucket_k32_v", "fs_bucket_k64", "fs_bucket_k64_v", "fs_split2_k64", "fs_part1_k64", "fs_part1_k64_v",
+    "fs_part2_k64", "fs_part2_k64_v", "fs_child_k64", "fs_child_k64_v", "fs_rest_k64", "fs_rest_k64_v",
 };
 enum {
     K_UP32, K_UP64, K_OS32, K_OS32V, K_OS64, K_OS64V, K_IOTA, K_ANY32, K_ANY64, K_SCRATCH_ADDR, K_FIRST32, K_FIRST64,
     K_SAMPLE32, K_SAMPLE64, K_LOCAL32, K_RESCATTER32, K_RESCATTER64, K_LOCAL64, K_DEFER64, K_LOOP64, K_DEFER32,
     K_LOCAL32W, K_DEFER32W, K_LOCAL64W, K_DEFER64W, K_OS32S, K_ANY32S, K_OS32VS, K_OS64S, K_ANY64S, K_OS64VS,
     K_SPLIT32, K_SPLIT64, K_PART32, K_PART32V, K_PART64, K_PART64V, K_BUCKET32, K_BUCKET32V, K_BUCKET64, K_BUCKET64V,
+    K_SPLIT2, K_PART1, K_PART1V, K_PART2, K_PART2V, K_CHILD, K_CHILDV, K_REST, K_RESTV,
     K_COUNT
 };
 // the stable digit-pass kernel and the keys-only first-pass kernel of each variant (FS_VAR_*)
@@ -74,14 +76,16 @@ struct fs_sorter {
     // [wide][64-bit keys] (fs_local_k32, fs_local_k64, fs_local_k32_w, fs_local_k64_w)
     uint32_t local_keys[2][2] = {};
     uint32_t local_block[2][2] = {};
-    // bucket path: threads per block, keys per tile of the partition by
-    // [64-bit keys], keys a block sorts by [64-bit keys][values], most samples
-    // and most buckets
-    uint32_t bk_block = 0, bk_part_block = 0, bk_split_block = 0, bk_tile[2] = {}, bk_cap[2][2] = {}, bk_samples = 0, bk_max = 0;
+    // bucket path: threads per block, most samples and buckets, keys per tile
+    // of the partition and keys a block sorts by [64-bit keys][values]
+    uint32_t bk_block = 0, bk_part_block = 0, bk_split_block = 0, bk_samples = 0, bk_max = 0;
+    uint32_t bk_tile[2][2] = {}, bk_cap[2][2] = {};
+    // ... two levels: a child's threads and keys, most samples of a bucket, keys per tile, by [values]
+    uint32_t bk_child_block = 0, bk_samples2 = 0, bk_child_cap[2] = {}, bk2_tile[2] = {};
     uint32_t local_min_bits32 = 8;  // fewest segment bits whose 32-bit segments fs_local_k32 sorts itself
     int num_cus = 256;
 
-    DevBuf s1k, s2k, s1v, s2v, lb0, lb1, iok, iov, tilemap;
+    DevBuf s1k, s2k, s1v, s2v, lb0, lb1, iok, iov, tilemap, bk2, rest;
     uint32_t* hist = nullptr;       // [FS_HIST_SLOTS][8][256], zero between sorts
     uint32_t* binbase = nullptr;    // [8][256]
     uint32_t* cursors = nullptr;    // [FS_REGIONS] region cursors of the fused pass, zero between sorts
@@ -109,7 +113,7 @@ struct fs_sorter {
     uint32_t fused_mode = 0;             // FS_TEST_FUSED: 0 by size, 1 never, 2 always
     uint32_t top16_mode = 0;             // FS_TEST_TOP16: 0 by size, 1 never, 2 always (even skewed), 3 sampled
     uint32_t seg_bits = 0;               // FS_TEST_SEG_BITS: 0 by size, else the segment bits
-    uint32_t bucket_mode = 0;            // FS_TEST_BUCKETS: 0 by size, 1 never, 2 always one block, 3 always buckets
+    uint32_t bucket_mode = 0;            // FS_TEST_BUCKETS: 0 by size, 1 never, 2 always one block, 3 always buckets, 4 two levels
     uint32_t bucket_lnb = 0;             // ... log2 of the buckets (0: by size)
     uint32_t local_wide_mode = 0;        // FS_TEST_LOCAL_WIDE: 0 by size, 1 wide local-sort blocks
     // the last sort's schedule (the sorter's, or the static scratch's) and
@@ -374,28 +378,35 @@ static bool top16_path(const fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) 
 // The bucket path (bucket_sort.h): sorts that one block does by itself in one
 // launch, and those that a sample, a partition and a block per bucket do in
 // three, where the digit passes take one launch per digit and one more.
-enum BucketPath { BK_NONE, BK_ONE_BLOCK, BK_BUCKETS };
+enum BucketPath { BK_NONE, BK_ONE_BLOCK, BK_BUCKETS, BK_TWO_LEVELS };
 struct BucketLimit {
-    uint64_t one_block, buckets;
+    uint64_t one_block, buckets, two_from, two_to;
 };
 static BucketLimit bucket_limit(fs_op op, fs_key_type t) {
     const bool v = op != FS_OP_SORT;
+    // f64: always; with values, u64 and i64 keys from FS_BK2_MIN_64V on (alone
+    // they have the top-16 path)
+    const bool f64 = t == FS_KEY_F64;
     if (key64(t))
-        return v ? BucketLimit{FS_BK_ONE_64V, FS_BK_MAX_64V} : BucketLimit{FS_BK_ONE_64, FS_BK_MAX_64};
-    return v ? BucketLimit{FS_BK_ONE_32V, FS_BK_MAX_32V} : BucketLimit{FS_BK_ONE_32, FS_BK_MAX_32};
+        return v ? BucketLimit{FS_BK_ONE_64V, FS_BK_MAX_64V, f64 ? 0u : FS_BK2_MIN_64V, FS_BK2_MAX_64V}
+                 : BucketLimit{FS_BK_ONE_64, FS_BK_MAX_64, 0, f64 ? FS_BK2_MAX_64 : 0u};
+    return v ? BucketLimit{FS_BK_ONE_32V, FS_BK_MAX_32V, 0, 0} : BucketLimit{FS_BK_ONE_32, FS_BK_MAX_32, 0, 0};
 }
 static BucketPath bucket_path(const fs_sorter* s, fs_op op, fs_key_type t, uint64_t n, bool no_alloc) {
     if (n < 2 || n >= (1ull << 31)) return BK_NONE;
     const uint32_t cap = s->bk_cap[key64(t) ? 1 : 0][op != FS_OP_SORT ? 1 : 0];
     if (s->bucket_mode == 2u) return n <= cap ? BK_ONE_BLOCK : BK_NONE;
     if (s->bucket_mode == 3u) return no_alloc || n < 64 ? BK_NONE : BK_BUCKETS;
+    if (s->bucket_mode == 4u) return no_alloc || n < 64 || !key64(t) ? BK_NONE : BK_TWO_LEVELS;
     // (the other test options ask for the paths that they are about)
     if (s->bucket_mode == 1u || s->fused_mode || s->top16_mode || s->force_wide || s->up_blocks_per_cu || s->stats_on ||
         s->fault != FS_FAULT_NONE)
         return BK_NONE;
     const BucketLimit lim = bucket_limit(op, t);
     if (n <= lim.one_block && n <= cap) return BK_ONE_BLOCK;
-    return !no_alloc && n <= lim.buckets ? BK_BUCKETS : BK_NONE;
+    if (no_alloc) return BK_NONE;
+    if (n <= lim.buckets) return BK_BUCKETS;
+    return n >= lim.two_from && n <= lim.two_to ? BK_TWO_LEVELS : BK_NONE;
 }
 
 // log2 of the buckets (about FS_BK_MEAN keys each) and of the samples (16 to a
@@ -404,31 +415,61 @@ static BucketPath bucket_path(const fs_sorter* s, fs_op op, fs_key_type t, uint6
 struct BucketShape {
     uint32_t lnb, lm, tile, tiles;
     uint64_t s1_keys;
+    // two levels: log2 of a bucket's children and of its samples, S2 keys per
+    // 256 keys of a bucket, tiles of the second partition, entries of the rest list
+    uint32_t lnb2, lm2, room2, tiles2, rests;
+    uint64_t s2_keys;
 };
-static BucketShape bucket_shape(const fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
+// Keys the regions of nb buckets of m samples take at most, per key of the input.
+static double bucket_room(double nb, double m) {
+    return (m + 6.0 * __builtin_sqrt(m * nb) + (double)FS_BK_ROOM * nb) / m * 1.01;
+}
+static BucketShape bucket_shape(const fs_sorter* s, fs_op op, fs_key_type t, uint64_t n, bool two) {
+    const int w = key64(t) ? 1 : 0, v = op != FS_OP_SORT ? 1 : 0;
     BucketShape b;
-    b.lnb = 3;
-    while ((1u << (b.lnb + 1)) <= s->bk_max && n > ((uint64_t)FS_BK_MEAN << b.lnb)) ++b.lnb;
-    if (s->bucket_lnb) b.lnb = s->bucket_lnb;
-    while ((1u << b.lnb) > s->bk_max) --b.lnb;
-    // samples per bucket: with s of them a bucket outgrows r times its mean
-    // with probability P(Poisson(r s) < s), below 2e-6 for 4 samples and r =
-    // 5.3, 8 and 3.6, 16 and 2.7 (the block of such a bucket then takes long,
-    // but the sort stays exact)
-    const uint32_t cap = s->bk_cap[key64(t) ? 1 : 0][op != FS_OP_SORT ? 1 : 0];
-    const double ratio = (double)cap * (double)(1u << b.lnb) / (double)n;
-    b.lm = b.lnb + (ratio >= 5.3 ? 2 : ratio >= 3.6 ? 3 : ratio >= 2.7 ? 4 : 5);
-    if (b.lm < 9) b.lm = 9;
+    memset(&b, 0, sizeof b);
+    const uint32_t most = (two ? s->bk2_tile[v] : s->bk_tile[w][v]) / s->bk_part_block;
+    uint64_t rows = most;
+    if (two) {
+        // children of half of a block's keys on average, up to two thirds at
+        // the largest sizes (with twice the samples, which then bound them closer)
+        const uint64_t cap = s->bk_child_cap[v], mean = cap / 2;
+        b.lnb = s->bucket_lnb && s->bucket_lnb < FS_BK2_LNB ? s->bucket_lnb : FS_BK2_LNB;
+        b.lnb2 = FS_BK2_LNB < 5u ? FS_BK2_LNB : 5u;
+        while (b.lnb2 < FS_BK2_LNB && n > (mean << (b.lnb + b.lnb2))) ++b.lnb2;
+        while ((1u << b.lm) < s->bk_samples) ++b.lm;
+        b.lm2 = b.lnb2 + ((n >> (b.lnb + b.lnb2)) * 19 > cap * 10 ? 5 : 4);
+        if (b.lm2 < 9) b.lm2 = 9;
+        while ((1u << b.lm2) > s->bk_samples2) --b.lm2;
+    } else {
+        b.lnb = 3;
+        while ((1u << (b.lnb + 1)) <= s->bk_max && n > ((uint64_t)FS_BK_MEAN << b.lnb)) ++b.lnb;
+        if (s->bucket_lnb) b.lnb = s->bucket_lnb;
+        while ((1u << b.lnb) > s->bk_max) --b.lnb;
+        // samples per bucket: with s of them a bucket outgrows r times its mean
+        // with probability P(Poisson(r s) < s), below 2e-6 for 4 samples and r =
+        // 5.3, 8 and 3.6, 16 and 2.7 (the block of such a bucket then takes long,
+        // but the sort stays exact)
+        const double ratio = (double)s->bk_cap[w][v] * (double)(1u << b.lnb) / (double)n;
+        b.lm = b.lnb + (ratio >= 5.3 ? 2 : ratio >= 3.6 ? 3 : ratio >= 2.7 ? 4 : 5);
+        if (b.lm < 9) b.lm = 9;
+        // a tile per CU where the keys suffice, of 1 to all of the partition's keys per thread
+        rows = n / ((uint64_t)s->bk_part_block * (uint64_t)s->num_cus) + 1;
+        if (rows > most) rows = most;
+    }
     while ((1u << b.lm) > s->bk_samples) --b.lm;
-    // a tile per CU where the keys suffice, of 1 to all of the partition's keys per thread
-    const uint32_t most = s->bk_tile[key64(t) ? 1 : 0] / s->bk_part_block;
-    uint64_t rows = n / ((uint64_t)s->bk_part_block * (uint64_t)s->num_cus) + 1;
-    if (rows > most) rows = most;
     b.tile = (uint32_t)rows * s->bk_part_block;
     b.tiles = (uint32_t)((n + b.tile - 1) / b.tile);
-    const double nb = (double)(1u << b.lnb), m = (double)(1u << b.lm);
-    b.s1_keys = (uint64_t)((double)n / m * (m + 6.0 * __builtin_sqrt(m * nb) + (double)FS_BK_ROOM * nb) * 1.01 + 32.0 * nb);
+    const double nb = (double)(1u << b.lnb);
+    b.s1_keys = (uint64_t)((double)n * bucket_room(nb, (double)(1u << b.lm)) + 32.0 * nb);
     if (b.s1_keys < n) b.s1_keys = n;
+    if (two) {
+        const double nb2 = (double)(1u << b.lnb2);
+        b.room2 = (uint32_t)(bucket_room(nb2, (double)(1u << b.lm2)) * 256.0) + 2u;
+        b.s2_keys = ((n * b.room2) >> 8) + (uint64_t)(nb * (32.0 * nb2 + 96.0));
+        b.tiles2 = b.tiles + (1u << b.lnb);
+        b.rests = (uint32_t)((1u << (b.lnb + b.lnb2)) * 2u + n / FS_REST_KEYS + 64u);
+    }
     return b;
 }
 
@@ -461,25 +502,72 @@ static uint32_t seg_bits_for(uint64_t n, uint64_t mean_max) {
     return b;
 }
 
-// Grows the scratch a sort of n keys needs (grow-only, like ensure_buffers*,
-// lib.rs:1120-1289): ping-pong buffers for keys (and values), and two
-// look-back arrays of tile entries followed by one 32-bit group entry per
-// FS_LB_GROUP tiles.
+// Look-back entries of a digit pass.
+static size_t lookback_bytes(const fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
+    const uint32_t tile = s->tile[sort_variant(s, op, t, n, false)];
+    const uint64_t num_tiles = (n + tile - 1) / tile;
+    return (size_t)num_tiles * FS_RADIX * (wide_lookback(s, n) ? 8 : 4) +
+           (size_t)((num_tiles + FS_LB_GROUP - 1) / FS_LB_GROUP) * FS_RADIX * 4;
+}
+
+// Scratch of the bucket path for sorts of up to n keys.  Larger sorts may need
+// less (more samples bound the regions closer), so the sizes here bound every
+// n: regions by the fewest samples a bucket (4) and a child (16) can have, the
+// look-back of one level by a tile per CU.
+static fs_status reserve_buckets(fs_sorter* s, fs_op op, fs_key_type t, uint64_t n, BucketPath bp) {
+    const bool two = bp == BK_TWO_LEVELS;
+    const size_t kb = key_bytes(t);
+    const BucketShape b = bucket_shape(s, op, t, n, two);
+    const double nb = (double)(1u << b.lnb);
+    uint64_t s1 = b.s1_keys, s2 = n;
+    uint64_t tiles = b.tiles > (uint32_t)s->num_cus + 2u ? b.tiles : (uint32_t)s->num_cus + 2u;
+    uint64_t lb = ((tiles + tiles / FS_LB_GROUP + 1) << b.lnb) * 4, rests = 0;
+    fs_status r;
+    if (two) {
+        const double nb2 = (double)(1u << b.lnb2);
+        const uint64_t all = (uint64_t)((double)n * (bucket_room(1.0, 16.0) + 0.02) + nb * (32.0 * nb2 + 96.0));
+        s2 = b.s2_keys > all ? b.s2_keys : all;
+        // (a bucket's groups of the second level start anew: one more for each)
+        const uint64_t lb2 = (((uint64_t)b.tiles2 + b.tiles2 / FS_LB_GROUP + (1u << b.lnb) + 1) << b.lnb2) * 4;
+        const uint64_t digit_lb = lookback_bytes(s, op, t, n);    // or the digit passes
+        if (lb2 > lb) lb = lb2;
+        if (digit_lb > lb) lb = digit_lb;
+        rests = b.rests;
+        if ((r = ensure(s, s->tilemap, (size_t)b.tiles2 * 4)) != FS_OK) return r;
+        if ((r = ensure(s, s->bk2, (size_t)FS_BK2_TAB_WORDS * 4)) != FS_OK) return r;
+        if ((r = ensure(s, s->rest, (size_t)rests * 8)) != FS_OK) return r;
+        if ((r = ensure(s, s->lb1, (size_t)digit_lb)) != FS_OK) return r;
+    } else {
+        const uint64_t all = (uint64_t)((double)n * bucket_room(1.0, 4.0) + 32.0 * nb);
+        if (all > s1) s1 = all;
+    }
+    if ((r = ensure(s, s->s1k, s1 * kb)) != FS_OK) return r;
+    if ((r = ensure(s, s->s2k, s2 * kb)) != FS_OK) return r;
+    if (two || op != FS_OP_SORT)
+        if ((r = ensure(s, s->lb0, (size_t)lb)) != FS_OK) return r;
+    if (op == FS_OP_SORT) return FS_OK;
+    if ((r = ensure(s, s->s1v, s1 * 4)) != FS_OK) return r;
+    return ensure(s, s->s2v, s2 * 4);
+}
+
+// Grows the scratch a sort of n keys needs, and every smaller one (grow-only,
+// like ensure_buffers*, lib.rs:1120-1289): ping-pong buffers for keys (and
+// values), two look-back arrays of tile entries followed by one 32-bit group
+// entry per FS_LB_GROUP tiles, and the bucket path's.
 static fs_status reserve(fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
     if (n <= 1) return FS_OK;
     const size_t kb = key_bytes(t);
     const BucketPath bp = bucket_path(s, op, t, n, false);
     if (bp == BK_ONE_BLOCK) return FS_OK;
-    if (bp == BK_BUCKETS) {
-        const BucketShape b = bucket_shape(s, op, t, n);
-        fs_status r;
-        if ((r = ensure(s, s->s1k, b.s1_keys * kb)) != FS_OK) return r;
-        if ((r = ensure(s, s->s2k, n * kb)) != FS_OK) return r;
-        if (op == FS_OP_SORT) return FS_OK;
-        if ((r = ensure(s, s->s1v, b.s1_keys * 4)) != FS_OK) return r;
-        if ((r = ensure(s, s->s2v, n * 4)) != FS_OK) return r;
-        return ensure(s, s->lb0, ((size_t)b.tiles + (b.tiles + FS_LB_GROUP - 1) / FS_LB_GROUP) * s->bk_max * 4);
+    const BucketLimit lim = bucket_limit(op, t);
+    const uint64_t sizes[2] = {n < lim.buckets ? n : lim.buckets, n < lim.two_to ? n : lim.two_to};
+    for (uint64_t m : sizes) {
+        const BucketPath mp = bucket_path(s, op, t, m, false);
+        fs_status r = FS_OK;
+        if (m < n && (mp == BK_BUCKETS || mp == BK_TWO_LEVELS)) r = reserve_buckets(s, op, t, m, mp);
+        if (r != FS_OK) return r;
     }
+    if (bp != BK_NONE) return reserve_buckets(s, op, t, n, bp);
     const uint32_t tile = s->tile[sort_variant(s, op, t, n, false)];
     const uint64_t num_tiles = (n + tile - 1) / tile;
     fs_status r;
@@ -491,8 +579,7 @@ static fs_status reserve(fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
         if ((r = ensure(s, s->s1v, n * 4)) != FS_OK) return r;
         if (op == FS_OP_PAIRS && (r = ensure(s, s->s2v, n * 4)) != FS_OK) return r;
     }
-    const size_t lb_bytes = (size_t)num_tiles * FS_RADIX * (wide_lookback(s, n) ? 8 : 4) +
-                            (size_t)((num_tiles + FS_LB_GROUP - 1) / FS_LB_GROUP) * FS_RADIX * 4;
+    const size_t lb_bytes = lookback_bytes(s, op, t, n);
     if ((r = ensure(s, s->lb0, lb_bytes)) != FS_OK) return r;
     return ensure(s, s->lb1, lb_bytes);
 }
@@ -521,11 +608,55 @@ static ScratchSet static_scratch(const fs_sorter* s) {
                       p + FS_NA_OFF_RTABLE, 0};   // (no top-16 path on the static scratch)
 }
 
+// The arguments of a sort's digit passes; returns the upsweep's blocks.
+static uint64_t digit_args(const fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint32_t* vals, uint64_t n,
+                           const ScratchSet& sc, uint32_t tile, bool wide, FsArgs& a) {
+    memset(&a, 0, sizeof a);
+    a.n = n;
+    a.key64 = key64(t) ? 1u : 0u;
+    a.xform = xform_of(t);
+    a.op = op == FS_OP_SORT ? FSK_OP_KEYS : (op == FS_OP_ARGSORT ? FSK_OP_ARGSORT : FSK_OP_PAIRS);
+    a.digits = key64(t) ? 8u : 4u;     // one 8-bit digit per key byte
+    a.num_tiles = (uint32_t)((n + tile - 1) / tile);
+    a.wide = wide ? 1u : 0u;
+    a.tile = tile;
+    a.vec_ok = ((uintptr_t)keys % 16 == 0) ? 1u : 0u;
+    // upsweep: 1 block per CU for 32-bit keys (measured faster than 2: fewer
+    // counter clears, folds and histogram atomics for the same keys), 2 for
+    // 64-bit keys (the blocks' 64 KiB of counters allow two resident); fewer
+    // when the keys give each block less than one step of FS_UPSWEEP_UNROLL
+    // units per thread (a test option can set the blocks per CU)
+    const uint64_t up_per_cu = s->up_blocks_per_cu ? s->up_blocks_per_cu : (key64(t) ? 2u : 1u);
+    const uint64_t up_units = a.vec_ok ? n / (16u / key_bytes(t)) : n;
+    const uint64_t up_span = (uint64_t)FS_UPSWEEP_UNROLL * FS_HIST_BLOCK;
+    uint64_t up_blocks = (up_units + up_span - 1) / up_span;
+    if (up_blocks > (uint64_t)s->num_cus * up_per_cu) up_blocks = (uint64_t)s->num_cus * up_per_cu;
+    if (up_blocks == 0) up_blocks = 1;
+    a.keys = (uint64_t)(uintptr_t)keys;
+    a.vals = (uint64_t)(uintptr_t)vals;
+    a.s1k = sc.s1k;
+    a.s2k = sc.s2k;
+    a.s1v = sc.s1v;
+    a.s2v = sc.s2v;
+    a.hist = sc.hist;
+    a.binbase = sc.binbase;
+    a.lookback0 = sc.lb0;
+    a.lookback1 = sc.lb1;
+    a.plan = sc.plan;
+    a.cursors = sc.cursors;
+    a.rstart = sc.rstart;
+    a.tilemap = sc.tilemap;
+    a.rtable = sc.rtable;
+    a.status = (uint64_t)(uintptr_t)s->status;
+    a.stats = s->stats_on ? (uint64_t)(uintptr_t)s->stats : 0u;
+    return up_blocks;
+}
+
 // The launches of the bucket path.
 static fs_status enqueue_buckets(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint32_t* vals, uint64_t n,
                                  hipStream_t st, BucketPath bp, bool no_alloc) {
     fs_status r;
-    if (bp == BK_BUCKETS && (r = reserve(s, op, t, n)) != FS_OK) return r;
+    if (bp != BK_ONE_BLOCK && (r = reserve(s, op, t, n)) != FS_OK) return r;
     const ScratchSet sc = no_alloc ? static_scratch(s) : sorter_scratch(s);
     const bool v = op != FS_OP_SORT, k64 = key64(t);
     FsArgs a;
@@ -545,7 +676,8 @@ static fs_status enqueue_buckets(fs_sorter* s, fs_op op, fs_key_type t, void* ke
     if (bp == BK_ONE_BLOCK) {
         if ((r = launch(s, kbucket, 1, s->bk_block, args, st, no_alloc)) != FS_OK) return r;
     } else {
-        const BucketShape b = bucket_shape(s, op, t, n);
+        const bool two = bp == BK_TWO_LEVELS;
+        const BucketShape b = bucket_shape(s, op, t, n, two);
         a.s1k = sc.s1k;
         a.s1v = sc.s1v;
         a.s2k = sc.s2k;
@@ -556,18 +688,59 @@ static fs_status enqueue_buckets(fs_sorter* s, fs_op op, fs_key_type t, void* ke
         a.s1_keys = (uint32_t)b.s1_keys;
         a.bk_lnb = b.lnb;
         a.bk_lm = b.lm;
+        if (two) {
+            a.tilemap = sc.tilemap;
+            a.bk2_lnb = b.lnb2;
+            a.bk2_lm = b.lm2;
+            a.bk2_room = b.room2;
+            a.s2_keys = (uint32_t)b.s2_keys;
+            a.tiles2 = b.tiles2;
+            a.rest_cap = b.rests;
+            a.bk2_tab = (uint64_t)(uintptr_t)s->bk2.p;
+            a.rest = (uint64_t)(uintptr_t)s->rest.p;
+        }
 #ifdef FS_FAULT_INJECTION
         a.fault = s->fault;
 #endif
-        const int kpart = k64 ? (v ? K_PART64V : K_PART64) : (v ? K_PART32V : K_PART32);
-        if ((r = launch(s, k64 ? K_SPLIT64 : K_SPLIT32, 1, s->bk_split_block, args, st)) != FS_OK) return r;
+        const int sel = v ? 1 : 0;
+        if (two) {
+            // the upsweep, which chooses, then the digit passes in slots 0 .. FS_BK2_FEW_DIGITS - 1
+            // (idle, each returns at once) before the buckets, since their
+            // schedule step hands a sort back when more digits vary than the
+            // sample showed
+            const int var = sort_variant(s, op, t, n, false);
+            FsArgs d;
+            const uint64_t up_blocks = digit_args(s, op, t, keys, vals, n, sc, s->tile[var], false, d);
+            d.bk2_tab = a.bk2_tab;
+            d.bk2_choose = 1u;
+            void* dargs[] = {&d};
+            if ((r = launch(s, K_UP64, (unsigned)up_blocks, FS_HIST_BLOCK, dargs, st)) != FS_OK) return r;
+            for (uint32_t sl = 0; sl < FS_BK2_FEW_DIGITS; ++sl) {
+                void* pargs[] = {&d, &sl};
+                // (a keys-only sort's first pass needs no stability)
+                const int k = sl == 0 && !v ? kAnyKernel[var] : kPassKernel[var];
+                if ((r = launch(s, k, d.num_tiles, s->block[var], pargs, st)) != FS_OK) return r;
+            }
+        }
+        // (with values, many tiles' look-back entries: cleared by more blocks than the sampling one)
+        const unsigned clear = v && b.tiles > 256 ? 1u + (unsigned)s->num_cus / 4u : 1u;
+        if ((r = launch(s, k64 ? K_SPLIT64 : K_SPLIT32, clear, s->bk_split_block, args, st)) != FS_OK) return r;
+        const int kpart = two ? K_PART1 + sel : (k64 ? K_PART64 : K_PART32) + sel;
         if ((r = launch(s, kpart, b.tiles, s->bk_part_block, args, st)) != FS_OK) return r;
-        if ((r = launch(s, kbucket, 1u << b.lnb, s->bk_block, args, st)) != FS_OK) return r;
+        if (!two) {
+            if ((r = launch(s, kbucket, 1u << b.lnb, s->bk_block, args, st)) != FS_OK) return r;
+        } else {
+            if ((r = launch(s, K_SPLIT2, 1u << b.lnb, s->bk_split_block, args, st)) != FS_OK) return r;
+            if ((r = launch(s, K_PART2 + sel, b.tiles2, s->bk_part_block, args, st)) != FS_OK) return r;
+            if ((r = launch(s, K_CHILD + sel, 1u << (b.lnb + b.lnb2), s->bk_child_block, args, st)) != FS_OK) return r;
+            if ((r = launch(s, K_REST + sel, (unsigned)s->num_cus, s->bk_block, args, st)) != FS_OK) return r;
+        }
     }
     s->last_stream = st;
     s->pending = true;
     s->last_plan = (uint32_t*)(uintptr_t)sc.plan;
-    s->last_fused = false;
+    // (a sort of the fused range whose first pass scatters into regions)
+    s->last_fused = bp == BK_TWO_LEVELS && op == FS_OP_SORT && n >= FS_FUSED_MIN_KEYS;
     s->last_top16 = false;
     return FS_OK;
 }
@@ -625,42 +798,7 @@ static fs_status enqueue(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint
                                  (!no_alloc || FS_FUSED_S1_KEYS(sub_keys) * kb <= (uint64_t)FS_NA_MAX_KEYS * 8));
 
     FsArgs a;
-    memset(&a, 0, sizeof a);
-    a.n = n;
-    a.key64 = key64(t) ? 1u : 0u;
-    a.xform = xform_of(t);
-    a.op = op == FS_OP_SORT ? FSK_OP_KEYS : (op == FS_OP_ARGSORT ? FSK_OP_ARGSORT : FSK_OP_PAIRS);
-    a.digits = key64(t) ? 8u : 4u;     // one 8-bit digit per key byte
-    a.num_tiles = num_tiles;
-    a.wide = wide ? 1u : 0u;
-    a.tile = tile;
-    a.vec_ok = ((uintptr_t)keys % 16 == 0) ? 1u : 0u;
-    // upsweep: 1 block per CU for 32-bit keys (measured faster than 2: fewer
-    // counter clears, folds and histogram atomics for the same keys), 2 for
-    // 64-bit keys (the blocks' 64 KiB of counters allow two resident); fewer
-    // when the keys give each block less than one step of FS_UPSWEEP_UNROLL
-    // units per thread (a test option can set the blocks per CU)
-    const uint64_t up_per_cu = s->up_blocks_per_cu ? s->up_blocks_per_cu : (key64(t) ? 2u : 1u);
-    const uint64_t up_units = a.vec_ok ? n / (16u / key_bytes(t)) : n;
-    const uint64_t up_span = (uint64_t)FS_UPSWEEP_UNROLL * FS_HIST_BLOCK;
-    uint64_t up_blocks = (up_units + up_span - 1) / up_span;
-    if (up_blocks > (uint64_t)s->num_cus * up_per_cu) up_blocks = (uint64_t)s->num_cus * up_per_cu;
-    if (up_blocks == 0) up_blocks = 1;
-    a.keys = (uint64_t)(uintptr_t)keys;
-    a.vals = (uint64_t)(uintptr_t)vals;
-    a.s1k = sc.s1k;
-    a.s2k = sc.s2k;
-    a.s1v = sc.s1v;
-    a.s2v = sc.s2v;
-    a.hist = sc.hist;
-    a.binbase = sc.binbase;
-    a.lookback0 = sc.lb0;
-    a.lookback1 = sc.lb1;
-    a.plan = sc.plan;
-    a.cursors = sc.cursors;
-    a.rstart = sc.rstart;
-    a.tilemap = sc.tilemap;
-    a.rtable = sc.rtable;
+    const uint64_t up_blocks = digit_args(s, op, t, keys, vals, n, sc, tile, wide, a);
     a.fused = fused ? 1u : 0u;
     a.sub_keys = fused ? (uint32_t)sub_keys : 0u;
     a.s1_keys = fused ? (uint32_t)FS_FUSED_S1_KEYS(sub_keys) : 0u;
@@ -678,8 +816,6 @@ static fs_status enqueue(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint
     // a segment the region sample estimates above 16 blocks' keys sends the
     // sort to the LSD passes (unless a test forces the top-16 path)
     a.seg_limit = s->top16_mode == 2u ? 0xFFFFFFFFu : 16u * local_keys_of(s, t, wide_local);
-    a.status = (uint64_t)(uintptr_t)s->status;
-    a.stats = s->stats_on ? (uint64_t)(uintptr_t)s->stats : 0u;
 #ifdef FS_FAULT_INJECTION
     a.fault = s->fault;
     if (s->fault == FS_FAULT_BAD_DIGITS) a.digits = 5u;
@@ -883,18 +1019,25 @@ static fs_status create(int device, hipStream_t stream, bool own, fs_sorter** ou
         s->local_min_bits32 = lg[4];
         hipDeviceptr_t kp = nullptr;
         size_t ksz = 0;
-        uint32_t bg[11] = {};
+        uint32_t bg[FS_BG_WORDS] = {};
         if (hipModuleGetGlobal(&kp, &ksz, s->module, "fs_kernel_bucket_geometry") != hipSuccess ||
-            ksz != sizeof(bg) || hipMemcpyDtoH(bg, kp, sizeof(bg)) != hipSuccess || bg[0] < FS_RADIX || bg[8] != FS_BK_NB)
+            ksz != sizeof(bg) || hipMemcpyDtoH(bg, kp, sizeof(bg)) != hipSuccess || bg[0] < FS_RADIX || bg[6] != FS_BK_NB)
             return create_failed(s, FS_ERR_SHADER_COMPILATION, "code object lacks a valid fs_kernel_bucket_geometry");
         s->bk_block = bg[0];
-        s->bk_tile[0] = bg[1];
-        s->bk_tile[1] = bg[2];
-        for (int i = 0; i < 4; ++i) s->bk_cap[i / 2][i % 2] = bg[3 + i];
-        s->bk_samples = bg[7];
-        s->bk_max = bg[8];
-        s->bk_part_block = bg[9];
-        s->bk_split_block = bg[10];
+        s->bk_part_block = bg[1];
+        s->bk_split_block = bg[2];
+        s->bk_child_block = bg[3];
+        s->bk_samples = bg[4];
+        s->bk_samples2 = bg[5];
+        s->bk_max = bg[6];
+        for (int i = 0; i < 4; ++i) {
+            s->bk_cap[i / 2][i % 2] = bg[7 + i];
+            s->bk_tile[i / 2][i % 2] = bg[11 + i];
+        }
+        for (int i = 0; i < 2; ++i) {
+            s->bk_child_cap[i] = bg[15 + i];
+            s->bk2_tile[i] = bg[17 + i];
+        }
     }
     const size_t tab = (size_t)FS_MAX_DIGITS * FS_RADIX * 4;
     if (hipMalloc(&s->hist, (size_t)FS_HIST_WORDS * 4) != hipSuccess || hipMalloc(&s->binbase, tab) != hipSuccess ||
@@ -950,7 +1093,7 @@ void fs_sorter_free(fs_sorter* s) {
     if (s->stream || s->own_stream) (void)hipStreamSynchronize(s->stream);
     recycle_profile(s);
     for (hipEvent_t e : s->event_pool) (void)hipEventDestroy(e);
-    DevBuf* bufs[] = {&s->s1k, &s->s2k, &s->s1v, &s->s2v, &s->lb0, &s->lb1, &s->iok, &s->iov, &s->tilemap};
+    DevBuf* bufs[] = {&s->s1k, &s->s2k, &s->s1v, &s->s2v, &s->lb0, &s->lb1, &s->iok, &s->iov, &s->tilemap, &s->bk2, &s->rest};
     for (DevBuf* b : bufs) free_buf(*b);
     if (s->hist) (void)hipFree(s->hist);
     if (s->cursors) (void)hipFree(s->cursors);
@@ -1113,7 +1256,7 @@ fs_status fs_sorter_set_test_option(fs_sorter* s, fs_test_option opt, uint64_t v
             s->local_wide_mode = (uint32_t)value;
             return FS_OK;
         case FS_TEST_BUCKETS:
-            if ((value & 0xFFu) > 3u || (value >> 8) > 16u)
+            if ((value & 0xFFu) > 4u || (value >> 8) > 16u)
                 return set_err(s, FS_ERR_INVALID_ARGUMENT, "bucket choice %llu", (unsigned long long)value);
             s->bucket_mode = (uint32_t)(value & 0xFFu);
             s->bucket_lnb = (uint32_t)(value >> 8);
@@ -1130,7 +1273,7 @@ fs_status fs_sorter_set_test_option(fs_sorter* s, fs_test_option opt, uint64_t v
             return FS_OK;
         case FS_TEST_INJECT_FAULT:
 #ifdef FS_FAULT_INJECTION
-            if (value > FS_FAULT_SMALL_REGIONS) return set_err(s, FS_ERR_INVALID_ARGUMENT, "unknown fault %llu",
+            if (value > FS_FAULT_SMALL_REGIONS2) return set_err(s, FS_ERR_INVALID_ARGUMENT, "unknown fault %llu",
                                                            (unsigned long long)value);
             s->fault = (uint32_t)value;
             return FS_OK;

@@ -407,17 +407,32 @@
 #define FS_BK_GBITS 12
 #endif
 #define FS_BK_GLIM(wide, vals) ((wide) ? ((vals) ? 32u : 40u) : ((vals) ? 16u : 24u))
-// Largest sorts that one block does alone, and that buckets do, by key width
-// and values (V); keys a bucket is meant to hold
+// Largest sorts that one block does alone, that buckets do, and that two
+// levels of buckets do (64-bit keys), by key width and values (V).  Where the
+// digit passes are as fast (us, buckets against passes, keys in place):
+// 32-bit keys of few values, f32, 1.1M: 66 / 67 (uniform 48 / 67); with values
+// u32 argsort, 20 varying bits, 0.7M: 52 / 51 (0.5M: 42 / 49); 64-bit keys with
+// values of 20 bits, 1M: 64 / 66 (uniform 68 / 136).  Two levels: f64 from
+// there on (3M: sort 170 / 190, argsort 163 / 184; 128M: 2,496 / 4,567), but
+// u64 and i64 with values from FS_BK2_MIN_64V: those of few varying digits,
+// which go back to the passes, pay 8 to 10 us for the launches that find
+// nothing to do (12M pairs: 329 / 321 for 20 bits, 420 / 671 uniform).  The
+// largest: 65,536 children of 3,072 keys (2,048 with values) each have room
+// for 1.4 times (1.7) their mean; those that need more are sorted by fs_rest_*.
 #ifndef FS_BK_ONE_32
 #define FS_BK_ONE_32 8192u
 #define FS_BK_ONE_32V 8192u
 #define FS_BK_ONE_64 8192u
 #define FS_BK_ONE_64V 6144u
-#define FS_BK_MAX_32 1500000u
-#define FS_BK_MAX_32V 1500000u
+#define FS_BK_MAX_32 1100000u
+#define FS_BK_MAX_32V 600000u
 #define FS_BK_MAX_64 1500000u
-#define FS_BK_MAX_64V 1100000u
+#define FS_BK_MAX_64V 1000000u
+#define FS_BK2_MAX_64 140000000u
+#define FS_BK2_MAX_64V 80000000u
+#endif
+#ifndef FS_BK2_MIN_64V
+#define FS_BK2_MIN_64V 12000000u
 #endif
 #ifndef FS_BK_MEAN
 #define FS_BK_MEAN 2048u
@@ -436,7 +451,65 @@
 #define FS_BK_BITS (FS_BK_CAPS + FS_BK_NB)
 #define FS_BK_BIT_SLOTS 16u
 #define FS_BK_LB (FS_BK_BITS + 4u * FS_BK_BIT_SLOTS)
-#define FS_BK_TAB_WORDS (FS_BK_LB + 2u * FS_BK_NB)
+// ... and how a key's bucket follows from its group: whether it does, by value
+// or by bits, the shift, then (two words each) the base, the span, the least
+// value and the scale; then 16 bits for each pair of groups, the splitters in
+// smaller pairs
+#define FS_BK_MAP_HEAD 12u
+#define FS_BK_MAP_WORDS (FS_BK_MAP_HEAD + (1u << (FS_BK_GBITS - 2)))
+#define FS_BK_MAP (FS_BK_LB + 2u * FS_BK_NB)
+#define FS_BK_TAB_WORDS (FS_BK_MAP + FS_BK_MAP_WORDS)
+// Two levels: children of a bucket, and the threads, keys per thread, group
+// bits and waves per SIMD of the blocks that sort them
+#ifndef FS_BK2_LNB
+#define FS_BK2_LNB 8
+#endif
+#define FS_BK2_NB (1u << FS_BK2_LNB)
+#ifndef FS_BC_BLOCK
+#define FS_BC_BLOCK 256
+#endif
+#ifndef FS_BC_GBITS
+#define FS_BC_GBITS 11
+#define FS_BCV_GBITS 10
+#endif
+#ifndef FS_BC64_ITEMS
+#define FS_BC64_ITEMS 12
+#define FS_BC64V_ITEMS 8
+#define FS_BS2_ITEMS 8
+#define FS_BP2_64_ITEMS 7
+#define FS_BP2_64V_ITEMS 5
+#endif
+#define FS_BC64_WAVES 5
+#define FS_BC64V_WAVES 5
+// Second-level table words: 1 when a first-level region overflowed, entries
+// of the rest list, the path taken, then per bucket its description (keys, S1 region, place in
+// the output, first tile, 1: one value), and per child the count, region base,
+// capacity and splitter
+#define FS_BK2_OVER 0u
+#define FS_BK2_RESTS 1u
+#define FS_BK2_MODE 2u             // 0: buckets; 1: digit passes (few digits vary)
+#define FS_BK2_INFO 4u
+#define FS_BK2_INFO_WORDS 8u
+#define FS_BK2_CHILDREN (FS_BK_NB * FS_BK2_NB)
+#define FS_BK2_CNT (FS_BK2_INFO + FS_BK_NB * FS_BK2_INFO_WORDS)
+#define FS_BK2_BASE (FS_BK2_CNT + FS_BK2_CHILDREN)
+#define FS_BK2_CAPS (FS_BK2_BASE + FS_BK2_CHILDREN)
+#define FS_BK2_LB (FS_BK2_CAPS + FS_BK2_CHILDREN)
+#define FS_BK2_MAP (FS_BK2_LB + 2u * FS_BK2_CHILDREN)
+#define FS_BK2_TAB_WORDS (FS_BK2_MAP + FS_BK_NB * FS_BK_MAP_WORDS)
+// Sorts of the two-level sizes launch both the digit passes (this many of
+// them) and the buckets: keys of which at most this many digits vary in a
+// sample take the passes, the others the buckets, and the launches of the
+// other side return at once.  (u64 pairs, 16M keys: the passes take 47 us and
+// 100 a digit, the buckets 480; f64 keys alone: 47 and 70 against 355.)
+#define FS_BK2_FEW_DIGITS 4u
+// Rest list entries: child (or a bucket's first child) and what to do: sort
+// it, sort its bucket from S1, or copy piece i (FS_REST_KEYS keys) of a child
+// of one value
+#define FS_REST_SORT 0xFFFFFFFFu
+#define FS_REST_BUCKET 0xFFFFFFFEu
+#define FS_REST_KEYS 4096u
+#define FS_BG_WORDS 19             // fs_kernel_bucket_geometry
 
 // Error bits additionally reported through the status word.
 #define FS_DEVERR_BAD_TILE 2u        // a digit pass block mapped to a tile >= num_tiles
@@ -456,6 +529,8 @@
 
 #define FS_FAULT_SMALL_REGIONS 6u  // the bucket path's region of bucket 1 gets one row's room (no error; the sort
                                    // stays exact, done by one block)
+
+#define FS_FAULT_SMALL_REGIONS2 7u // the same for child 1 of every bucket, of two levels
 
 // Scratch of the entry point that allocates nothing (fs_encode_no_alloc): a
 // file-scope static device array of FS_NA_SCRATCH_BYTES in the code object,
@@ -530,7 +605,14 @@ typedef struct FsArgs {
     uint32_t bk_lnb;            // bucket path: log2 of the buckets (0: one block sorts everything)
     uint64_t bk_tab;            // u32[FS_BK_TAB_WORDS] bucket table
     uint32_t bk_lm;             // log2 of the samples
-    uint32_t reserved0;
+    uint32_t bk2_lnb, bk2_lm;   // two levels: log2 of a bucket's children, of its samples
+    uint32_t bk2_room;          // S2 keys per key of a bucket, times 256
+    uint32_t s2_keys;           // keys S2 holds for the children's regions
+    uint32_t tiles2;            // second-level tiles (at most)
+    uint32_t rest_cap;          // entries the rest list holds
+    uint64_t bk2_tab;           // u32[FS_BK2_TAB_WORDS] second-level table (0: one level)
+    uint64_t rest;              // u32[rest_cap][2] rest list
+    uint32_t bk2_choose;        // 1: a sort that launches two levels of buckets and the digit passes
 } FsArgs;
 
 // Look-back statistics (accumulated only when FsArgs.stats is set).

@@ -273,6 +273,22 @@ DEV uint32_t slot_in_digit(uint32_t* hist, uint32_t d, uint32_t lane, bool valid
     return in_grp ? lanes_below(grp, gbase) : old;
 }
 
+// Position of sample s of 2^lm of n > 0 keys: hashed, within the s-th of as many parts.
+DEV uint32_t sample_position(uint32_t s, uint32_t lm, uint32_t n) {
+    const uint64_t p0 = ((uint64_t)s * n) >> lm, p1 = ((uint64_t)(s + 1u) * n) >> lm;
+    const uint32_t h = (s * 0x9E3779B9u) ^ ((s * 0x85EBCA6Bu) >> 13);
+    const uint64_t p = p0 + (((uint64_t)h * (p1 - p0)) >> 32);
+    return p < n ? (uint32_t)p : n - 1u;
+}
+
+// Sorts that launch the digit passes and two levels of buckets
+// (FS_BK2_FEW_DIGITS): the buckets do the sort.  (One thread writes this.)
+DEV void leave_to_buckets(const FsArgs& a) {
+    for (uint32_t i = 0; i < FS_PLAN_WORDS; ++i)
+        if (i != FS_PLAN_TICKET) st_agent(gptr<uint32_t>(a.plan) + i, 0u);
+    st_agent(gptr<uint32_t>(a.bk2_tab) + FS_BK2_MODE, 0u);
+}
+
 template <bool K64>
 DEV void upsweep_body(const FsArgs& a) {
     typedef typename KeyT<K64>::type K;
@@ -292,8 +308,20 @@ DEV void upsweep_body(const FsArgs& a) {
     static_assert(R == 16 || R == 32, "replicas");
     static_assert((B / R) * (FS_UP_CHUNK_STEPS * KPV + 1) <= 0xFFFFu, "16-bit counters");
     __shared__ uint32_t h[P][FS_RADIX][R];
-
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
+
+    // Sorts that may go to the buckets: every block looks at the same sample
+    // (the loads are in flight while the counters are cleared).
+    K ref = 0, probe = 0;
+    __shared__ uint32_t s_vary;
+    if (K64 && a.bk2_choose) {
+        constexpr uint32_t LB = __builtin_ctz(B);
+        static_assert(B == 1u << LB, "a sample per thread");
+        const GLOBAL K* keys = gptr<const K>(a.keys);
+        ref = keys[sample_position(0u, LB, (uint32_t)a.n)];
+        probe = keys[sample_position(tid, LB, (uint32_t)a.n)];
+        if (tid == 0) s_vary = 0u;
+    }
     for (uint32_t i = tid; i < P * FS_RADIX * R; i += B) (&h[0][0][0])[i] = 0u;
 
     // Clear the look-back array (tile and group entries) the first executed
@@ -306,6 +334,19 @@ DEV void upsweep_body(const FsArgs& a) {
             st_agent(&lb[i], 0u);
     }
     __syncthreads();
+    if (K64 && a.bk2_choose) {
+        const K v = xf_fwd<K64>(probe, a.xform) ^ xf_fwd<K64>(ref, a.xform);
+        uint32_t mine = 0;                               // digits that vary within the wave's samples
+#pragma unroll
+        for (uint32_t j = 0; j < 8u; ++j)
+            mine |= __builtin_amdgcn_uicmp((uint32_t)((uint64_t)v >> (8u * j)) & 0xFFu, 0u, 33) ? 1u << j : 0u;
+        if (lane == 0u) atomicOr(&s_vary, mine);
+        __syncthreads();
+        if ((uint32_t)__builtin_popcount(s_vary) > FS_BK2_FEW_DIGITS) {   // (uniform over the grid)
+            if (blockIdx.x == 0 && tid == 0) leave_to_buckets(a);
+            return;
+        }
+    }
 
     const GLOBAL K* src = gptr<const K>(a.keys);
     const GLOBAL uint4* src4 = (const GLOBAL uint4*)src;
@@ -499,6 +540,16 @@ DEV void write_schedule(const FsArgs& a, uint32_t cmask, uint32_t D) {
         uint32_t p = 0, mask = 0;
         for (uint32_t j = 0; j < D; ++j)
             if (active[j]) { ++p; mask |= 1u << j; }
+        if (a.bk2_choose) {
+            if (p > FS_BK2_FEW_DIGITS) {                 // more digits vary than the sample showed
+                leave_to_buckets(a);
+                return;
+            }
+            st_agent(gptr<uint32_t>(a.bk2_tab) + FS_BK2_MODE, 1u);
+        }
+        // Fewer launch slots than digits: the passes that run take slots in
+        // order, after a copy if there is one.
+        const bool compact = a.bk2_choose != 0u;
 
         // Destination of executed pass e for keys (dk) and values (dv).
         uint32_t dk[FS_MAX_DIGITS], dv[FS_MAX_DIGITS];
@@ -532,7 +583,7 @@ DEV void write_schedule(const FsArgs& a, uint32_t cmask, uint32_t D) {
         uint32_t single_digit = 0;
         for (uint32_t j = D; j-- > 0;)
             if (active[j]) single_digit = j;
-        const bool copy_before = single && single_digit > 0u;
+        const bool copy_before = single && (compact || single_digit > 0u);
         const bool pairs = a.op == FSK_OP_PAIRS;
         uint32_t duty_digit = FS_MAX_DIGITS, duty = FS_DUTY_NONE, duty_ids = 0;
         if (p == 0u && a.op == FSK_OP_ARGSORT) {
@@ -540,7 +591,7 @@ DEV void write_schedule(const FsArgs& a, uint32_t cmask, uint32_t D) {
             duty = FS_DUTY_IOTA;
             duty_ids = FS_BUF_VALS << 24;
         } else if (copy_before) {
-            duty_digit = single_digit - 1u;
+            duty_digit = compact ? 0u : single_digit - 1u;
             duty = FS_DUTY_COPY;
             duty_ids = FS_BUF_KEYS | (FS_BUF_S1K << 8) | (pairs ? (FS_BUF_VALS << 16) | (FS_BUF_S1V << 24) : 0u);
         } else if (single) {
@@ -549,8 +600,14 @@ DEV void write_schedule(const FsArgs& a, uint32_t cmask, uint32_t D) {
             duty_ids = FS_BUF_S1K | (FS_BUF_KEYS << 8) | (pairs ? (FS_BUF_S1V << 16) | (FS_BUF_VALS << 24) : 0u);
         }
         uint32_t e = 0;
+        uint32_t slot = compact && duty != FS_DUTY_NONE ? 1u : 0u;
+        if (slot) {
+            st_agent(&plan[0], duty << 24);
+            st_agent(&plan[1], duty_ids);
+        }
         for (uint32_t j = 0; j < FS_MAX_DIGITS; ++j) {
             uint32_t w0 = 0, w1 = 0;
+            if (compact && !(j < D && active[j])) continue;
             if (j < D && active[j]) {
                 const uint32_t flags = (e == 0 ? FS_PASS_FIRST : 0u) | (e + 1 == p ? FS_PASS_LAST : 0u) |
                                        ((cmask >> j) & FS_SKEW_BIT ? FS_PASS_SKEWED : 0u);
@@ -571,9 +628,11 @@ DEV void write_schedule(const FsArgs& a, uint32_t cmask, uint32_t D) {
                 w0 = duty << 24;
                 w1 = duty_ids;
             }
-            st_agent(&plan[j * FS_PLAN_PASS_WORDS], w0);
-            st_agent(&plan[j * FS_PLAN_PASS_WORDS + 1], w1);
+            const uint32_t at = (compact ? slot++ : j) * FS_PLAN_PASS_WORDS;
+            st_agent(&plan[at], w0);
+            st_agent(&plan[at + 1], w1);
         }
+        for (; compact && slot < FS_BK2_FEW_DIGITS; ++slot) st_agent(&plan[slot * FS_PLAN_PASS_WORDS], 0u);
         st_agent(&plan[FS_PLAN_NPASSES], p);
         st_agent(&plan[FS_PLAN_MASK], mask);
         st_agent(&plan[FS_PLAN_LOCAL], 0u);
@@ -680,9 +739,10 @@ DEV void rank_wave(const uint32_t (&x)[ITEMS], uint32_t xshift, uint16_t* wb, Ra
 // that is published; it stops at the first INC or at tile 0 (which publishes
 // INC).  Then it publishes this tile's INC.  Every wait is bounded
 // (FS_SPIN_LIMIT).  WIDE selects the 64-bit tile entries.
-template <bool WIDE, uint32_t RADIX = FS_RADIX>
+template <bool WIDE>
 DEV uint32_t lookback(GLOBAL uint32_t* lb, const GLOBAL uint32_t* grp, uint32_t tile, uint32_t d,
-                      uint32_t valid, uint64_t status, uint32_t& rounds, uint32_t& stalls, uint32_t& entries) {
+                      uint32_t valid, uint64_t status, uint32_t& rounds, uint32_t& stalls, uint32_t& entries,
+                      uint32_t radix = FS_RADIX) {
     typedef LbEntry<WIDE> E;
     uint32_t excl = 0;
     uint32_t spins = 0;
@@ -707,7 +767,7 @@ DEV uint32_t lookback(GLOBAL uint32_t* lb, const GLOBAL uint32_t* grp, uint32_t 
         typename E::type e[FS_LB_WINDOW];
 #pragma unroll
         for (int j = 0; j < FS_LB_WINDOW; ++j)
-            e[j] = (j < (int)avail) ? E::load(lb, (uint64_t)(t - 1 - j) * RADIX + d) : 0u;
+            e[j] = (j < (int)avail) ? E::load(lb, (uint64_t)(t - 1 - j) * radix + d) : 0u;
         uint32_t used = 0;
         bool stalled = false;
 #pragma unroll
@@ -735,8 +795,8 @@ DEV uint32_t lookback(GLOBAL uint32_t* lb, const GLOBAL uint32_t* grp, uint32_t 
 #pragma unroll
         for (int j = 0; j < FS_LB_GWIN; ++j) {
             const uint64_t gg = g - 1 - j;
-            ei[j] = (j < (int)avail) ? E::load(lb, (gg * FS_LB_GROUP + FS_LB_GROUP - 1) * RADIX + d) : 0u;
-            eg[j] = (j < (int)avail) ? ld_agent(&grp[gg * RADIX + d]) : 0u;
+            ei[j] = (j < (int)avail) ? E::load(lb, (gg * FS_LB_GROUP + FS_LB_GROUP - 1) * radix + d) : 0u;
+            eg[j] = (j < (int)avail) ? ld_agent(&grp[gg * radix + d]) : 0u;
         }
         uint32_t used = 0;
         bool stalled = false;
@@ -759,7 +819,7 @@ DEV uint32_t lookback(GLOBAL uint32_t* lb, const GLOBAL uint32_t* grp, uint32_t 
         entries += used;
         if (!done && stalled) stall();
     }
-    E::store(lb, (uint64_t)tile * RADIX + d, FS_LB_INC, excl + valid);
+    E::store(lb, (uint64_t)tile * radix + d, FS_LB_INC, excl + valid);
     return excl;
 }
 
@@ -3165,13 +3225,16 @@ extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_tile_keys[FS_VA
 extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_local_geometry[9] = {
     FS_L32_BLOCK * FS_L32_ITEMS, FS_L32_BLOCK, FS_L64_BLOCK * FS_L64_ITEMS, FS_L64_BLOCK, 32u - (FS_LOCAL_UBITS + 8u),
     FS_LW_BLOCK * FS_L32_ITEMS, FS_LW_BLOCK, FS_LW_BLOCK * FS_L64_ITEMS, FS_LW_BLOCK};
-// Bucket path: threads per block, keys per tile of the partition (32-bit keys,
-// 64-bit), keys a block sorts in LDS (32-bit, with values, 64-bit, with
-// values), most samples, most buckets, threads per block of the partition and of the sample.
-extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_bucket_geometry[11] = {
-    FS_BK_BLOCK, FS_BP_BLOCK * FS_BP32_ITEMS, FS_BP_BLOCK * FS_BP64_ITEMS, FS_BK_BLOCK * FS_BK32_ITEMS,
-    FS_BK_BLOCK * FS_BK32V_ITEMS, FS_BK_BLOCK * FS_BK64_ITEMS, FS_BK_BLOCK * FS_BK64V_ITEMS,
-    FS_BS_BLOCK * FS_BS_ITEMS, FS_BK_NB, FS_BP_BLOCK, FS_BS_BLOCK};
+// Bucket path: threads per block of the bucket kernels, the partition, the
+// sample and a child; most samples of the input and of a bucket; most buckets;
+// then keys of a bucket's block and of the partition's tile, each for 32-bit
+// keys, with values, 64-bit, with values; then keys of a child's block and of
+// the tiles of two levels, for 64-bit keys and with values.
+extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_bucket_geometry[FS_BG_WORDS] = {
+    FS_BK_BLOCK, FS_BP_BLOCK, FS_BS_BLOCK, FS_BC_BLOCK, FS_BS_BLOCK * FS_BS_ITEMS, FS_BS_BLOCK * FS_BS2_ITEMS, FS_BK_NB,
+    FS_BK_BLOCK * FS_BK32_ITEMS, FS_BK_BLOCK * FS_BK32V_ITEMS, FS_BK_BLOCK * FS_BK64_ITEMS, FS_BK_BLOCK * FS_BK64V_ITEMS,
+    FS_BP_BLOCK * FS_BP32_ITEMS, FS_BP_BLOCK * FS_BP32_ITEMS, FS_BP_BLOCK * FS_BP64_ITEMS, FS_BP_BLOCK * FS_BP64_ITEMS,
+    FS_BC_BLOCK * FS_BC64_ITEMS, FS_BC_BLOCK * FS_BC64V_ITEMS, FS_BP_BLOCK * FS_BP2_64_ITEMS, FS_BP_BLOCK * FS_BP2_64V_ITEMS};
 // Threads per block of the same variants.
 extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_block_threads[FS_VARIANTS] = {
     FS_K32_BLOCK, FS_K32V_BLOCK, FS_K64_BLOCK, FS_K64V_BLOCK, FS_K32S_BLOCK, FS_KS_BLOCK, FS_KS_BLOCK, FS_KS_BLOCK};

@@ -38,7 +38,7 @@ NO_ALLOC_MAX_KEYS = 1 << 20          # FS_NO_ALLOC_MAX_KEYS
 TEST_WIDE_LOOKBACK, TEST_UPSWEEP_BLOCKS_PER_CU, TEST_INJECT_FAULT, TEST_FUSED, TEST_TOP16, TEST_SEG_BITS = \
     0, 1, 2, 3, 4, 5
 TEST_LOCAL_WIDE, TEST_BUCKETS = 6, 7
-BUCKETS_BY_SIZE, BUCKETS_NEVER, BUCKETS_ONE_BLOCK, BUCKETS_ALWAYS = 0, 1, 2, 3   # TEST_BUCKETS values
+BUCKETS_BY_SIZE, BUCKETS_NEVER, BUCKETS_ONE_BLOCK, BUCKETS_ALWAYS, BUCKETS_TWO_LEVELS = 0, 1, 2, 3, 4   # TEST_BUCKETS values
 FUSED_BY_SIZE, FUSED_NEVER, FUSED_ALWAYS = 0, 1, 2       # TEST_FUSED values
 TOP16_BY_SIZE, TOP16_NEVER, TOP16_ALWAYS, TOP16_SAMPLED = 0, 1, 2, 3   # TEST_TOP16 values
 FUSED_MIN_KEYS = 1 << 25                                 # FS_FUSED_MIN_KEYS
@@ -47,7 +47,7 @@ TOP16_MIN_KEYS64 = 1 << 21                               # FS_TOP16_MIN_KEYS64
 # fs_sorter_first_pass: how the last sort began
 FIRST_HISTOGRAM, FIRST_FUSED, FIRST_FUSED_OVERFLOW, FIRST_TOP16, FIRST_TOP16_RESCATTER = 0, 1, 2, 3, 4
 FAULT_NONE, FAULT_BAD_DIGITS, FAULT_BAD_BUFFER, FAULT_EXTRA_BLOCK, FAULT_STALL_TILE, FAULT_SMALL_S1 = 0, 1, 2, 3, 4, 5
-FAULT_SMALL_REGIONS = 6
+FAULT_SMALL_REGIONS, FAULT_SMALL_REGIONS2 = 6, 7
 
 FS_OK = 0
 FS_ERR_DEVICE_NOT_FOUND = 1

@@ -255,7 +255,9 @@ typedef enum fs_test_option {
                                            1 = wide blocks at every size */
     FS_TEST_BUCKETS = 7                 /* bucket path: 0 = by size (the default), 1 = never, 2 = one
                                            block for every sort that fits it, 3 = buckets for every
-                                           sort of at least 64 keys; + (b << 8): 2^b buckets */
+                                           sort of at least 64 keys, 4 = two levels of buckets (64-bit
+                                           keys, or the digit passes where few digits vary) for them;
+                                           + (b << 8): 2^b buckets */
 } fs_test_option;
 fs_status fs_sorter_set_test_option(fs_sorter *s, fs_test_option opt, uint64_t value);
 
@@ -287,11 +289,13 @@ fs_status fs_sorter_set_test_option(fs_sorter *s, fs_test_option opt, uint64_t v
 #define FS_TOP16_MIN_KEYS64 2097152u
 
 /* How the last completed sort began: 0 = the histogram read (argsort, pairs,
- * and keys-only sorts outside the fused range), 1 = the fused first pass of a
- * keys-only sort, its regions read by the next pass,
+ * and keys-only sorts outside the fused range, also where buckets did them), 1 = the fused first pass of a
+ * keys-only sort, its regions read by the next pass (or, f64, the partition
+ * into buckets),
  * 2 = the fused first pass after a region overflowed (the keys re-scattered
  * into exact regions by its second launch), or every digit constant (no
- * pass after it),
+ * pass after it), or f64 keys of so few varying digits that the digit passes
+ * sort them from the caller's buffer,
  * 3 = the top-16 path (fused pass on the second-highest byte, its regions
  * read by the pass on the highest byte, then the local sort),
  * 4 = the top-16 path after a region of its fused pass overflowed (the keys

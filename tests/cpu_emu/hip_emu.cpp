@@ -389,7 +389,7 @@ void fs_gather_elems(uint64_t, uint64_t, uint64_t, uint64_t, uint64_t, uint32_t,
 extern uint32_t fs_kernel_tile_keys[FS_VARIANTS];
 extern uint32_t fs_kernel_block_threads[FS_VARIANTS];
 extern uint32_t fs_kernel_local_geometry[9];
-extern uint32_t fs_kernel_bucket_geometry[11];
+extern uint32_t fs_kernel_bucket_geometry[FS_BG_WORDS];
 void fs_split_k32(FsArgs);
 void fs_split_k64(FsArgs);
 void fs_part_k32(FsArgs);
@@ -400,6 +400,15 @@ void fs_bucket_k32(FsArgs);
 void fs_bucket_k32_v(FsArgs);
 void fs_bucket_k64(FsArgs);
 void fs_bucket_k64_v(FsArgs);
+void fs_part1_k64_v(FsArgs);
+void fs_part1_k64(FsArgs);
+void fs_split2_k64(FsArgs);
+void fs_part2_k64(FsArgs);
+void fs_part2_k64_v(FsArgs);
+void fs_child_k64(FsArgs);
+void fs_child_k64_v(FsArgs);
+void fs_rest_k64(FsArgs);
+void fs_rest_k64_v(FsArgs);
 }
 
 struct emu_function {
@@ -420,6 +429,15 @@ static emu_function g_funcs[] = {
     {"fs_bucket_k32_v", [](void** p) { fs_bucket_k32_v(A0); }},
     {"fs_bucket_k64", [](void** p) { fs_bucket_k64(A0); }},
     {"fs_bucket_k64_v", [](void** p) { fs_bucket_k64_v(A0); }},
+    {"fs_split2_k64", [](void** p) { fs_split2_k64(A0); }},
+    {"fs_part2_k64", [](void** p) { fs_part2_k64(A0); }},
+    {"fs_part2_k64_v", [](void** p) { fs_part2_k64_v(A0); }},
+    {"fs_child_k64", [](void** p) { fs_child_k64(A0); }},
+    {"fs_child_k64_v", [](void** p) { fs_child_k64_v(A0); }},
+    {"fs_rest_k64", [](void** p) { fs_rest_k64(A0); }},
+    {"fs_rest_k64_v", [](void** p) { fs_rest_k64_v(A0); }},
+    {"fs_part1_k64", [](void** p) { fs_part1_k64(A0); }},
+    {"fs_part1_k64_v", [](void** p) { fs_part1_k64_v(A0); }},
     {"fs_upsweep_k32", [](void** p) { fs_upsweep_k32(A0); }},
     {"fs_upsweep_k64", [](void** p) { fs_upsweep_k64(A0); }},
     {"fs_onesweep_k32", [](void** p) { fs_onesweep_k32(A0, D1); }},

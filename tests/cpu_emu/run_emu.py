@@ -43,6 +43,9 @@ def keys_for(kind, n, dist, seed, tile=None):
         b = np.full(n, 7, dtype=BITS[kind])
     elif dist == "low12":
         b = g.integers(0, 1 << 12, size=n, dtype=BITS[kind])
+    elif dist == "lone":        # 12 low bits vary, but for one key: a sample shows two digits varying of all
+        b = g.integers(0, 1 << 12, size=n, dtype=BITS[kind])
+        b[n // 2 + 1] = ~BITS[kind](0)
     elif dist == "byte0":
         # one varying digit (the lowest): a single-pass schedule whose pass
         # writes scratch, copied back afterwards
@@ -327,20 +330,24 @@ def check_first_pass(sorter, op, kind, n, dist, seed):
 
 def check(sorter, op, kind, n, dist, seed):
     # one_<op>: one block sorts everything; bk_<op>, bk<b>_<op>: the bucket
-    # path (2^b buckets); bkover_<op>: with a region that overflows (fault build)
-    bucket = re.fullmatch(r"(one|bk|bkover)(\d*)_(sort|argsort|pairs|offset)", op)
+    # path (2^b buckets), two_<op>: two levels of them; bkover_<op>, twoover_<op>,
+    # twosecond_<op>: with a region (of the second level) that overflows (fault build)
+    bucket = re.fullmatch(r"(one|bk|bkover|two|twoover|twosecond)(\d*)_(sort|argsort|pairs|offset)", op)
     if bucket:
         one, b, rest = bucket.groups()
         sorter.set_test_option(forge_sort.TEST_BUCKETS,
                                forge_sort.BUCKETS_ONE_BLOCK if one == "one"
-                               else forge_sort.BUCKETS_ALWAYS + (int(b or 0) << 8))
-        if one == "bkover":
-            sorter.set_test_option(forge_sort.TEST_INJECT_FAULT, forge_sort.FAULT_SMALL_REGIONS)
+                               else (forge_sort.BUCKETS_TWO_LEVELS if one.startswith("two")
+                                     else forge_sort.BUCKETS_ALWAYS) + (int(b or 0) << 8))
+        fault = {"bkover": forge_sort.FAULT_SMALL_REGIONS, "twoover": forge_sort.FAULT_SMALL_REGIONS,
+                 "twosecond": forge_sort.FAULT_SMALL_REGIONS2}.get(one)
+        if fault:
+            sorter.set_test_option(forge_sort.TEST_INJECT_FAULT, fault)
         try:
             return check(sorter, rest, kind, n, dist, seed)
         finally:
             sorter.set_test_option(forge_sort.TEST_BUCKETS, forge_sort.BUCKETS_BY_SIZE)
-            if one == "bkover":
+            if fault:
                 sorter.set_test_option(forge_sort.TEST_INJECT_FAULT, forge_sort.FAULT_NONE)
     if op in FIRST_PASS or op.startswith(("top16s", "top16w")):
         return check_first_pass(sorter, op, kind, n, dist, seed)

@@ -22,29 +22,43 @@ CASES = [
     # few buckets of many keys: blocks that sort theirs through device memory
     "bk2_sort:u32:5000:uniform:20", "bk2_pairs:f64:4000:few:21", "bk2_argsort:u32:4000:uniform:22",
 ]
+# two levels: uniform, buckets and children of one value, larger than a block,
+# the least size; the digit passes for one, two and no varying digit; a sample
+# that shows two digits of eight
+TWO = [
+    "two_sort:u64:9000:uniform:1", "two_sort:i64:6000:uniform:2", "two_pairs:u64:6000:uniform:3",
+    "two_argsort:f64:9000:uniform:4", "two_sort:f64:9000:few:5", "two_pairs:f64:9000:few:6", "two_sort:u64:64:uniform:10",
+    "two2_sort:i64:9000:uniform:12", "two2_argsort:u64:12000:uniform:13",
+    "two_sort:u64:5000:same:8", "two_argsort:i64:5000:same:9", "two_argsort:u64:9000:low12:14", "two_pairs:u64:5000:byte0:3",
+    "two_sort:u64:5000:byte1:3", "two_pairs:u64:9000:lone:1", "two_sort:i64:9000:lone:1",
+]
 
 
 def test_emulated_buckets(emulator):  # noqa: F811
-    run_cases("small", CASES, parallel=4)
-    run_cases("prod", ["one_sort:u32:8192:uniform:1", "one_pairs:f64:6144:few:2", "bk_sort:u32:40000:uniform:3",
+    run_cases("small", CASES + TWO, parallel=4)
+    run_cases("prod", ["two4_sort:f64:60000:uniform:6", "two4_pairs:u64:50000:lone:7", "one_sort:u32:8192:uniform:1", "one_pairs:f64:6144:few:2", "bk_sort:u32:40000:uniform:3",
                        "bk_argsort:f32:30000:few:4", "bk_pairs:u64:20000:zipf:5"], parallel=3, env={"EMU_CUS": "8"})
 
 
 @pytest.mark.parametrize("order", ["wave", "wave_rev"])
 def test_emulated_buckets_wave_serial(emulator, order):  # noqa: F811
-    run_cases("small", CASES, timeout=900, env={"EMU_SCHED": order}, parallel=4)
+    run_cases("small", CASES + TWO, timeout=900, env={"EMU_SCHED": order}, parallel=4)
 
 
 def test_emulated_buckets_overflow(emulator):  # noqa: F811
     """A region with room for one row only: its keys do not fit, and one block
     sorts the caller's keys instead (the fault-injection build)."""
     run_cases("faults", ["bkover_sort:u32:3000:uniform:1", "bkover_pairs:u64:2000:few:2", "bkover_argsort:f32:3000:uniform:3",
-                         "bkover_sort:i64:2000:uniform:4"])
+                         "bkover_sort:i64:2000:uniform:4",
+                         # two levels: of the first (one block sorts all) or of every bucket's second child
+                         "twoover_sort:u64:9000:uniform:1", "twoover_pairs:u64:6000:few:2",
+                         "twosecond_sort:u64:9000:uniform:3", "twosecond_pairs:f64:9000:uniform:4"],
+              env={"EMU_WORKERS": "1", "EMU_XCDS": "1"})   # (tiles in order: this build soon gives up a look-back wait)
 
 
 def test_emulated_buckets_sanitizers(emulator):  # noqa: F811
     libasan = subprocess.run(["g++", "-print-file-name=libasan.so"], capture_output=True, text=True).stdout.strip()
     if not os.path.isabs(libasan):
         pytest.skip("libasan not found")
-    run_cases("san", CASES[::2], timeout=600, env={"LD_PRELOAD": libasan, "EMU_NO_SEGV_HANDLER": "1", "EMU_CUS": "4",
+    run_cases("san", CASES[::2] + TWO[::2], timeout=600, env={"LD_PRELOAD": libasan, "EMU_NO_SEGV_HANDLER": "1", "EMU_CUS": "4",
                                                   "ASAN_OPTIONS": "detect_leaks=0:detect_stack_use_after_return=0"}, parallel=3)

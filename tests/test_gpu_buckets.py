@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle
-from test_gpu_parity import BITS, KINDS, NP, bits_equal, first_diff
+from test_gpu_parity import BITS, KINDS, NP, bits_equal, first_diff, hip_stream  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -42,6 +42,13 @@ def keys_of(kind, n, data, seed):
     elif data == "clusters":                      # two narrow ranges far apart, and a lone key between
         b = g.integers(0, 1 << 12, size=n, dtype=u) + np.where(g.random(n) < 0.5, u(0), ~u(0) - u(1 << 13)).astype(u)
         b[n // 2] = u(1) << u(20)
+    elif data == "narrow":                        # 20 varying bits
+        b = g.integers(0, 1 << 20, size=n, dtype=u)
+    elif data == "lone":                          # 12, but for one key that a sample misses
+        b = g.integers(0, 1 << 12, size=n, dtype=u)
+        b[n // 3 + 1] = ~u(0)
+    elif data == "runs":                          # random keys, each five times in a row
+        b = np.repeat(g.integers(0, 1 << (64 if wide else 32), size=n // 5 + 1, dtype=u, endpoint=False), 5)[:n]
     elif data == "sorted":
         b = np.sort(g.integers(0, 1 << (64 if wide else 32), size=n, dtype=u, endpoint=False))
     else:
@@ -90,11 +97,82 @@ def test_bucket_path(sorter, op, kind, shape, n):
         sorter.set_test_option(TEST_BUCKETS, BUCKETS_BY_SIZE)
 
 
+@pytest.mark.parametrize("kind", ["u64", "i64", "f64"])
+@pytest.mark.parametrize("op", ["sort", "argsort", "pairs"])
+@pytest.mark.parametrize("lnb,n", [(0, 64), (0, 5121), (1, 30_000), (0, 300_001), (2, 150_000)])
+def test_two_levels(sorter, op, kind, lnb, n):
+    """Two levels of buckets, or the digit passes where few digits vary: least
+    size, tile edges, few buckets (children larger than a block), every kind of
+    data that takes another branch."""
+    from forge_sort import BUCKETS_BY_SIZE, BUCKETS_TWO_LEVELS, TEST_BUCKETS
+    sorter.set_test_option(TEST_BUCKETS, BUCKETS_TWO_LEVELS + (lnb << 8))
+    try:
+        for i, data in enumerate(("normal", "quantised", "specials", "clusters", "sorted", "same", "narrow", "lone", "runs")):
+            keys = keys_of(kind, n, data, seed=7200 + i)
+            check(sorter, op, kind, keys)
+            b = keys.view(np.uint64)
+            top = np.uint64(1 << 63)
+            b = np.where(b & top, ~b, b | top) if kind == "f64" else b
+            varying = int(np.bitwise_or.reduce(b ^ b[0]))
+            assert sorter.last_pass_info()[1] == sum(1 << j for j in range(8) if varying >> (8 * j) & 0xFF)
+    finally:
+        sorter.set_test_option(TEST_BUCKETS, BUCKETS_BY_SIZE)
+
+
+@pytest.mark.parametrize("kind,op,n", [("f64", "sort", 1_500_001), ("f64", "argsort", 1_000_001), ("i64", "pairs", 12_000_000)])
+@pytest.mark.parametrize("data", ["normal", "quantised", "narrow", "lone"])
+def test_two_levels_by_size(sorter, kind, op, n, data):
+    """The least sizes that take two levels by size."""
+    check(sorter, op, kind, keys_of(kind, n, data, seed=7300))
+
+
 @pytest.mark.parametrize("kind,op", [("u32", "sort"), ("f32", "argsort"), ("i64", "sort"), ("f64", "pairs")])
-@pytest.mark.parametrize("data", ["normal", "quantised", "specials", "clusters"])
+@pytest.mark.parametrize("data", ["normal", "quantised", "specials", "clusters", "runs"])
 def test_bucket_path_largest(sorter, kind, op, data):
     """The largest sizes that take the path by size (512 buckets, the most
-    samples), and one key more (the digit passes)."""
-    n = 1_100_000 if kind == "f64" else 1_500_000
+    samples), and one key more (the digit passes; f64: two levels)."""
+    n = {"u32": 1_100_000, "f32": 600_000, "i64": 1_500_000, "f64": 1_000_000}[kind]
     for m in (n, n + 1):
         check(sorter, op, kind, keys_of(kind, m, data, seed=7100 + m % 2))
+
+
+@pytest.mark.parametrize("kind,op,n,reserved", [("u32", "sort", 790_000, 1_000_000), ("u64", "pairs", 380_001, 400_000),
+                                                ("f64", "pairs", 1_200_001, 1_300_000), ("f64", "sort", 1_600_001, 1_700_000)])
+def test_bucket_path_captured(hip_stream, kind, op, n, reserved):  # noqa: F811
+    """Scratch reserved for more keys holds the sort of fewer (a smaller sort's
+    regions may be larger); captured into a HIP graph and replayed on data that
+    takes other branches (two levels: the buckets, the digit passes, and back),
+    eager sorts between the replays."""
+    import ctypes
+    from forge_sort import OP_PAIRS, OP_SORT, GpuSorter
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    st = ctypes.c_void_p(hip_stream)
+    s = GpuSorter.with_context(0, hip_stream)
+    code = OP_PAIRS if op == "pairs" else OP_SORT
+    graph, exe = ctypes.c_void_p(), ctypes.c_void_p()
+    vals = np.arange(n, dtype=np.uint32)
+    try:
+        kb, vb = s.alloc_sort_buffer(kind, n), s.alloc_sort_buffer("u32", n)
+        s.reserve(code, kind, reserved)
+        assert hip.hipStreamBeginCapture(st, 0) == 0
+        s.encode(code, kind, kb.device_ptr(), vb.device_ptr(), n, stream=hip_stream)
+        assert hip.hipStreamEndCapture(st, ctypes.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
+        for r, data in enumerate(("uniform", "narrow", "lone", "quantised", "same", "normal")):
+            keys = keys_of(kind, n, data, seed=7400 + r)
+            kb.copy_from_slice(keys)
+            vb.copy_from_slice(vals)
+            assert hip.hipGraphLaunch(exe, st) == 0
+            assert hip.hipStreamSynchronize(st) == 0
+            ek, ev = oracle.sort_pairs(kind, keys, vals)
+            assert bits_equal(kb.as_slice(), ek, kind), f"replay {r} ({data})"
+            assert op == "sort" or np.array_equal(vb.as_slice(), ev), f"replay {r} ({data})"
+            check(s, "sort", kind, keys_of(kind, n // 3, "normal", seed=7500 + r))
+        kb.free()
+        vb.free()
+    finally:
+        if exe.value:
+            hip.hipGraphExecDestroy(exe)
+        if graph.value:
+            hip.hipGraphDestroy(graph)
+        s.close()

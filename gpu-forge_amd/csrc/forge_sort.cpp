@@ -390,7 +390,9 @@ static BucketLimit bucket_limit(fs_op op, fs_key_type t) {
     if (key64(t))
         return v ? BucketLimit{FS_BK_ONE_64V, FS_BK_MAX_64V, f64 ? 0u : FS_BK2_MIN_64V, FS_BK2_MAX_64V}
                  : BucketLimit{FS_BK_ONE_64, FS_BK_MAX_64, 0, f64 ? FS_BK2_MAX_64 : 0u};
-    return v ? BucketLimit{FS_BK_ONE_32V, FS_BK_MAX_32V, 0, 0} : BucketLimit{FS_BK_ONE_32, FS_BK_MAX_32, 0, 0};
+    const bool f32 = t == FS_KEY_F32;
+    return v ? BucketLimit{FS_BK_ONE_32V, f32 ? FS_BK_MAX_F32 : FS_BK_MAX_32V, 0, 0}
+             : BucketLimit{FS_BK_ONE_32, f32 ? FS_BK_MAX_F32 : FS_BK_MAX_32, 0, 0};
 }
 static BucketPath bucket_path(const fs_sorter* s, fs_op op, fs_key_type t, uint64_t n, bool no_alloc) {
     if (n < 2 || n >= (1ull << 31)) return BK_NONE;

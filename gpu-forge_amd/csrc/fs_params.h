@@ -410,7 +410,9 @@
 // Largest sorts that one block does alone, that buckets do, and that two
 // levels of buckets do (64-bit keys), by key width and values (V).  Where the
 // digit passes are as fast (us, buckets against passes, keys in place):
-// 32-bit keys of few values, f32, 1.1M: 66 / 67 (uniform 48 / 67); with values
+// f32 keys with zeros, infinities, NaN and subnormals, which crowd the sample
+// and one bucket, 0.1M: 45 / 52, 0.22M: 61 / 53 (without them 1.1M: 48 / 67);
+// 32-bit integers, uniform, 1.1M: 46 / 66, of few values 41 / 45; with values
 // u32 argsort, 20 varying bits, 0.7M: 52 / 51 (0.5M: 42 / 49); 64-bit keys with
 // values of 20 bits, 1M: 64 / 66 (uniform 68 / 136).  Two levels: f64 from
 // there on (3M: sort 170 / 190, argsort 163 / 184; 128M: 2,496 / 4,567), but
@@ -426,6 +428,7 @@
 #define FS_BK_ONE_64V 6144u
 #define FS_BK_MAX_32 1100000u
 #define FS_BK_MAX_32V 600000u
+#define FS_BK_MAX_F32 190000u
 #define FS_BK_MAX_64 1500000u
 #define FS_BK_MAX_64V 1000000u
 #define FS_BK2_MAX_64 140000000u

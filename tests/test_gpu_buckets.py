@@ -126,12 +126,13 @@ def test_two_levels_by_size(sorter, kind, op, n, data):
     check(sorter, op, kind, keys_of(kind, n, data, seed=7300))
 
 
-@pytest.mark.parametrize("kind,op", [("u32", "sort"), ("f32", "argsort"), ("i64", "sort"), ("f64", "pairs")])
+@pytest.mark.parametrize("kind,op", [("u32", "sort"), ("i32", "pairs"), ("f32", "argsort"), ("i64", "sort"),
+                                     ("f64", "pairs")])
 @pytest.mark.parametrize("data", ["normal", "quantised", "specials", "clusters", "runs"])
 def test_bucket_path_largest(sorter, kind, op, data):
     """The largest sizes that take the path by size (512 buckets, the most
     samples), and one key more (the digit passes; f64: two levels)."""
-    n = {"u32": 1_100_000, "f32": 600_000, "i64": 1_500_000, "f64": 1_000_000}[kind]
+    n = {"u32": 1_100_000, "i32": 600_000, "f32": 190_000, "i64": 1_500_000, "f64": 1_000_000}[kind]
     for m in (n, n + 1):
         check(sorter, op, kind, keys_of(kind, m, data, seed=7100 + m % 2))
 

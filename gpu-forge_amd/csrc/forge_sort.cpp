@@ -49,13 +49,14 @@ const char* const kKernelNames[] = {
     "fs_split_k32", "fs_split_k64", "fs_part_k32", "fs_part_k32_v", "fs_part_k64", "fs_part_k64_v", "fs_bucket_k32",
     "fs_bucket_k32_v", "fs_bucket_k64", "fs_bucket_k64_v", "fs_split2_k64", "fs_part1_k64", "fs_part1_k64_v",
     "fs_part2_k64", "fs_part2_k64_v", "fs_child_k64", "fs_child_k64_v", "fs_rest_k64", "fs_rest_k64_v",
+    "fs_upsweep_choose_k64",
 };
 enum {
     K_UP32, K_UP64, K_OS32, K_OS32V, K_OS64, K_OS64V, K_IOTA, K_ANY32, K_ANY64, K_SCRATCH_ADDR, K_FIRST32, K_FIRST64,
     K_SAMPLE32, K_SAMPLE64, K_LOCAL32, K_RESCATTER32, K_RESCATTER64, K_LOCAL64, K_DEFER64, K_LOOP64, K_DEFER32,
     K_LOCAL32W, K_DEFER32W, K_LOCAL64W, K_DEFER64W, K_OS32S, K_ANY32S, K_OS32VS, K_OS64S, K_ANY64S, K_OS64VS,
     K_SPLIT32, K_SPLIT64, K_PART32, K_PART32V, K_PART64, K_PART64V, K_BUCKET32, K_BUCKET32V, K_BUCKET64, K_BUCKET64V,
-    K_SPLIT2, K_PART1, K_PART1V, K_PART2, K_PART2V, K_CHILD, K_CHILDV, K_REST, K_RESTV,
+    K_SPLIT2, K_PART1, K_PART1V, K_PART2, K_PART2V, K_CHILD, K_CHILDV, K_REST, K_RESTV, K_UP64C,
     K_COUNT
 };
 // the stable digit-pass kernel and the keys-only first-pass kernel of each variant (FS_VAR_*)
@@ -714,9 +715,8 @@ static fs_status enqueue_buckets(fs_sorter* s, fs_op op, fs_key_type t, void* ke
             FsArgs d;
             const uint64_t up_blocks = digit_args(s, op, t, keys, vals, n, sc, s->tile[var], false, d);
             d.bk2_tab = a.bk2_tab;
-            d.bk2_choose = 1u;
             void* dargs[] = {&d};
-            if ((r = launch(s, K_UP64, (unsigned)up_blocks, FS_HIST_BLOCK, dargs, st)) != FS_OK) return r;
+            if ((r = launch(s, K_UP64C, (unsigned)up_blocks, FS_HIST_BLOCK, dargs, st)) != FS_OK) return r;
             for (uint32_t sl = 0; sl < FS_BK2_FEW_DIGITS; ++sl) {
                 void* pargs[] = {&d, &sl};
                 // (a keys-only sort's first pass needs no stability)

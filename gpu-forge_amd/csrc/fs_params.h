@@ -615,7 +615,6 @@ typedef struct FsArgs {
     uint32_t rest_cap;          // entries the rest list holds
     uint64_t bk2_tab;           // u32[FS_BK2_TAB_WORDS] second-level table (0: one level)
     uint64_t rest;              // u32[rest_cap][2] rest list
-    uint32_t bk2_choose;        // 1: a sort that launches two levels of buckets and the digit passes
 } FsArgs;
 
 // Look-back statistics (accumulated only when FsArgs.stats is set).

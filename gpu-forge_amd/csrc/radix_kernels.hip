@@ -220,7 +220,9 @@ DEV uint32_t wave_inclusive_scan(uint32_t v) {
 // fs_upsweep: all-digit histograms in one read
 // ---------------------------------------------------------------------------
 
+template <bool CHOOSE>
 DEV void plan_body(const FsArgs& a);
+template <bool CHOOSE>
 DEV void write_schedule(const FsArgs& a, uint32_t cmask, uint32_t D);
 
 // Lanes of one LDS atomic that hit the same counter are serialised; on skewed
@@ -289,7 +291,7 @@ DEV void leave_to_buckets(const FsArgs& a) {
     st_agent(gptr<uint32_t>(a.bk2_tab) + FS_BK2_MODE, 0u);
 }
 
-template <bool K64>
+template <bool K64, bool CHOOSE>
 DEV void upsweep_body(const FsArgs& a) {
     typedef typename KeyT<K64>::type K;
     constexpr int D = K64 ? 8 : 4;
@@ -314,7 +316,7 @@ DEV void upsweep_body(const FsArgs& a) {
     // (the loads are in flight while the counters are cleared).
     K ref = 0, probe = 0;
     __shared__ uint32_t s_vary;
-    if (K64 && a.bk2_choose) {
+    if constexpr (CHOOSE) {
         constexpr uint32_t LB = __builtin_ctz(B);
         static_assert(B == 1u << LB, "a sample per thread");
         const GLOBAL K* keys = gptr<const K>(a.keys);
@@ -334,7 +336,7 @@ DEV void upsweep_body(const FsArgs& a) {
             st_agent(&lb[i], 0u);
     }
     __syncthreads();
-    if (K64 && a.bk2_choose) {
+    if constexpr (CHOOSE) {
         const K v = xf_fwd<K64>(probe, a.xform) ^ xf_fwd<K64>(ref, a.xform);
         uint32_t mine = 0;                               // digits that vary within the wave's samples
 #pragma unroll
@@ -452,17 +454,23 @@ DEV void upsweep_body(const FsArgs& a) {
     __syncthreads();
     if (!s_last) return;
     __threadfence();
-    plan_body(a);
+    plan_body<CHOOSE>(a);
     if (tid == 0) st_agent(ticket, 0u);
 }
 
 // two blocks per CU: at most 64 VGPRs at 1024 threads
 #define FS_UP_OCC __attribute__((amdgpu_waves_per_eu(FS_HIST_BLOCK / 64 / 4 * 2)))
 extern "C" __global__ void __launch_bounds__(FS_HIST_BLOCK) FS_UP_OCC fs_upsweep_k32(FsArgs a) {
-    upsweep_body<false>(a);
+    upsweep_body<false, false>(a);
 }
 extern "C" __global__ void __launch_bounds__(FS_HIST_BLOCK) FS_UP_OCC fs_upsweep_k64(FsArgs a) {
-    upsweep_body<true>(a);
+    upsweep_body<true, false>(a);
+}
+// ... of sorts that may go to two levels of buckets: a kernel of its own, since
+// the choice within the kernels above, unused, cost the other sorts 0.3 to 2 us
+// (u64 keys, 2.0M: 167.6 -> 165.8; u32, 2.5M: 94.0 -> 93.7)
+extern "C" __global__ void __launch_bounds__(FS_HIST_BLOCK) FS_UP_OCC fs_upsweep_choose_k64(FsArgs a) {
+    upsweep_body<true, true>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -471,6 +479,7 @@ extern "C" __global__ void __launch_bounds__(FS_HIST_BLOCK) FS_UP_OCC fs_upsweep
 // thread of the block reaches the barriers)
 // ---------------------------------------------------------------------------
 
+template <bool CHOOSE>
 DEV void plan_body(const FsArgs& a) {
     __shared__ uint32_t wsum[FS_MAX_DIGITS][FS_RADIX / 64];
     __shared__ uint32_t cmask;                 // bit j: digit j is constant
@@ -525,13 +534,15 @@ DEV void plan_body(const FsArgs& a) {
         st_agent(&hist[j * FS_RADIX + d], 0u);        // ready for the next sort
     }
 
-    if (d == 0) write_schedule(a, cmask, D);
+    if (d == 0) write_schedule<CHOOSE>(a, cmask, D);
 }
 
 // The standard schedule, written by one thread: which digit passes run (the
 // digits whose bit in cmask is clear), their order of execution, flags and
 // buffers.  Every pass reads the previous pass's output, the first the
-// caller's keys.
+// caller's keys.  CHOOSE: the sort may go to the buckets instead, and has
+// FS_BK2_FEW_DIGITS launch slots.
+template <bool CHOOSE>
 DEV void write_schedule(const FsArgs& a, uint32_t cmask, uint32_t D) {
     {
         GLOBAL uint32_t* plan = gptr<uint32_t>(a.plan);
@@ -540,7 +551,7 @@ DEV void write_schedule(const FsArgs& a, uint32_t cmask, uint32_t D) {
         uint32_t p = 0, mask = 0;
         for (uint32_t j = 0; j < D; ++j)
             if (active[j]) { ++p; mask |= 1u << j; }
-        if (a.bk2_choose) {
+        if (CHOOSE) {
             if (p > FS_BK2_FEW_DIGITS) {                 // more digits vary than the sample showed
                 leave_to_buckets(a);
                 return;
@@ -549,7 +560,7 @@ DEV void write_schedule(const FsArgs& a, uint32_t cmask, uint32_t D) {
         }
         // Fewer launch slots than digits: the passes that run take slots in
         // order, after a copy if there is one.
-        const bool compact = a.bk2_choose != 0u;
+        constexpr bool compact = CHOOSE;
 
         // Destination of executed pass e for keys (dk) and values (dv).
         uint32_t dk[FS_MAX_DIGITS], dv[FS_MAX_DIGITS];
@@ -2145,7 +2156,7 @@ DEV void fused_plan(const FsArgs& a, uint32_t* lds) {
     if (tid == 0) {
         if (fast && top16) write_top16_schedule(a, f_cmask, exact);
         else if (fast) write_fused_schedule(a, f_cmask, D, exact);
-        else write_schedule(a, f_cmask, D);
+        else write_schedule<false>(a, f_cmask, D);
     }
 }
 

@@ -356,6 +356,7 @@ void launch(const char* name, void (*entry)(void**), uint32_t grid, uint32_t blo
 extern "C" {
 void fs_upsweep_k32(FsArgs);
 void fs_upsweep_k64(FsArgs);
+void fs_upsweep_choose_k64(FsArgs);
 void fs_onesweep_k32(FsArgs, uint32_t);
 void fs_onesweep_k32_v(FsArgs, uint32_t);
 void fs_onesweep_k64(FsArgs, uint32_t);
@@ -440,6 +441,7 @@ static emu_function g_funcs[] = {
     {"fs_part1_k64_v", [](void** p) { fs_part1_k64_v(A0); }},
     {"fs_upsweep_k32", [](void** p) { fs_upsweep_k32(A0); }},
     {"fs_upsweep_k64", [](void** p) { fs_upsweep_k64(A0); }},
+    {"fs_upsweep_choose_k64", [](void** p) { fs_upsweep_choose_k64(A0); }},
     {"fs_onesweep_k32", [](void** p) { fs_onesweep_k32(A0, D1); }},
     {"fs_onesweep_k32_v", [](void** p) { fs_onesweep_k32_v(A0, D1); }},
     {"fs_onesweep_k64", [](void** p) { fs_onesweep_k64(A0, D1); }},

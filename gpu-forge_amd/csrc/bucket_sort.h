@@ -484,10 +484,11 @@ DEV bool count_groups(const typename KeyT<K64>::type (&k)[ITEMS], uint32_t len, 
     return fine;
 }
 
-// The schedule words fs_last_pass_info reads: a digit counts as sorted when
-// some key has a bit of it set that another has clear.
+// The schedule words fs_last_pass_info and fs_last_bucket_info read: a digit
+// counts as sorted when some key has a bit of it set that another has clear;
+// overs: regions (second level: buckets with such a region) that overflowed.
 template <bool K64>
-DEV void bucket_pass_info(const FsArgs& a, uint64_t varying) {
+DEV void bucket_pass_info(const FsArgs& a, uint64_t varying, uint32_t overs) {
     uint32_t mask = 0, p = 0;
     for (uint32_t j = 0; j < (K64 ? 8u : 4u); ++j)
         if ((varying >> (8u * j)) & 0xFFu) {
@@ -496,8 +497,8 @@ DEV void bucket_pass_info(const FsArgs& a, uint64_t varying) {
         }
     GLOBAL uint32_t* plan = gptr<uint32_t>(a.plan);
     st_agent(&plan[FS_PLAN_NPASSES], p);
-    st_agent(&plan[FS_PLAN_MASK], mask | FS_MASK_FUSED);
-    st_agent(&plan[FS_PLAN_RESCATTER], 0u);
+    st_agent(&plan[FS_PLAN_MASK], mask | FS_MASK_FUSED | FS_MASK_BUCKETS);
+    st_agent(&plan[FS_PLAN_RESCATTER], overs);
 }
 
 // ---------------------------------------------------------------------------
@@ -596,7 +597,7 @@ DEV void split_body(const FsArgs& a) {
         if (blockIdx.x) return;                          // (uniform)
         for (uint32_t i = tid; i < nb; i += BLOCK) st_agent(&cnt[i], 0u);
         for (uint32_t i = tid; i < 4u * FS_BK_BIT_SLOTS; i += BLOCK) st_agent(&tab1[FS_BK_BITS + i], 0u);
-        if (a.bk2_tab && tid < 2u) st_agent(&tab2[FS_BK2_OVER + tid], 0u);
+        if (a.bk2_tab && tid < FS_BK2_INFO && tid != FS_BK2_MODE) st_agent(&tab2[tid], 0u);
     }
 
     // sample i: the key at a hashed position within the i-th of m equal parts
@@ -1143,7 +1144,7 @@ DEV void block_range_sort(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool 
     if (whole) {
         K on = 0, off = 0;
         block_fold<K64, VALS, BLOCK, ITEMS, true>(k, len, per, L, on, off);
-        if (tid == 0) bucket_pass_info<K64>(a, (uint64_t)(on & off));
+        if (tid == 0) bucket_pass_info<K64>(a, (uint64_t)(on & off), 0u);
     }
     K base = 0;
     sort_rows<K64, VALS, BLOCK, ITEMS>(k, p, len, per, a.xform == FS_XF_FLOAT, L, base);
@@ -1206,7 +1207,7 @@ DEV void bucket_body(const FsArgs& a) {
         const GLOBAL K* lbs = reinterpret_cast<const GLOBAL K*>(tab + FS_BK_LB);
         const uint32_t ex = block_exclusive_scan<BLOCK>(c, L.wsum);
         if (tid < nb) {
-            if (c > cap) s_over = 1u;
+            if (c > cap) atomicAdd(&s_over, 1u);
             // buckets of one value that outgrow a block: copied by every block
             // in turn, a block's keys at a time
             if (c > CAP && (tid + 1u < nb ? lbs[tid + 1u] - lbs[tid] == (K)1 : lbs[tid] == ~(K)0))
@@ -1226,7 +1227,7 @@ DEV void bucket_body(const FsArgs& a) {
             uint32_t b[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
             for (uint32_t i = 0; i < 4u * FS_BK_BIT_SLOTS; ++i) b[i % 4u] |= tab[FS_BK_BITS + i];
-            bucket_pass_info<K64>(a, ((uint64_t)(b[1] & b[3]) << 32) | (b[0] & b[2]));
+            bucket_pass_info<K64>(a, ((uint64_t)(b[1] & b[3]) << 32) | (b[0] & b[2]), s_over);
         }
         if (s_over) {                                   // (uniform) a region overflowed: block 0 sorts the caller's keys
             __syncthreads();
@@ -1354,7 +1355,10 @@ DEV void child_body(const FsArgs& a) {
     ChildPlace c;
     if (!child_place<K64, BLOCK>(a, id, L.wsum, s_seg, c)) return;
     if (c.over) {                                        // (uniform)
-        if (tid == 0 && (id & ((1u << a.bk2_lnb) - 1u)) == 0u) push_rest(a, id, FS_REST_BUCKET);
+        if (tid == 0 && (id & ((1u << a.bk2_lnb) - 1u)) == 0u) {
+            __hip_atomic_fetch_add(gptr<uint32_t>(a.bk2_tab) + FS_BK2_OVERS, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            push_rest(a, id, FS_REST_BUCKET);
+        }
         return;
     }
     if (c.len == 0u) return;
@@ -1415,7 +1419,7 @@ DEV void rest_body(const FsArgs& a) {
         uint32_t b[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
         for (uint32_t i = 0; i < 4u * FS_BK_BIT_SLOTS; ++i) b[i % 4u] |= tab1[FS_BK_BITS + i];
-        bucket_pass_info<K64>(a, ((uint64_t)(b[1] & b[3]) << 32) | (b[0] & b[2]));
+        bucket_pass_info<K64>(a, ((uint64_t)(b[1] & b[3]) << 32) | (b[0] & b[2]), tab2[FS_BK2_OVER] + tab2[FS_BK2_OVERS]);
     }
     if (tab2[FS_BK2_OVER]) {                             // (uniform)
         if (blockIdx.x == 0)

@@ -122,6 +122,7 @@ struct fs_sorter {
     uint32_t* last_plan = nullptr;
     bool last_fused = false;
     bool last_top16 = false;
+    uint32_t last_buckets = 0;           // the last sort's BucketPath
     uint32_t up_blocks_per_cu = 0;       // upsweep blocks per CU (0: by key width)
     uint32_t fault = FS_FAULT_NONE;      // injected fault (FS_FAULT_INJECTION builds only)
 
@@ -744,6 +745,7 @@ static fs_status enqueue_buckets(fs_sorter* s, fs_op op, fs_key_type t, void* ke
     // (a sort of the fused range whose first pass scatters into regions)
     s->last_fused = bp == BK_TWO_LEVELS && op == FS_OP_SORT && n >= FS_FUSED_MIN_KEYS;
     s->last_top16 = false;
+    s->last_buckets = bp;
     return FS_OK;
 }
 
@@ -1433,6 +1435,18 @@ fs_status fs_sorter_first_pass(fs_sorter* s, uint32_t* kind) {
         *kind = w[FS_PLAN_RESCATTER] ? 4u : 3u;
     else
         *kind = !s->last_fused ? 0u : ((mask & FS_MASK_FUSED) && !w[FS_PLAN_RESCATTER]) ? 1u : 2u;
+    return FS_OK;
+}
+
+fs_status fs_last_bucket_info(fs_sorter* s, uint32_t* path, uint32_t* overflows) {
+    if (!s || !path || !overflows) return FS_ERR_INVALID_ARGUMENT;
+    fs_status r = drain(s);
+    if (r != FS_OK) return r;
+    uint32_t w[FS_PLAN_WORDS];
+    HIP_TRY(s, hipMemcpy(w, s->last_plan ? s->last_plan : s->plan, sizeof w, hipMemcpyDeviceToHost));
+    const bool buckets = (w[FS_PLAN_MASK] & FS_MASK_BUCKETS) != 0u;
+    *path = buckets ? s->last_buckets : 0u;
+    *overflows = buckets ? w[FS_PLAN_RESCATTER] : 0u;
     return FS_OK;
 }
 

@@ -277,6 +277,7 @@
 #define FS_PLAN_NPASSES (FS_MAX_DIGITS * FS_PLAN_PASS_WORDS)      // passes that run
 #define FS_PLAN_MASK (FS_PLAN_NPASSES + 1)                         // bit j: digit j sorted
 #define FS_MASK_FUSED (1u << 8)     // mask word: the fused first pass's regions were used
+#define FS_MASK_BUCKETS (1u << 10)  // mask word: buckets did the sort (bucket_sort.h)
 #define FS_MASK_TOP16 (1u << 9)     // mask word: the top-16 path ran (digit passes on the two top
                                     // digits, then the local sort of each top-16-bit segment)
 #define FS_PLAN_TICKET (FS_PLAN_NPASSES + 2)                       // upsweep blocks finished (0 between sorts)
@@ -485,12 +486,14 @@
 #define FS_BC64_WAVES 5
 #define FS_BC64V_WAVES 5
 // Second-level table words: 1 when a first-level region overflowed, entries
-// of the rest list, the path taken, then per bucket its description (keys, S1 region, place in
+// of the rest list, the path taken, the buckets of which a child's region
+// overflowed, then per bucket its description (keys, S1 region, place in
 // the output, first tile, 1: one value), and per child the count, region base,
 // capacity and splitter
 #define FS_BK2_OVER 0u
 #define FS_BK2_RESTS 1u
 #define FS_BK2_MODE 2u             // 0: buckets; 1: digit passes (few digits vary)
+#define FS_BK2_OVERS 3u
 #define FS_BK2_INFO 4u
 #define FS_BK2_INFO_WORDS 8u
 #define FS_BK2_CHILDREN (FS_BK_NB * FS_BK2_NB)

@@ -44,6 +44,8 @@ TOP16_BY_SIZE, TOP16_NEVER, TOP16_ALWAYS, TOP16_SAMPLED = 0, 1, 2, 3   # TEST_TO
 FUSED_MIN_KEYS = 1 << 25                                 # FS_FUSED_MIN_KEYS
 TOP16_MIN_KEYS32 = 44_040_192                            # FS_TOP16_MIN_KEYS32
 TOP16_MIN_KEYS64 = 1 << 21                               # FS_TOP16_MIN_KEYS64
+# fs_last_bucket_info: what did the last sort
+PATH_DIGITS, PATH_ONE_BLOCK, PATH_BUCKETS, PATH_TWO_LEVELS = 0, 1, 2, 3
 # fs_sorter_first_pass: how the last sort began
 FIRST_HISTOGRAM, FIRST_FUSED, FIRST_FUSED_OVERFLOW, FIRST_TOP16, FIRST_TOP16_RESCATTER = 0, 1, 2, 3, 4
 FAULT_NONE, FAULT_BAD_DIGITS, FAULT_BAD_BUFFER, FAULT_EXTRA_BLOCK, FAULT_STALL_TILE, FAULT_SMALL_S1 = 0, 1, 2, 3, 4, 5
@@ -141,6 +143,7 @@ def _load():
         "fs_allow_scratch_growth": ([vp], i),
         "fs_sorter_set_test_option": ([vp, i, u64], i),
         "fs_sorter_first_pass": ([vp, u32p], i),
+        "fs_last_bucket_info": ([vp, u32p, u32p], i),
         "fs_synchronize": ([vp], i),
         "fs_last_pass_info": ([vp, u32p, u32p], i),
         "fs_set_profiling": ([vp, i], i),
@@ -406,6 +409,14 @@ class GpuSorter:
         k = ctypes.c_uint32()
         self._check(_load().fs_sorter_first_pass(self._h, ctypes.byref(k)))
         return k.value
+
+    def last_bucket_info(self):
+        """(path, overflows) of the last sort: PATH_DIGITS (no buckets),
+        PATH_ONE_BLOCK, PATH_BUCKETS or PATH_TWO_LEVELS, and the bucket
+        regions that were too small for their keys."""
+        p, o = ctypes.c_uint32(), ctypes.c_uint32()
+        self._check(_load().fs_last_bucket_info(self._h, ctypes.byref(p), ctypes.byref(o)))
+        return p.value, o.value
 
     def device_synchronize(self):
         """Wait for everything on the device (hipDeviceSynchronize)."""

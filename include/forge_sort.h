@@ -302,6 +302,13 @@ fs_status fs_sorter_set_test_option(fs_sorter *s, fs_test_option opt, uint64_t v
  * re-scattered into exact regions by a second launch of the fused pass). */
 fs_status fs_sorter_first_pass(fs_sorter *s, uint32_t *kind);
 
+/* Whether buckets did the last completed sort: path 0 = no (digit passes, or
+ * the top-16 path), 1 = one block did all of it, 2 = one level of buckets,
+ * 3 = two levels.  overflows: the bucket regions (two levels: first-level
+ * regions, and buckets with an overflowed second-level one) that were too
+ * small for their keys; the sort is exact all the same, but slower. */
+fs_status fs_last_bucket_info(fs_sorter *s, uint32_t *path, uint32_t *overflows);
+
 /* ---- GpuGather (forge-runtime/src/gather.rs:26-173) --------------------------
  * output[i] = source[indices[i]] for u32 or u64 elements, u32 indices
  * (shaders/gather.metal:5-27).  The reference reads past the source for an

@@ -344,7 +344,19 @@ def check(sorter, op, kind, n, dist, seed):
         if fault:
             sorter.set_test_option(forge_sort.TEST_INJECT_FAULT, fault)
         try:
-            return check(sorter, rest, kind, n, dist, seed)
+            ok = check(sorter, rest, kind, n, dist, seed)
+            path, overflows = sorter.last_bucket_info()
+            want = {"one": forge_sort.PATH_ONE_BLOCK, "bk": forge_sort.PATH_BUCKETS, "bkover": forge_sort.PATH_BUCKETS}.get(
+                one, forge_sort.PATH_TWO_LEVELS)
+            # (two levels: keys of few varying digits go to the digit passes)
+            if path != want and not (want == forge_sort.PATH_TWO_LEVELS and path == forge_sort.PATH_DIGITS and not fault):
+                print(f"  path {path}, expected {want}", flush=True)
+                ok = False
+            # an injected small region overflows, and nothing else does
+            if bool(overflows) != bool(fault):
+                print(f"  {overflows} regions overflowed", flush=True)
+                ok = False
+            return ok
         finally:
             sorter.set_test_option(forge_sort.TEST_BUCKETS, forge_sort.BUCKETS_BY_SIZE)
             if fault:

@@ -51,7 +51,7 @@ def test_emulated_buckets_overflow(emulator):  # noqa: F811
     run_cases("faults", ["bkover_sort:u32:3000:uniform:1", "bkover_pairs:u64:2000:few:2", "bkover_argsort:f32:3000:uniform:3",
                          "bkover_sort:i64:2000:uniform:4",
                          # two levels: of the first (one block sorts all) or of every bucket's second child
-                         "twoover_sort:u64:9000:uniform:1", "twoover_pairs:u64:6000:few:2",
+                         "twoover_sort:u64:9000:uniform:1", "twoover_pairs:u64:6000:few:3",
                          "twosecond_sort:u64:9000:uniform:3", "twosecond_pairs:f64:9000:uniform:4"],
               env={"EMU_WORKERS": "1", "EMU_XCDS": "1"})   # (tiles in order: this build soon gives up a look-back wait)
 

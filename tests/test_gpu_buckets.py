@@ -104,7 +104,7 @@ def test_two_levels(sorter, op, kind, lnb, n):
     """Two levels of buckets, or the digit passes where few digits vary: least
     size, tile edges, few buckets (children larger than a block), every kind of
     data that takes another branch."""
-    from forge_sort import BUCKETS_BY_SIZE, BUCKETS_TWO_LEVELS, TEST_BUCKETS
+    from forge_sort import BUCKETS_BY_SIZE, BUCKETS_TWO_LEVELS, PATH_DIGITS, PATH_TWO_LEVELS, TEST_BUCKETS
     sorter.set_test_option(TEST_BUCKETS, BUCKETS_TWO_LEVELS + (lnb << 8))
     try:
         for i, data in enumerate(("normal", "quantised", "specials", "clusters", "sorted", "same", "narrow", "lone", "runs")):
@@ -115,6 +115,9 @@ def test_two_levels(sorter, op, kind, lnb, n):
             b = np.where(b & top, ~b, b | top) if kind == "f64" else b
             varying = int(np.bitwise_or.reduce(b ^ b[0]))
             assert sorter.last_pass_info()[1] == sum(1 << j for j in range(8) if varying >> (8 * j) & 0xFF)
+            path, _ = sorter.last_bucket_info()
+            digits = bin(sorter.last_pass_info()[1]).count("1")
+            assert path == PATH_TWO_LEVELS if digits > 4 else path in (PATH_TWO_LEVELS, PATH_DIGITS), (path, digits)
     finally:
         sorter.set_test_option(TEST_BUCKETS, BUCKETS_BY_SIZE)
 

@@ -41,8 +41,10 @@
 // block (16 bits) and the values follow by one gather at the end.
 //
 // Buckets are sized by the sample, so a bucket can outgrow its region or a
-// block's LDS (a region has room for its samples, six standard deviations of
-// them and FS_BK_ROOM more: below 10^-9 a bucket).  Such a sort stays exact:
+// block's LDS.  A region has room for the samples c that fell in its bucket,
+// six standard deviations of them and FS_BK_ROOM more: with as many keys, a
+// sample would show c or fewer of them below once in 10^9 (none at all: 10^7).
+// Such a sort stays exact:
 // the block of an oversized bucket, or block 0 for every key after an
 // overflowed region, sorts it alone through device memory (slow_sort).
 
@@ -630,7 +632,7 @@ DEV void split_body(const FsArgs& a) {
     // than two quantiles' share), their counts alone give the splitters: the
     // key a quantile's share of the way through its group.
     GroupMap<K64> map = group_map<K64>(least, most, a.xform == FS_XF_FLOAT);
-    uint32_t s0 = 0, s1 = 0;                             // samples below this thread's bucket, and below the next
+    uint32_t share = 0;                                  // samples in this thread's bucket
     bool spread = count_groups<K64, false, BLOCK, ITEMS>(k, m, map, per, 2u * stride, L);   // (uniform)
     if (!spread && map.by_value) {
         map = group_map<K64>(least, most, false);
@@ -639,9 +641,8 @@ DEV void split_body(const FsArgs& a) {
     if (spread) {
         for (uint32_t i = tid; i < NB; i += BLOCK) lbs[i] = i ? ~(K)0 : (K)0;
         __syncthreads();
-        s0 = tid * stride;
-        s1 = s0 + stride;
         if (tid >= 1u && tid < nb) {
+            const uint32_t s0 = tid * stride;
             uint32_t g = 0;                              // the group holding sample s0 (in order)
 #pragma unroll
             for (uint32_t step = 1u << (FS_BK_GBITS - 1); step; step >>= 1)
@@ -666,9 +667,29 @@ DEV void split_body(const FsArgs& a) {
 #pragma unroll
         for (uint32_t j = 0; j < TPT; ++j) {
             if (tid * TPT + j >= TG) continue;
+            const uint32_t here = tc[tid * TPT + j];
             gt[tid * TPT + j] = (uint16_t)tx;
-            tx += tc[tid * TPT + j];
+            tc[tid * TPT + j] = tx;
+            tx += here;
         }
+        // The bucket's share: the samples that fall in it, found as the
+        // partition finds its keys'.  (A quantile's share of samples each
+        // would hold only where keys spread within a group: two groups of one
+        // value each can share a bucket, four quantiles' share in all.)
+        uint32_t* const sc = reinterpret_cast<uint32_t*>(&L.wcnt[0][0]);
+        static_assert(sizeof(L.wcnt) >= 4u * NB, "the buckets' shares in the stable passes' words");
+        for (uint32_t i = tid; i < NB; i += BLOCK) sc[i] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if ((uint32_t)i >= per || row0 + (uint32_t)i * 64u >= m) continue;
+            const K key = k[i] + base;
+            uint32_t b = tc[map.of_key(key) >> 1];
+            while (b + 1u < nb && lbs[b + 1u] <= key) ++b;
+            atomicAdd(&sc[b], 1u);
+        }
+        __syncthreads();
+        if (tid < nb) share = sc[tid];
         if (tid == 0) {
             const uint64_t w64[4] = {(uint64_t)map.base, (uint64_t)map.span, __builtin_bit_cast(uint64_t, map.low),
                                      __builtin_bit_cast(uint64_t, map.scale)};
@@ -740,8 +761,8 @@ DEV void split_body(const FsArgs& a) {
             return x + ((x < m && L.keys[x] < t) ? 1u : 0u);
         };
         if (tid < nb) {
-            s0 = tid ? below(lbs[tid]) : 0u;
-            s1 = tid + 1u < nb ? below(lbs[tid + 1u]) : m;
+            const uint32_t s0 = tid ? below(lbs[tid]) : 0u, s1 = tid + 1u < nb ? below(lbs[tid + 1u]) : m;
+            share = s1 > s0 ? s1 - s0 : 0u;
         }
     }
 
@@ -751,7 +772,7 @@ DEV void split_body(const FsArgs& a) {
     // the sort stays exact.)
     uint32_t cap = 0;
     if (tid < nb) {
-        const float c = (float)(s1 > s0 ? s1 - s0 : 0u);
+        const float c = (float)share;
         const float room = c + 6.0f * __builtin_sqrtf(c) + FS_BK_ROOM;
         cap = ((uint32_t)(room * ((float)n / (float)m)) + 16u) & ~15u;
         if (cap > n) cap = (n + 15u) & ~15u;

@@ -39,6 +39,12 @@ def keys_for(kind, n, dist, seed, tile=None):
         b = g.integers(0, 1 << (64 if wide else 32), size=n, dtype=BITS[kind], endpoint=False)
     elif dist == "few":
         b = g.choice(g.integers(0, 1 << (64 if wide else 32), size=5, dtype=BITS[kind], endpoint=False), size=n)
+    elif dist.startswith("steps"):   # as many evenly spaced values (f64: k / (values - 1))
+        v = int(dist[5:])
+        k = g.integers(0, v, size=n, dtype=BITS[kind])
+        b = (k / (v - 1)).view(np.uint64) if kind == "f64" else k * BITS[kind](~BITS[kind](0) // BITS[kind](v))
+    elif dist.startswith("tenths"):  # f64: multiples of 0.1
+        b = (g.integers(0, int(dist[6:]), size=n) * 0.1).view(np.uint64)
     elif dist == "same":
         b = np.full(n, 7, dtype=BITS[kind])
     elif dist == "low12":

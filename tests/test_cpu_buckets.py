@@ -40,6 +40,16 @@ def test_emulated_buckets(emulator):  # noqa: F811
                        "bk_argsort:f32:30000:few:4", "bk_pairs:u64:20000:zipf:5"], parallel=3, env={"EMU_CUS": "8"})
 
 
+def test_emulated_buckets_of_repeated_values(emulator):  # noqa: F811
+    """Evenly spaced values, each in a group of the sample's own, so that a
+    bucket between two splitters can hold two of them: no region of either
+    level overflows (256 values each of a bucket: steps384 of two buckets)."""
+    run_cases("prod", ["two_sort:f64:200000:steps256:1", "two_pairs:f64:200000:tenths190:2",
+                       "two_sort:u64:200000:steps192:1", "two_argsort:i64:200000:steps256:1",
+                       "two1_sort:f64:850000:steps384:2", "two1_sort:u64:850000:steps384:3",
+                       "bk_sort:u32:200000:steps400:1", "bk_pairs:u64:200000:steps300:2"], parallel=4, env={"EMU_CUS": "8"})
+
+
 @pytest.mark.parametrize("order", ["wave", "wave_rev"])
 def test_emulated_buckets_wave_serial(emulator, order):  # noqa: F811
     run_cases("small", CASES + TWO, timeout=900, env={"EMU_SCHED": order}, parallel=4)

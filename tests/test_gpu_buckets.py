@@ -115,9 +115,10 @@ def test_two_levels(sorter, op, kind, lnb, n):
             b = np.where(b & top, ~b, b | top) if kind == "f64" else b
             varying = int(np.bitwise_or.reduce(b ^ b[0]))
             assert sorter.last_pass_info()[1] == sum(1 << j for j in range(8) if varying >> (8 * j) & 0xFF)
-            path, _ = sorter.last_bucket_info()
+            path, overflows = sorter.last_bucket_info()
             digits = bin(sorter.last_pass_info()[1]).count("1")
             assert path == PATH_TWO_LEVELS if digits > 4 else path in (PATH_TWO_LEVELS, PATH_DIGITS), (path, digits)
+            assert overflows == 0
     finally:
         sorter.set_test_option(TEST_BUCKETS, BUCKETS_BY_SIZE)
 

@@ -43,8 +43,8 @@
 // Buckets are sized by the sample, so a bucket can outgrow its region or a
 // block's LDS.  A region has room for the samples c that fell in its bucket,
 // six standard deviations of them and FS_BK_ROOM more: with as many keys, a
-// sample would show c or fewer of them below once in 10^9 (none at all: 10^7).
-// Such a sort stays exact:
+// sample would show c or fewer of them below once in 10^9 (none at all: 10^7;
+// c not counted but bounded, see split_body: 10^5).  Such a sort stays exact:
 // the block of an oversized bucket, or block 0 for every key after an
 // overflowed region, sorts it alone through device memory (slow_sort).
 
@@ -640,17 +640,32 @@ DEV void split_body(const FsArgs& a) {
     }
     if (spread) {
         for (uint32_t i = tid; i < NB; i += BLOCK) lbs[i] = i ? ~(K)0 : (K)0;
+        uint32_t* const gi = reinterpret_cast<uint32_t*>(&L.wcnt[0][0]);   // each splitter's group
+        static_assert(sizeof(L.wcnt) >= 4u * NB, "the splitters' groups, then the shares, in the stable passes' words");
+        if (tid == 0) L.flag = 0u;
         __syncthreads();
+        uint32_t g = 0;                                  // the group holding sample s0 (in order)
         if (tid >= 1u && tid < nb) {
             const uint32_t s0 = tid * stride;
-            uint32_t g = 0;                              // the group holding sample s0 (in order)
 #pragma unroll
             for (uint32_t step = 1u << (FS_BK_GBITS - 1); step; step >>= 1)
                 if (L.starts[g + step] <= s0) g += step;
             const uint32_t g0 = L.starts[g], gn = L.starts[g + 1u] - g0;
             lbs[tid] = map.inside(g, gn ? (float)(s0 - g0) / (float)gn : 0.0f);
+            gi[tid] = g;
         }
         __syncthreads();
+        // A bucket's share of the samples: a quantile's where keys spread
+        // within the splitters' groups, but up to all of both its splitters'
+        // groups where those are of a value each.  Where that is more, in any
+        // bucket, than a quantile's room holds but for once in 10^5, the
+        // samples are counted below.  (Counting them always took 1.6 us more:
+        // u32, 1M keys, 44.1 -> 45.8.)
+        if (tid < nb) {
+            const uint32_t to = tid + 1u < nb ? L.starts[gi[tid + 1u] + 1u] : m;
+            if ((float)(to - L.starts[g]) > (float)stride + 2.0f * __builtin_sqrtf((float)stride) + 4.0f) L.flag = 1u;
+            share = stride;
+        }
         // The partition finds a key's bucket from its group: the splitters in
         // smaller groups, all below the key, then the few in its own.
         constexpr uint32_t TG = 1u << (FS_BK_GBITS - 1), TPT = (TG + BLOCK - 1) / BLOCK;
@@ -672,24 +687,21 @@ DEV void split_body(const FsArgs& a) {
             tc[tid * TPT + j] = tx;
             tx += here;
         }
-        // The bucket's share: the samples that fall in it, found as the
-        // partition finds its keys'.  (A quantile's share of samples each
-        // would hold only where keys spread within a group: two groups of one
-        // value each can share a bucket, four quantiles' share in all.)
-        uint32_t* const sc = reinterpret_cast<uint32_t*>(&L.wcnt[0][0]);
-        static_assert(sizeof(L.wcnt) >= 4u * NB, "the buckets' shares in the stable passes' words");
-        for (uint32_t i = tid; i < NB; i += BLOCK) sc[i] = 0u;
-        __syncthreads();
+        if (L.flag) {                                    // (uniform) count them, found as the partition finds its keys'
+            uint32_t* const sc = reinterpret_cast<uint32_t*>(&L.wcnt[0][0]);
+            for (uint32_t i = tid; i < NB; i += BLOCK) sc[i] = 0u;
+            __syncthreads();
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            if ((uint32_t)i >= per || row0 + (uint32_t)i * 64u >= m) continue;
-            const K key = k[i] + base;
-            uint32_t b = tc[map.of_key(key) >> 1];
-            while (b + 1u < nb && lbs[b + 1u] <= key) ++b;
-            atomicAdd(&sc[b], 1u);
+            for (int i = 0; i < ITEMS; ++i) {
+                if ((uint32_t)i >= per || row0 + (uint32_t)i * 64u >= m) continue;
+                const K key = k[i] + base;
+                uint32_t b = tc[map.of_key(key) >> 1];
+                while (b + 1u < nb && lbs[b + 1u] <= key) ++b;
+                atomicAdd(&sc[b], 1u);
+            }
+            __syncthreads();
+            if (tid < nb) share = sc[tid];
         }
-        __syncthreads();
-        if (tid < nb) share = sc[tid];
         if (tid == 0) {
             const uint64_t w64[4] = {(uint64_t)map.base, (uint64_t)map.span, __builtin_bit_cast(uint64_t, map.low),
                                      __builtin_bit_cast(uint64_t, map.scale)};

@@ -45,8 +45,10 @@
 // six standard deviations of them and FS_BK_ROOM more: with as many keys, a
 // sample would show c or fewer of them below once in 10^9 (none at all: 10^7;
 // c not counted but bounded, see split_body: 10^5).  Such a sort stays exact:
-// the block of an oversized bucket, or block 0 for every key after an
-// overflowed region, sorts it alone through device memory (slow_sort).
+// the block of an oversized bucket sorts it alone through device memory
+// (slow_sort); after an overflowed region every bucket's block gathers its keys
+// from the caller's first (sort_overflowed; of two levels, fs_rest_*'s block 0
+// sorts everything).
 
 // Elements of the LDS block sort of WAVES waves: rows of 64 keys, `per` rows
 // to each wave (wave w: rows w * per ...), so that a small segment still uses
@@ -599,6 +601,7 @@ DEV void split_body(const FsArgs& a) {
         if (blockIdx.x) return;                          // (uniform)
         for (uint32_t i = tid; i < nb; i += BLOCK) st_agent(&cnt[i], 0u);
         for (uint32_t i = tid; i < 4u * FS_BK_BIT_SLOTS; i += BLOCK) st_agent(&tab1[FS_BK_BITS + i], 0u);
+        if (tid == 0) st_agent(&tab1[FS_BK_DONE], 0u);
         if (a.bk2_tab && tid < FS_BK2_INFO && tid != FS_BK2_MODE) st_agent(&tab2[tid], 0u);
     }
 
@@ -1146,18 +1149,19 @@ DEV void slow_sort(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool fwd, ui
 }
 
 // One block sorts len keys (at most its LDS's) at src_k, with their values at
-// src_v (0: their positions, argsort), into the caller's keys and values from
-// `start` on.  whole: the source is the caller's (transformed on load).
+// src_v (0: their positions, argsort), into dst_k (not of an argsort) and
+// dst_v, as the caller's keys.  whole: the source is the caller's (transformed
+// on load).
 template <bool K64, bool VALS, int BLOCK, int ITEMS>
-DEV void block_range_sort(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool whole, uint32_t start, uint32_t len,
-                          BlockSortLds<K64, VALS, BLOCK, ITEMS>& L) {
+DEV void block_range_sort(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool whole, uint32_t len, uint64_t dst_k,
+                          uint64_t dst_v, BlockSortLds<K64, VALS, BLOCK, ITEMS>& L) {
     typedef typename KeyT<K64>::type K;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
     const bool put_keys = a.op != FSK_OP_ARGSORT;
     K xa, xb;
     xf_inv_masks<K64>(a.xform, xa, xb);
-    GLOBAL K* dk = gptr<K>(a.keys);
-    GLOBAL uint32_t* dv = gptr<uint32_t>(a.vals);
+    GLOBAL K* dk = gptr<K>(dst_k);
+    GLOBAL uint32_t* dv = gptr<uint32_t>(dst_v);
     const uint32_t per = (len + BLOCK - 1u) / BLOCK;     // rows per wave
     const uint32_t row0 = w * per * 64u + lane;
     const GLOBAL K* src = gptr<const K>(src_k);
@@ -1191,20 +1195,115 @@ DEV void block_range_sort(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool 
             const uint32_t x = (uint32_t)i * BLOCK + tid;
             v[i] = x < len ? (src_v ? sv[L.pos[x]] : L.pos[x]) : 0u;
         }
-        if (whole) __syncthreads();                     // in place: every value read before any is written
+        if (src_v == dst_v) __syncthreads();            // (uniform) in place: every value read before any is written
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
             const uint32_t x = (uint32_t)i * BLOCK + tid;
-            if (x < len) dv[start + x] = v[i];
+            if (x < len) dv[x] = v[i];
         }
     }
     if (put_keys) {
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
             const uint32_t x = (uint32_t)i * BLOCK + tid;
-            if (x < len) dk[start + x] = xf_inv_apply<K64>((K)(L.keys[x] + base), xa, xb);
+            if (x < len) dk[x] = xf_inv_apply<K64>((K)(L.keys[x] + base), xa, xb);
         }
     }
+}
+
+// The keys of one bucket (lo <= key, and key < hi unless it is the last), in
+// order, from the len keys at src_k to dst_k, with their values (dst_v 0: none;
+// src_v 0: their positions, argsort).  fwd: the source holds the caller's keys.
+// ws: 2 * BLOCK / 64 words of LDS.
+template <bool K64, int BLOCK>
+DEV void gather_bucket(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool fwd, uint32_t len, typename KeyT<K64>::type lo,
+                       typename KeyT<K64>::type hi, bool last, uint64_t dst_k, uint64_t dst_v, uint32_t count, uint32_t* ws) {
+    typedef typename KeyT<K64>::type K;
+    constexpr int WAVES = BLOCK / 64, IT = 4;
+    constexpr uint32_t CH = BLOCK * IT;
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, wb = w * 64u * IT + lane;
+    const uint32_t xf = fwd ? a.xform : FS_XF_NONE;
+    const GLOBAL K* in = gptr<const K>(src_k);
+    GLOBAL K* out = gptr<K>(dst_k);
+    uint32_t done = 0, half = 0;                         // (the waves' counts alternate between two halves of ws)
+    for (uint32_t c0 = 0; c0 < len; c0 += CH, half ^= 1u) {
+        K k[IT];
+        uint64_t in_bucket[IT];
+        uint32_t mine = 0;
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const uint32_t p = c0 + wb + (uint32_t)i * 64u;
+            k[i] = p < len ? xf_fwd<K64>(in[p], xf) : (K)0;
+        }
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const bool is = c0 + wb + (uint32_t)i * 64u < len && k[i] >= lo && (last || k[i] < hi);
+            in_bucket[i] = __builtin_amdgcn_uicmp((uint32_t)is, 0u, 33);
+            mine += (uint32_t)__builtin_popcountll(in_bucket[i]);
+        }
+        if (lane == 0u) ws[half * WAVES + w] = mine;
+        __syncthreads();
+        uint32_t at = done;
+#pragma unroll
+        for (uint32_t ww = 0; ww < (uint32_t)WAVES; ++ww) {
+            const uint32_t c = ws[half * WAVES + ww];
+            at += ww < w ? c : 0u;
+            done += c;
+        }
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const uint32_t p = c0 + wb + (uint32_t)i * 64u, r = lanes_below(in_bucket[i], at);
+            if (((in_bucket[i] >> lane) & 1u) && r < count) {
+                out[r] = k[i];
+                if (dst_v) gptr<uint32_t>(dst_v)[r] = src_v ? gptr<const uint32_t>(src_v)[p] : p;
+            }
+            at += (uint32_t)__builtin_popcountll(in_bucket[i]);
+        }
+    }
+    __syncthreads();
+}
+
+// A sort of which some region overflowed, its keys incomplete in S1: every
+// bucket's block gathers its keys from the caller's into S2, at their place in
+// the output, and sorts them there; the block that ends last copies S2 back
+// (the others may still read the caller's keys before).  start, len: the
+// block's bucket by the partition's counts, which are whole.
+template <bool K64, bool VALS, int BLOCK, int ITEMS>
+DEV void sort_overflowed(const FsArgs& a, uint32_t start, uint32_t len, BlockSortLds<K64, VALS, BLOCK, ITEMS>& L) {
+    typedef typename KeyT<K64>::type K;
+    __shared__ uint32_t s_last;
+    const uint32_t tid = threadIdx.x, nb = 1u << a.bk_lnb, j = blockIdx.x, n = (uint32_t)a.n;
+    const bool put_keys = a.op != FSK_OP_ARGSORT, last = j + 1u == nb;
+    GLOBAL uint32_t* tab = gptr<uint32_t>(a.bk_tab);
+    const GLOBAL K* lbs = reinterpret_cast<const GLOBAL K*>(tab + FS_BK_LB);
+    const K lo = lbs[j], hi = last ? (K)0 : lbs[j + 1u];
+    const uint64_t k1 = a.s1k + (uint64_t)start * sizeof(K), v1 = a.s1v + (uint64_t)start * 4u;
+    const uint64_t k2 = a.s2k + (uint64_t)start * sizeof(K), v2 = a.s2v + (uint64_t)start * 4u;
+    K xa, xb;
+    xf_inv_masks<K64>(a.xform, xa, xb);
+    if (len) {                                           // (uniform, as every branch here)
+        gather_bucket<K64, BLOCK>(a, a.keys, a.op == FSK_OP_PAIRS ? a.vals : 0u, true, n, lo, hi, last, k2, VALS ? v2 : 0u,
+                                  len, reinterpret_cast<uint32_t*>(&L.red[0][0]));
+        if (last ? lo == ~(K)0 : hi - lo == (K)1) {      // one value: in order as it is
+            const K v = xf_inv_apply<K64>(lo, xa, xb);
+            for (uint32_t p = tid; p < len; p += BLOCK) gptr<K>(k2)[p] = v;
+        } else if (len <= (uint32_t)(BLOCK * ITEMS)) {
+            block_range_sort<K64, VALS, BLOCK, ITEMS>(a, k2, VALS ? v2 : 0u, false, len, k2, v2, L);
+        } else {
+            slow_sort<K64, VALS, BLOCK, ITEMS>(a, k2, v2, false, k1, v1, k2, v2, k2, v2, len, L);
+        }
+    }
+    __threadfence();                                     // the bucket in S2, before it is counted as done
+    __syncthreads();
+    if (tid == 0)
+        s_last = __hip_atomic_fetch_add(&tab[FS_BK_DONE], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nb - 1u;
+    __syncthreads();
+    if (!s_last) return;                                 // (uniform)
+    __threadfence();
+    if (put_keys)
+        for (uint32_t p = tid; p < n; p += BLOCK) gptr<K>(a.keys)[p] = gptr<const K>(a.s2k)[p];
+    if (VALS)
+        for (uint32_t p = tid; p < n; p += BLOCK) gptr<uint32_t>(a.vals)[p] = gptr<const uint32_t>(a.s2v)[p];
 }
 
 template <bool K64, bool VALS, int BLOCK, int ITEMS>
@@ -1262,11 +1361,9 @@ DEV void bucket_body(const FsArgs& a) {
             for (uint32_t i = 0; i < 4u * FS_BK_BIT_SLOTS; ++i) b[i % 4u] |= tab[FS_BK_BITS + i];
             bucket_pass_info<K64>(a, ((uint64_t)(b[1] & b[3]) << 32) | (b[0] & b[2]), s_over);
         }
-        if (s_over) {                                   // (uniform) a region overflowed: block 0 sorts the caller's keys
+        if (s_over) {                                   // (uniform) a region overflowed
             __syncthreads();
-            if (blockIdx.x == 0)
-                slow_sort<K64, VALS, BLOCK, ITEMS>(a, a.keys, src_v, true, a.s2k, a.s2v, a.s1k, a.s1v, a.keys, a.vals,
-                                                   (uint32_t)a.n, L);
+            sort_overflowed<K64, VALS, BLOCK, ITEMS>(a, start, len, L);
             return;
         }
         const uint32_t giants = s_giants;
@@ -1299,7 +1396,8 @@ DEV void bucket_body(const FsArgs& a) {
         return;
     }
 
-    block_range_sort<K64, VALS, BLOCK, ITEMS>(a, src_k, src_v, whole, start, len, L);
+    block_range_sort<K64, VALS, BLOCK, ITEMS>(a, src_k, src_v, whole, len, a.keys + (uint64_t)start * sizeof(K),
+                                              a.vals + (uint64_t)start * 4u, L);
 }
 
 // ---------------------------------------------------------------------------
@@ -1482,7 +1580,8 @@ DEV void rest_body(const FsArgs& a) {
             const uint64_t sk = bucket ? k1 : k2, sv = bucket ? v1 : v2;
             if (bucket || what == FS_REST_SORT) {
                 if (!bucket && len <= (uint32_t)(BLOCK * ITEMS))
-                    block_range_sort<K64, VALS, BLOCK, ITEMS>(a, sk, VALS ? sv : 0u, false, start, len, L);
+                    block_range_sort<K64, VALS, BLOCK, ITEMS>(a, sk, VALS ? sv : 0u, false, len, a.keys + (uint64_t)start * sizeof(K),
+                                                              a.vals + (uint64_t)start * 4u, L);
                 else
                     slow_sort<K64, VALS, BLOCK, ITEMS>(a, sk, sv, false, bucket ? k2 : k1, bucket ? v2 : v1, sk, sv,
                                                        a.keys + (uint64_t)start * sizeof(K),

@@ -462,7 +462,9 @@
 #define FS_BK_MAP_HEAD 12u
 #define FS_BK_MAP_WORDS (FS_BK_MAP_HEAD + (1u << (FS_BK_GBITS - 2)))
 #define FS_BK_MAP (FS_BK_LB + 2u * FS_BK_NB)
-#define FS_BK_TAB_WORDS (FS_BK_MAP + FS_BK_MAP_WORDS)
+// ... and, after an overflow, the buckets' blocks that are done
+#define FS_BK_DONE (FS_BK_MAP + FS_BK_MAP_WORDS)
+#define FS_BK_TAB_WORDS (FS_BK_DONE + 1u)
 // Two levels: children of a bucket, and the threads, keys per thread, group
 // bits and waves per SIMD of the blocks that sort them
 #ifndef FS_BK2_LNB

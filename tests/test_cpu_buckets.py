@@ -56,10 +56,15 @@ def test_emulated_buckets_wave_serial(emulator, order):  # noqa: F811
 
 
 def test_emulated_buckets_overflow(emulator):  # noqa: F811
-    """A region with room for one row only: its keys do not fit, and one block
-    sorts the caller's keys instead (the fault-injection build)."""
+    """A region with room for one row only: its keys do not fit, and every
+    bucket's block gathers its keys from the caller's instead (the
+    fault-injection build): every op, few values, buckets larger than a block
+    and of one value, an odd start."""
     run_cases("faults", ["bkover_sort:u32:3000:uniform:1", "bkover_pairs:u64:2000:few:2", "bkover_argsort:f32:3000:uniform:3",
-                         "bkover_sort:i64:2000:uniform:4",
+                         "bkover_sort:i64:2000:uniform:4", "bkover_pairs:f64:3001:uniform:5", "bkover_sort:f32:3000:few:6",
+                         "bkover_argsort:u64:3000:few:1", "bkover2_sort:u32:5000:uniform:2", "bkover2_pairs:u64:5000:uniform:3",
+                         "bkover2_argsort:i32:5000:few:3", "bkover_pairs:u32:5000:zipf:9", "bkover_sort:u32:5000:zipf:9",
+                         "bkover_offset:i64:3001:uniform:7",
                          # two levels: of the first (one block sorts all) or of every bucket's second child
                          "twoover_sort:u64:9000:uniform:1", "twoover_pairs:u64:6000:few:3",
                          "twosecond_sort:u64:9000:uniform:3", "twosecond_pairs:f64:9000:uniform:4"],

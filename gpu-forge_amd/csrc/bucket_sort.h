@@ -47,8 +47,8 @@
 // c not counted but bounded, see split_body: 10^5).  Such a sort stays exact:
 // the block of an oversized bucket sorts it alone through device memory
 // (slow_sort); after an overflowed region every bucket's block gathers its keys
-// from the caller's first (sort_overflowed; of two levels, fs_rest_*'s block 0
-// sorts everything).
+// from the caller's first (sort_overflowed; of two levels, fs_split2_*), and a
+// bucket with an overflowed child is sorted from S1 by one block (fs_rest_*).
 
 // Elements of the LDS block sort of WAVES waves: rows of 64 keys, `per` rows
 // to each wave (wave w: rows w * per ...), so that a small segment still uses
@@ -505,6 +505,61 @@ DEV void bucket_pass_info(const FsArgs& a, uint64_t varying, uint32_t overs) {
     st_agent(&plan[FS_PLAN_RESCATTER], overs);
 }
 
+// The keys of one bucket (lo <= key, and key < hi unless it is the last), in
+// order, from the len keys at src_k to dst_k, with their values (dst_v 0: none;
+// src_v 0: their positions, argsort).  fwd: the source holds the caller's keys.
+// ws: 2 * BLOCK / 64 words of LDS.  Every block reads the whole source, which
+// bounds it: 3 TB/s of a grid of 256 (8 keys per thread in flight: a tenth
+// faster).  With one region too small, us, against a sort without: u32, 1M keys
+// 1,420 / 54; f64, two levels, 2M 1,250 / 170, 16M 10,000 / 390, 128M 91,900 / 2,260.
+template <bool K64, int BLOCK>
+DEV void gather_bucket(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool fwd, uint32_t len, typename KeyT<K64>::type lo,
+                       typename KeyT<K64>::type hi, bool last, uint64_t dst_k, uint64_t dst_v, uint32_t count, uint32_t* ws) {
+    typedef typename KeyT<K64>::type K;
+    constexpr int WAVES = BLOCK / 64, IT = 4;
+    constexpr uint32_t CH = BLOCK * IT;
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, wb = w * 64u * IT + lane;
+    const uint32_t xf = fwd ? a.xform : FS_XF_NONE;
+    const GLOBAL K* in = gptr<const K>(src_k);
+    GLOBAL K* out = gptr<K>(dst_k);
+    uint32_t done = 0, half = 0;                         // (the waves' counts alternate between two halves of ws)
+    for (uint32_t c0 = 0; c0 < len; c0 += CH, half ^= 1u) {
+        K k[IT];
+        uint64_t in_bucket[IT];
+        uint32_t mine = 0;
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const uint32_t p = c0 + wb + (uint32_t)i * 64u;
+            k[i] = p < len ? xf_fwd<K64>(in[p], xf) : (K)0;
+        }
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const bool is = c0 + wb + (uint32_t)i * 64u < len && k[i] >= lo && (last || k[i] < hi);
+            in_bucket[i] = __builtin_amdgcn_uicmp((uint32_t)is, 0u, 33);
+            mine += (uint32_t)__builtin_popcountll(in_bucket[i]);
+        }
+        if (lane == 0u) ws[half * WAVES + w] = mine;
+        __syncthreads();
+        uint32_t at = done;
+#pragma unroll
+        for (uint32_t ww = 0; ww < (uint32_t)WAVES; ++ww) {
+            const uint32_t c = ws[half * WAVES + ww];
+            at += ww < w ? c : 0u;
+            done += c;
+        }
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const uint32_t p = c0 + wb + (uint32_t)i * 64u, r = lanes_below(in_bucket[i], at);
+            if (((in_bucket[i] >> lane) & 1u) && r < count) {
+                out[r] = k[i];
+                if (dst_v) gptr<uint32_t>(dst_v)[r] = src_v ? gptr<const uint32_t>(src_v)[p] : p;
+            }
+            at += (uint32_t)__builtin_popcountll(in_bucket[i]);
+        }
+    }
+    __syncthreads();
+}
+
 // ---------------------------------------------------------------------------
 // fs_split_*: the splitters
 // ---------------------------------------------------------------------------
@@ -555,7 +610,7 @@ DEV void split_body(const FsArgs& a) {
         const bool one = tid < nb1 && (tid + 1u < nb1 ? lb1[tid + 1u] - lb1[tid] == (K)1 : lb1[tid] == ~(K)0);
         if (tid == 0) L.flag = 0u;
         const uint32_t start = block_exclusive_scan<BLOCK>(c, L.wsum), tstart = block_exclusive_scan<BLOCK>(t, L.wsum);
-        if (tid < nb1 && c > tab1[FS_BK_CAPS + tid]) L.flag = 1u;
+        if (tid < nb1 && c > tab1[FS_BK_CAPS + tid]) atomicAdd(&L.flag, 1u);
         if (tid == par) {
             s_par[0] = c;
             s_par[1] = start;
@@ -563,14 +618,23 @@ DEV void split_body(const FsArgs& a) {
             s_par[3] = one ? 1u : 0u;
         }
         __syncthreads();
-        if (L.flag) {                                    // (uniform) a region overflowed: fs_rest_* sorts the caller's keys
-            if (tid == 0 && par == 0u) st_agent(&tab2[FS_BK2_OVER], 1u);
-            return;
-        }
         n = s_par[0];
         origin = (uint32_t)(((uint64_t)s_par[1] * a.bk2_room) >> 8) + par * (32u * nb + 64u);
         origin = (origin + 15u) & ~15u;
-        const uint32_t rbase = tab1[FS_BK_BASE + par], ts = s_par[2], tn = (n + a.tile - 1u) / a.tile;
+        uint32_t rbase = tab1[FS_BK_BASE + par];
+        const uint32_t ts = s_par[2], tn = (n + a.tile - 1u) / a.tile;
+        if (L.flag) {
+            // (uniform over the grid) a region overflowed: every block gathers
+            // its bucket's keys from the caller's, which are still whole, to
+            // their place in the output within S1
+            if (tid == 0 && par == 0u) st_agent(&tab2[FS_BK2_OVER], L.flag);
+            rbase = s_par[1];
+            const bool last = par + 1u == nb1;
+            gather_bucket<K64, BLOCK>(a, a.keys, a.op == FSK_OP_PAIRS ? a.vals : 0u, true, (uint32_t)a.n, lb1[par],
+                                      last ? (K)0 : lb1[par + 1u], last, a.s1k + (uint64_t)rbase * sizeof(K),
+                                      a.op != FSK_OP_KEYS ? a.s1v + (uint64_t)rbase * 4u : 0u, n,
+                                      reinterpret_cast<uint32_t*>(&L.red[0][0]));
+        }
         if (tid < FS_BK2_INFO_WORDS) {
             const uint32_t v = tid == 0u ? n : tid == 1u ? rbase : tid == 2u ? s_par[1] : tid == 3u ? ts : tid == 4u ? s_par[3] : 0u;
             tab2[FS_BK2_INFO + par * FS_BK2_INFO_WORDS + tid] = v;
@@ -846,7 +910,6 @@ DEV void part_body(const FsArgs& a) {
     uint64_t src_k = a.keys, src_v = a.vals;
     uint64_t lb_at = 0, grp_at = (uint64_t)a.num_tiles * nb;
     if constexpr (L2) {
-        if (((const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab)[FS_BK2_OVER]) return;   // (uniform)
         par = ((const CONSTANT uint32_t*)(uintptr_t)a.tilemap)[blockIdx.x];
         if (par >= 1u << a.bk_lnb) return;              // no tile for this block
         const CONSTANT uint32_t* info = (const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab + FS_BK2_INFO + par * FS_BK2_INFO_WORDS;
@@ -1211,58 +1274,6 @@ DEV void block_range_sort(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool 
     }
 }
 
-// The keys of one bucket (lo <= key, and key < hi unless it is the last), in
-// order, from the len keys at src_k to dst_k, with their values (dst_v 0: none;
-// src_v 0: their positions, argsort).  fwd: the source holds the caller's keys.
-// ws: 2 * BLOCK / 64 words of LDS.
-template <bool K64, int BLOCK>
-DEV void gather_bucket(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool fwd, uint32_t len, typename KeyT<K64>::type lo,
-                       typename KeyT<K64>::type hi, bool last, uint64_t dst_k, uint64_t dst_v, uint32_t count, uint32_t* ws) {
-    typedef typename KeyT<K64>::type K;
-    constexpr int WAVES = BLOCK / 64, IT = 4;
-    constexpr uint32_t CH = BLOCK * IT;
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, wb = w * 64u * IT + lane;
-    const uint32_t xf = fwd ? a.xform : FS_XF_NONE;
-    const GLOBAL K* in = gptr<const K>(src_k);
-    GLOBAL K* out = gptr<K>(dst_k);
-    uint32_t done = 0, half = 0;                         // (the waves' counts alternate between two halves of ws)
-    for (uint32_t c0 = 0; c0 < len; c0 += CH, half ^= 1u) {
-        K k[IT];
-        uint64_t in_bucket[IT];
-        uint32_t mine = 0;
-#pragma unroll
-        for (int i = 0; i < IT; ++i) {
-            const uint32_t p = c0 + wb + (uint32_t)i * 64u;
-            k[i] = p < len ? xf_fwd<K64>(in[p], xf) : (K)0;
-        }
-#pragma unroll
-        for (int i = 0; i < IT; ++i) {
-            const bool is = c0 + wb + (uint32_t)i * 64u < len && k[i] >= lo && (last || k[i] < hi);
-            in_bucket[i] = __builtin_amdgcn_uicmp((uint32_t)is, 0u, 33);
-            mine += (uint32_t)__builtin_popcountll(in_bucket[i]);
-        }
-        if (lane == 0u) ws[half * WAVES + w] = mine;
-        __syncthreads();
-        uint32_t at = done;
-#pragma unroll
-        for (uint32_t ww = 0; ww < (uint32_t)WAVES; ++ww) {
-            const uint32_t c = ws[half * WAVES + ww];
-            at += ww < w ? c : 0u;
-            done += c;
-        }
-#pragma unroll
-        for (int i = 0; i < IT; ++i) {
-            const uint32_t p = c0 + wb + (uint32_t)i * 64u, r = lanes_below(in_bucket[i], at);
-            if (((in_bucket[i] >> lane) & 1u) && r < count) {
-                out[r] = k[i];
-                if (dst_v) gptr<uint32_t>(dst_v)[r] = src_v ? gptr<const uint32_t>(src_v)[p] : p;
-            }
-            at += (uint32_t)__builtin_popcountll(in_bucket[i]);
-        }
-    }
-    __syncthreads();
-}
-
 // A sort of which some region overflowed, its keys incomplete in S1: every
 // bucket's block gathers its keys from the caller's into S2, at their place in
 // the output, and sorts them there; the block that ends last copies S2 back
@@ -1432,7 +1443,7 @@ DEV bool child_place(const FsArgs& a, uint32_t id, uint32_t* wsum, uint32_t* s_s
     const uint32_t par = id >> a.bk2_lnb, j = id & (nb - 1u);
     const CONSTANT uint32_t* tab2 = (const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab;
     const CONSTANT uint32_t* info = tab2 + FS_BK2_INFO + par * FS_BK2_INFO_WORDS;
-    if (tab2[FS_BK2_OVER] || info[0] == 0u || info[4]) return false;          // (uniform)
+    if (info[0] == 0u || info[4]) return false;          // (uniform)
     const GLOBAL uint32_t* t = gptr<const uint32_t>(a.bk2_tab);
     const uint32_t n = tid < nb ? t[FS_BK2_CNT + par * FS_BK2_NB + tid] : 0u;
     const uint32_t cap = tid < nb ? t[FS_BK2_CAPS + par * FS_BK2_NB + tid] : 0u;
@@ -1473,7 +1484,7 @@ DEV void child_body(const FsArgs& a) {
     const CONSTANT uint32_t* ctab = (const CONSTANT uint32_t*)(uintptr_t)a.bk2_tab;
     const uint32_t child = (id >> a.bk2_lnb) * FS_BK2_NB + (id & ((1u << a.bk2_lnb) - 1u));
     const CONSTANT uint32_t* cinfo = ctab + FS_BK2_INFO + (id >> a.bk2_lnb) * FS_BK2_INFO_WORDS;
-    if (ctab[FS_BK2_OVER] || ctab[FS_BK2_MODE] || cinfo[0] == 0u || cinfo[4]) return;   // (uniform)
+    if (ctab[FS_BK2_MODE] || cinfo[0] == 0u || cinfo[4]) return;   // (uniform)
     const uint32_t len0 = ctab[FS_BK2_CNT + child] <= CAP ? ctab[FS_BK2_CNT + child] : 0u;
     const uint32_t per = (len0 + BLOCK - 1u) / BLOCK, row0 = w * per * 64u + lane;
     const GLOBAL K* src = gptr<const K>(a.s2k) + ctab[FS_BK2_BASE + child];
@@ -1535,8 +1546,7 @@ DEV void child_body(const FsArgs& a) {
 // Second launch: a small grid takes the rest list in turn: children on the
 // one-level path's block sort (or through device memory when that is too
 // small), pieces of a child of one value, whole buckets whose children
-// outgrew their regions; everything, by one block, when a first-level region
-// did.
+// outgrew their regions.
 template <bool K64, bool VALS, int BLOCK, int ITEMS>
 DEV void rest_body(const FsArgs& a) {
     typedef typename KeyT<K64>::type K;
@@ -1551,12 +1561,6 @@ DEV void rest_body(const FsArgs& a) {
 #pragma unroll
         for (uint32_t i = 0; i < 4u * FS_BK_BIT_SLOTS; ++i) b[i % 4u] |= tab1[FS_BK_BITS + i];
         bucket_pass_info<K64>(a, ((uint64_t)(b[1] & b[3]) << 32) | (b[0] & b[2]), tab2[FS_BK2_OVER] + tab2[FS_BK2_OVERS]);
-    }
-    if (tab2[FS_BK2_OVER]) {                             // (uniform)
-        if (blockIdx.x == 0)
-            slow_sort<K64, VALS, BLOCK, ITEMS>(a, a.keys, a.op == FSK_OP_PAIRS ? a.vals : 0u, true, a.s2k, a.s2v, a.s1k,
-                                               a.s1v, a.keys, a.vals, (uint32_t)a.n, L);
-        return;
     }
     const uint32_t count = min(tab2[FS_BK2_RESTS], a.rest_cap);
     for (uint32_t e = blockIdx.x; e < count; e += gridDim.x) {

@@ -65,8 +65,9 @@ def test_emulated_buckets_overflow(emulator):  # noqa: F811
                          "bkover_argsort:u64:3000:few:1", "bkover2_sort:u32:5000:uniform:2", "bkover2_pairs:u64:5000:uniform:3",
                          "bkover2_argsort:i32:5000:few:3", "bkover_pairs:u32:5000:zipf:9", "bkover_sort:u32:5000:zipf:9",
                          "bkover_offset:i64:3001:uniform:7",
-                         # two levels: of the first (one block sorts all) or of every bucket's second child
-                         "twoover_sort:u64:9000:uniform:1", "twoover_pairs:u64:6000:few:3",
+                         # two levels: of the first (every bucket gathered by its block) or of every bucket's second child
+                         "twoover_sort:u64:9000:uniform:1", "twoover_pairs:u64:6000:few:3", "twoover_argsort:f64:9000:uniform:2",
+                         "twoover2_sort:i64:9000:uniform:5", "twoover_pairs:f64:9000:uniform:6", "twoover_sort:f64:9000:few:1",
                          "twosecond_sort:u64:9000:uniform:3", "twosecond_pairs:f64:9000:uniform:4"],
               env={"EMU_WORKERS": "1", "EMU_XCDS": "1"})   # (tiles in order: this build soon gives up a look-back wait)
 

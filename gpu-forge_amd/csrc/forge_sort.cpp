@@ -554,24 +554,12 @@ static fs_status reserve_buckets(fs_sorter* s, fs_op op, fs_key_type t, uint64_t
     return ensure(s, s->s2v, s2 * 4);
 }
 
-// Grows the scratch a sort of n keys needs, and every smaller one (grow-only,
-// like ensure_buffers*, lib.rs:1120-1289): ping-pong buffers for keys (and
-// values), two look-back arrays of tile entries followed by one 32-bit group
-// entry per FS_LB_GROUP tiles, and the bucket path's.
-static fs_status reserve(fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
-    if (n <= 1) return FS_OK;
+// Grows the scratch that a sort of n keys on the digit passes (or the top-16
+// path) needs (grow-only, like ensure_buffers*, lib.rs:1120-1289): ping-pong
+// buffers for keys (and values), and two look-back arrays of tile entries
+// followed by one 32-bit group entry per FS_LB_GROUP tiles.
+static fs_status reserve_digits(fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
     const size_t kb = key_bytes(t);
-    const BucketPath bp = bucket_path(s, op, t, n, false);
-    if (bp == BK_ONE_BLOCK) return FS_OK;
-    const BucketLimit lim = bucket_limit(op, t);
-    const uint64_t sizes[2] = {n < lim.buckets ? n : lim.buckets, n < lim.two_to ? n : lim.two_to};
-    for (uint64_t m : sizes) {
-        const BucketPath mp = bucket_path(s, op, t, m, false);
-        fs_status r = FS_OK;
-        if (m < n && (mp == BK_BUCKETS || mp == BK_TWO_LEVELS)) r = reserve_buckets(s, op, t, m, mp);
-        if (r != FS_OK) return r;
-    }
-    if (bp != BK_NONE) return reserve_buckets(s, op, t, n, bp);
     const uint32_t tile = s->tile[sort_variant(s, op, t, n, false)];
     const uint64_t num_tiles = (n + tile - 1) / tile;
     fs_status r;
@@ -586,6 +574,27 @@ static fs_status reserve(fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
     const size_t lb_bytes = lookback_bytes(s, op, t, n);
     if ((r = ensure(s, s->lb0, lb_bytes)) != FS_OK) return r;
     return ensure(s, s->lb1, lb_bytes);
+}
+
+// Scratch for a sort of n keys and for every smaller one.  Within one path the
+// need grows with n, but not from path to path: smaller sorts may have smaller
+// tiles (more look-back entries), regions of more room than their keys, or
+// paths with tables of their own.  So every size at which the path or the
+// tiles change is reserved for too.
+static fs_status reserve(fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
+    const BucketLimit lim = bucket_limit(op, t);
+    const uint64_t sizes[] = {n, lim.two_to, 1ull << 31, FS_LB_WIDE_KEYS - 1ull, local_mean_max(s, t, true) << 16,
+                              (key64(t) ? FS_TOP16_MIN_KEYS64 : FS_TOP16_MIN_KEYS32) - 1ull, FS_FUSED_MIN_KEYS - 1ull,
+                              lim.two_from ? lim.two_from - 1 : 0u, lim.buckets,
+                              (key64(t) ? FS_SMALL_TILE_KEYS64 : FS_SMALL_TILE_KEYS) - 1ull};
+    for (uint64_t m : sizes) {
+        if (m > n || m <= 1) continue;
+        const BucketPath bp = bucket_path(s, op, t, m, false);
+        if (bp == BK_ONE_BLOCK) continue;
+        const fs_status r = bp == BK_NONE ? reserve_digits(s, op, t, m) : reserve_buckets(s, op, t, m, bp);
+        if (r != FS_OK) return r;
+    }
+    return FS_OK;
 }
 
 // Device addresses of the scratch a sort uses: the sorter's own grow-only
@@ -660,7 +669,7 @@ static uint64_t digit_args(const fs_sorter* s, fs_op op, fs_key_type t, void* ke
 static fs_status enqueue_buckets(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint32_t* vals, uint64_t n,
                                  hipStream_t st, BucketPath bp, bool no_alloc) {
     fs_status r;
-    if (bp != BK_ONE_BLOCK && (r = reserve(s, op, t, n)) != FS_OK) return r;
+    if (bp != BK_ONE_BLOCK && (r = reserve_buckets(s, op, t, n, bp)) != FS_OK) return r;
     const ScratchSet sc = no_alloc ? static_scratch(s) : sorter_scratch(s);
     const bool v = op != FS_OP_SORT, k64 = key64(t);
     FsArgs a;
@@ -790,7 +799,7 @@ static fs_status enqueue(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint
                            (unsigned long long)n, (unsigned)FS_NA_MAX_KEYS);
         if (num_tiles > FS_NA_MAX_TILES)      // every variant's tile is at least FS_NA_MIN_TILE keys
             return set_err(s, FS_ERR_INVALID_ARGUMENT, "tile geometry exceeds the no-allocation scratch layout");
-    } else if ((r = reserve(s, op, t, n)) != FS_OK) {
+    } else if ((r = reserve_digits(s, op, t, n)) != FS_OK) {
         return r;
     }
     const ScratchSet sc = no_alloc ? static_scratch(s) : sorter_scratch(s);

@@ -296,7 +296,10 @@ static int workers() {
     return (w + x - 1) / x * x;
 }
 
+std::atomic<bool> g_skip{false};      // launches do nothing (emu_test_skip_launches)
+
 void launch(const char* name, void (*entry)(void**), uint32_t grid, uint32_t block, void** params) {
+    if (g_skip) return;
     g_kernel = name;
     if (getenv("EMU_TRACE")) fprintf(stderr, "hip_emu: launch %s grid=%u block=%u\n", name, grid, block);
     const int nx = xcds();
@@ -629,5 +632,7 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
 
 // Test helpers the emulator tests call through ctypes (TEST INFRASTRUCTURE).
 extern "C" void* emu_test_stream_create() { hipStream_t s = nullptr; hipStreamCreateWithFlags(&s, 0); return s; }
+// Launches do nothing from now on: tests of the host's scratch sizes, at any n.
+extern "C" void emu_test_skip_launches(int on) { emu::g_skip = on != 0; }
 extern "C" int emu_test_begin_capture(void* s) { return hipStreamBeginCapture((hipStream_t)s, 0); }
 extern "C" int emu_test_end_capture(void* s) { return hipStreamEndCapture((hipStream_t)s, nullptr); }

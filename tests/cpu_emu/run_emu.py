@@ -251,6 +251,49 @@ def check_capture(sorter, kind, n, seed):
     return ok
 
 
+# sizes at which the path or its scratch changes: one block, small tiles, one
+# level of buckets, the fused and top-16 ranges, two levels
+EDGES = [2, 513, 6144, 8192, 190_000, 600_000, 1_000_000, 1 << 20, 1_100_000, 1_500_000, 1 << 21, 12_000_000, 1 << 25,
+         44_040_192, 80_000_000, 140_000_000, 1 << 30, 1 << 31]
+
+
+def check_reserve(kind, most, seed):
+    """fs_reserve(n) holds every smaller sort of its op and type: none captured
+    after it has to grow the scratch.  Launches do nothing here; the values
+    reserved are edges of the paths and numbers drawn up to `most`, the sorts
+    the edges below, one key to either side of them, and drawn numbers."""
+    L = forge_sort._load()
+    L.emu_test_stream_create.restype = ctypes.c_void_p
+    g = np.random.Generator(np.random.PCG64(seed))
+    ok, sorts = True, 0
+    probe = forge_sort.GpuSorter.new()
+    keys = probe.alloc_sort_buffer(kind, most)        # (address space only: nothing touches it)
+    vals = probe.alloc_sort_buffer("u32", most)
+    for op in (forge_sort.OP_SORT, forge_sort.OP_ARGSORT, forge_sort.OP_PAIRS):
+        for n in [*(e for e in EDGES if e <= most), *(int(x) for x in np.exp(g.uniform(np.log(1e4), np.log(most), 6)))]:
+            sorter = forge_sort.GpuSorter.new()
+            stream = L.emu_test_stream_create()
+            L.emu_test_skip_launches(1)
+            sorter.reserve(op, kind, n)
+            L.emu_test_begin_capture(ctypes.c_void_p(stream))
+            for m in {n, *(e + d for e in EDGES for d in (-1, 0, 1) if 2 <= e + d <= n),
+                      *(int(x) for x in np.exp(g.uniform(np.log(2), np.log(n), 20)))}:
+                sorts += 1
+                try:
+                    sorter.encode(op, kind, keys.device_ptr(), vals.device_ptr(), m, stream=stream)
+                except forge_sort.InvalidArgument as e:
+                    print(f"  op {op}: {m:,} after a reserve of {n:,}: {e}", flush=True)
+                    ok = False
+            L.emu_test_end_capture(ctypes.c_void_p(stream))
+            sorter.close()
+            L.emu_test_skip_launches(0)
+    keys.free()
+    vals.free()
+    probe.close()
+    print(f"  {sorts} sorts", flush=True)
+    return ok
+
+
 def check_no_alloc(sorter, kind, n, dist, seed):
     """fs_encode_no_alloc (static scratch) against fs_encode for every op,
     then the same with a smaller input (which finds the first call's contents
@@ -373,9 +416,11 @@ def check(sorter, op, kind, n, dist, seed):
         ok = check_no_alloc(sorter, kind, n, dist, seed)
         print(f"{'PASS' if ok else 'FAIL'} {op} {kind} n={n}", flush=True)
         return ok
-    if op in FAULTS or op in ("hold_timeout", "hold_exact", "capture", "small_s1"):
+    if op in FAULTS or op in ("hold_timeout", "hold_exact", "capture", "small_s1", "reserve"):
         if op == "capture":
             ok = check_capture(sorter, kind, n, seed)
+        elif op == "reserve":
+            ok = check_reserve(kind, n, seed)
         elif op == "small_s1":
             ok = check_small_s1(sorter, kind, keys_for(kind, n, dist, seed))
         elif op.startswith("hold_"):

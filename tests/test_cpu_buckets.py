@@ -72,6 +72,14 @@ def test_emulated_buckets_overflow(emulator):  # noqa: F811
               env={"EMU_WORKERS": "1", "EMU_XCDS": "1"})   # (tiles in order: this build soon gives up a look-back wait)
 
 
+@pytest.mark.parametrize("kind", ["u32", "i32", "f32", "u64", "i64", "f64"])
+def test_reserve_holds_smaller_sorts(emulator, kind):  # noqa: F811
+    """fs_reserve(n), then captured sorts of every smaller size, by the
+    product's limits: paths, tiles and regions change with the size, and none
+    may need more scratch than was reserved."""
+    run_cases("limits", [f"reserve:{kind}:4294967295:uniform:1"], env={"EMU_CUS": "256"})
+
+
 def test_emulated_buckets_sanitizers(emulator):  # noqa: F811
     libasan = subprocess.run(["g++", "-print-file-name=libasan.so"], capture_output=True, text=True).stdout.strip()
     if not os.path.isabs(libasan):

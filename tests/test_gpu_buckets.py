@@ -142,7 +142,9 @@ def test_bucket_path_largest(sorter, kind, op, data):
 
 
 @pytest.mark.parametrize("kind,op,n,reserved", [("u32", "sort", 790_000, 1_000_000), ("u64", "pairs", 380_001, 400_000),
-                                                ("f64", "pairs", 1_200_001, 1_300_000), ("f64", "sort", 1_600_001, 1_700_000)])
+                                                ("f64", "pairs", 1_200_001, 1_300_000), ("f64", "sort", 1_600_001, 1_700_000),
+                                                # (more look-back entries than the reserved sort: smaller tiles)
+                                                ("u32", "sort", 2_000_000, 2_200_000), ("f64", "pairs", 1_040_000, 1_300_000)])
 def test_bucket_path_captured(hip_stream, kind, op, n, reserved):  # noqa: F811
     """Scratch reserved for more keys holds the sort of fewer (a smaller sort's
     regions may be larger); captured into a HIP graph and replayed on data that

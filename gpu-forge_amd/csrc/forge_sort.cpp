@@ -87,6 +87,10 @@ struct fs_sorter {
     int num_cus = 256;
 
     DevBuf s1k, s2k, s1v, s2v, lb0, lb1, iok, iov, tilemap, bk2, rest;
+    // Bucket-path scratch of this many bytes or more could not be had: such
+    // sorts take the digit passes, which need less (0: all of them).
+    // fs_reserve tries anew.
+    size_t buckets_refused = SIZE_MAX;
     uint32_t* hist = nullptr;       // [FS_HIST_SLOTS][8][256], zero between sorts
     uint32_t* binbase = nullptr;    // [8][256]
     uint32_t* cursors = nullptr;    // [FS_REGIONS] region cursors of the fused pass, zero between sorts
@@ -514,10 +518,22 @@ static size_t lookback_bytes(const fs_sorter* s, fs_op op, fs_key_type t, uint64
            (size_t)((num_tiles + FS_LB_GROUP - 1) / FS_LB_GROUP) * FS_RADIX * 4;
 }
 
+// The scratch every path shares.
+static void release_scratch(fs_sorter* s) {
+    DevBuf* bufs[] = {&s->s1k, &s->s2k, &s->s1v, &s->s2v, &s->lb0, &s->lb1, &s->tilemap, &s->bk2, &s->rest};
+    for (DevBuf* b : bufs) free_buf(*b);
+}
+static size_t scratch_bytes(const fs_sorter* s) {
+    return s->s1k.bytes + s->s2k.bytes + s->s1v.bytes + s->s2v.bytes + s->lb0.bytes + s->lb1.bytes + s->tilemap.bytes +
+           s->bk2.bytes + s->rest.bytes;
+}
+
 // Scratch of the bucket path for sorts of up to n keys.  Larger sorts may need
 // less (more samples bound the regions closer), so the sizes here bound every
 // n: regions by the fewest samples a bucket (4) and a child (16) can have, the
-// look-back of one level by a tile per CU.
+// look-back of one level by a tile per CU.  FS_ERR_OUT_OF_MEMORY (all scratch
+// then released) and FS_ERR_INVALID_ARGUMENT (growth refused after a capture)
+// leave the sort to the digit passes.
 static fs_status reserve_buckets(fs_sorter* s, fs_op op, fs_key_type t, uint64_t n, BucketPath bp) {
     const bool two = bp == BK_TWO_LEVELS;
     const size_t kb = key_bytes(t);
@@ -525,33 +541,46 @@ static fs_status reserve_buckets(fs_sorter* s, fs_op op, fs_key_type t, uint64_t
     const double nb = (double)(1u << b.lnb);
     uint64_t s1 = b.s1_keys, s2 = n;
     uint64_t tiles = b.tiles > (uint32_t)s->num_cus + 2u ? b.tiles : (uint32_t)s->num_cus + 2u;
-    uint64_t lb = ((tiles + tiles / FS_LB_GROUP + 1) << b.lnb) * 4, rests = 0;
-    fs_status r;
+    uint64_t lb = ((tiles + tiles / FS_LB_GROUP + 1) << b.lnb) * 4, digit_lb = 0;
     if (two) {
         const double nb2 = (double)(1u << b.lnb2);
         const uint64_t all = (uint64_t)((double)n * (bucket_room(1.0, 16.0) + 0.02) + nb * (32.0 * nb2 + 96.0));
         s2 = b.s2_keys > all ? b.s2_keys : all;
         // (a bucket's groups of the second level start anew: one more for each)
         const uint64_t lb2 = (((uint64_t)b.tiles2 + b.tiles2 / FS_LB_GROUP + (1u << b.lnb) + 1) << b.lnb2) * 4;
-        const uint64_t digit_lb = lookback_bytes(s, op, t, n);    // or the digit passes
+        digit_lb = lookback_bytes(s, op, t, n);                   // or the digit passes
         if (lb2 > lb) lb = lb2;
         if (digit_lb > lb) lb = digit_lb;
-        rests = b.rests;
-        if ((r = ensure(s, s->tilemap, (size_t)b.tiles2 * 4)) != FS_OK) return r;
-        if ((r = ensure(s, s->bk2, (size_t)FS_BK2_TAB_WORDS * 4)) != FS_OK) return r;
-        if ((r = ensure(s, s->rest, (size_t)rests * 8)) != FS_OK) return r;
-        if ((r = ensure(s, s->lb1, (size_t)digit_lb)) != FS_OK) return r;
     } else {
         const uint64_t all = (uint64_t)((double)n * bucket_room(1.0, 4.0) + 32.0 * nb);
         if (all > s1) s1 = all;
+        if (op == FS_OP_SORT) lb = 0;
     }
-    if ((r = ensure(s, s->s1k, s1 * kb)) != FS_OK) return r;
-    if ((r = ensure(s, s->s2k, s2 * kb)) != FS_OK) return r;
-    if (two || op != FS_OP_SORT)
-        if ((r = ensure(s, s->lb0, (size_t)lb)) != FS_OK) return r;
-    if (op == FS_OP_SORT) return FS_OK;
-    if ((r = ensure(s, s->s1v, s1 * 4)) != FS_OK) return r;
-    return ensure(s, s->s2v, s2 * 4);
+    const bool v = op != FS_OP_SORT;
+    const struct {
+        DevBuf& buf;
+        size_t bytes;
+    } needs[] = {{s->s1k, s1 * kb},
+                 {s->s2k, s2 * kb},
+                 {s->s1v, v ? s1 * 4 : 0},
+                 {s->s2v, v ? s2 * 4 : 0},
+                 {s->lb0, lb},
+                 {s->lb1, digit_lb},
+                 {s->tilemap, two ? (size_t)b.tiles2 * 4 : 0},
+                 {s->bk2, two ? (size_t)FS_BK2_TAB_WORDS * 4 : 0},
+                 {s->rest, two ? (size_t)b.rests * 8 : 0}};
+    size_t total = 0;
+    for (const auto& need : needs) total += need.bytes;
+    if (total >= s->buckets_refused) return FS_ERR_OUT_OF_MEMORY;
+    for (const auto& need : needs) {
+        const fs_status r = ensure(s, need.buf, need.bytes);
+        if (r == FS_ERR_OUT_OF_MEMORY) {
+            s->buckets_refused = total;
+            release_scratch(s);                          // (the digit passes may need it)
+        }
+        if (r != FS_OK) return r;
+    }
+    return FS_OK;
 }
 
 // Grows the scratch that a sort of n keys on the digit passes (or the top-16
@@ -581,20 +610,39 @@ static fs_status reserve_digits(fs_sorter* s, fs_op op, fs_key_type t, uint64_t 
 // tiles (more look-back entries), regions of more room than their keys, or
 // paths with tables of their own.  So every size at which the path or the
 // tiles change is reserved for too.
+// A path that finds no memory gives way to the digit passes at every size
+// before the reserve fails.
 static fs_status reserve(fs_sorter* s, fs_op op, fs_key_type t, uint64_t n) {
     const BucketLimit lim = bucket_limit(op, t);
     const uint64_t sizes[] = {n, lim.two_to, 1ull << 31, FS_LB_WIDE_KEYS - 1ull, local_mean_max(s, t, true) << 16,
                               (key64(t) ? FS_TOP16_MIN_KEYS64 : FS_TOP16_MIN_KEYS32) - 1ull, FS_FUSED_MIN_KEYS - 1ull,
                               lim.two_from ? lim.two_from - 1 : 0u, lim.buckets,
                               (key64(t) ? FS_SMALL_TILE_KEYS64 : FS_SMALL_TILE_KEYS) - 1ull};
-    for (uint64_t m : sizes) {
-        if (m > n || m <= 1) continue;
-        const BucketPath bp = bucket_path(s, op, t, m, false);
-        if (bp == BK_ONE_BLOCK) continue;
-        const fs_status r = bp == BK_NONE ? reserve_digits(s, op, t, m) : reserve_buckets(s, op, t, m, bp);
-        if (r != FS_OK) return r;
+    s->buckets_refused = SIZE_MAX;
+    for (;;) {
+        const size_t refused = s->buckets_refused;
+        fs_status r = FS_OK;
+        for (uint64_t m : sizes) {
+            if (m > n || m <= 1) continue;
+            const BucketPath bp = bucket_path(s, op, t, m, false);
+            if (bp == BK_ONE_BLOCK) continue;
+            if (bp != BK_NONE) {
+                r = reserve_buckets(s, op, t, m, bp);
+                if (s->buckets_refused != refused) break;            // (what was reserved so far is gone)
+            }
+            if (bp == BK_NONE || r == FS_ERR_OUT_OF_MEMORY) r = reserve_digits(s, op, t, m);
+            if (r != FS_OK) break;
+        }
+        if (r != FS_ERR_OUT_OF_MEMORY) return r;
+        if (refused == 0) {
+            s->buckets_refused = SIZE_MAX;               // (smaller sorts may fit)
+            return r;
+        }
+        if (s->buckets_refused == refused) {             // the digit passes' scratch: without any buckets', then
+            s->buckets_refused = 0;
+            release_scratch(s);
+        }
     }
-    return FS_OK;
 }
 
 // Device addresses of the scratch a sort uses: the sorter's own grow-only
@@ -665,11 +713,10 @@ static uint64_t digit_args(const fs_sorter* s, fs_op op, fs_key_type t, void* ke
     return up_blocks;
 }
 
-// The launches of the bucket path.
+// The launches of the bucket path, its scratch reserved.
 static fs_status enqueue_buckets(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint32_t* vals, uint64_t n,
                                  hipStream_t st, BucketPath bp, bool no_alloc) {
     fs_status r;
-    if (bp != BK_ONE_BLOCK && (r = reserve_buckets(s, op, t, n, bp)) != FS_OK) return r;
     const ScratchSet sc = no_alloc ? static_scratch(s) : sorter_scratch(s);
     const bool v = op != FS_OP_SORT, k64 = key64(t);
     FsArgs a;
@@ -784,14 +831,24 @@ static fs_status enqueue(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint
     const size_t kb = key_bytes(t);
     if ((uintptr_t)keys % kb != 0 || (vals && (uintptr_t)vals % 4 != 0))
         return set_err(s, FS_ERR_INVALID_ARGUMENT, "misaligned key or value pointer");
-    const BucketPath bp = bucket_path(s, op, t, n, no_alloc);
+    fs_status r;
+    BucketPath bp = bucket_path(s, op, t, n, no_alloc);
+    if (bp == BK_BUCKETS || bp == BK_TWO_LEVELS) {
+        const std::string err = s->err;
+        r = reserve_buckets(s, op, t, n, bp);
+        if (r == FS_ERR_OUT_OF_MEMORY || r == FS_ERR_INVALID_ARGUMENT) {
+            s->err = err;
+            bp = BK_NONE;
+        } else if (r != FS_OK) {
+            return r;
+        }
+    }
     if (bp != BK_NONE) return enqueue_buckets(s, op, t, keys, vals, n, st, bp, no_alloc);
     const int var = sort_variant(s, op, t, n, no_alloc);
     const uint32_t tile = s->tile[var];
     const uint32_t num_tiles = (uint32_t)((n + tile - 1) / tile);
     // the static scratch holds narrow look-back entries (n < 2^30 there)
     const bool wide = !no_alloc && wide_lookback(s, n);
-    fs_status r;
     if (no_alloc) {
         if (n > FS_NA_MAX_KEYS)
             return set_err(s, FS_ERR_INVALID_ARGUMENT,
@@ -799,8 +856,15 @@ static fs_status enqueue(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint
                            (unsigned long long)n, (unsigned)FS_NA_MAX_KEYS);
         if (num_tiles > FS_NA_MAX_TILES)      // every variant's tile is at least FS_NA_MIN_TILE keys
             return set_err(s, FS_ERR_INVALID_ARGUMENT, "tile geometry exceeds the no-allocation scratch layout");
-    } else if ((r = reserve_digits(s, op, t, n)) != FS_OK) {
-        return r;
+    } else {
+        r = reserve_digits(s, op, t, n);
+        const size_t held = scratch_bytes(s);
+        if (r == FS_ERR_OUT_OF_MEMORY && held) {         // (never after a capture) without what other paths hold, then
+            if (held < s->buckets_refused) s->buckets_refused = held;
+            release_scratch(s);
+            r = reserve_digits(s, op, t, n);
+        }
+        if (r != FS_OK) return r;
     }
     const ScratchSet sc = no_alloc ? static_scratch(s) : sorter_scratch(s);
     // the fused first pass, when its regions fit the scratch (the static

@@ -515,8 +515,12 @@ struct SegvInstaller {
 } g_segv;
 }  // namespace
 
+// Device memory (emu_test_memory_limit) and the calls that allocated some.
+static std::atomic<size_t> g_limit{~(size_t)0}, g_live{0}, g_mallocs{0};
+
 hipError_t hipMalloc(void** p, size_t n) {
     const size_t body = (n + kPage - 1) / kPage * kPage;
+    if (g_live + body > g_limit) return hipErrorOutOfMemory;
     const size_t len = body + 2 * kPage;
     char* m = (char*)mmap(nullptr, len, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
     if (m == MAP_FAILED) return hipErrorOutOfMemory;
@@ -526,6 +530,8 @@ hipError_t hipMalloc(void** p, size_t n) {
     char* user = m + kPage + body - n16;       // ends on the trailing guard page (16-byte aligned)
     std::lock_guard<std::mutex> g(g_mu);
     g_allocs[user] = {m, len};
+    g_live += body;
+    ++g_mallocs;
     *p = user;
     return hipSuccess;
 }
@@ -537,6 +543,7 @@ hipError_t hipFree(void* p) {
     std::lock_guard<std::mutex> g(g_mu);
     auto it = g_allocs.find(p);
     if (it == g_allocs.end()) return hipErrorInvalidValue;
+    g_live -= it->second.second - 2 * kPage;
     munmap(it->second.first, it->second.second);
     g_allocs.erase(it);
     return hipSuccess;
@@ -633,6 +640,11 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
 // Test helpers the emulator tests call through ctypes (TEST INFRASTRUCTURE).
 extern "C" void* emu_test_stream_create() { hipStream_t s = nullptr; hipStreamCreateWithFlags(&s, 0); return s; }
 // Launches do nothing from now on: tests of the host's scratch sizes, at any n.
+// hipMalloc fails where more than `bytes` of device memory would be in use; the
+// bytes in use; the allocations made so far.
+extern "C" void emu_test_memory_limit(size_t bytes) { g_limit = bytes; }
+extern "C" size_t emu_test_memory_used() { return g_live; }
+extern "C" size_t emu_test_mallocs() { return g_mallocs; }
 extern "C" void emu_test_skip_launches(int on) { emu::g_skip = on != 0; }
 extern "C" int emu_test_begin_capture(void* s) { return hipStreamBeginCapture((hipStream_t)s, 0); }
 extern "C" int emu_test_end_capture(void* s) { return hipStreamEndCapture((hipStream_t)s, nullptr); }

@@ -294,6 +294,107 @@ def check_reserve(kind, most, seed):
     return ok
 
 
+def check_memory(kind, n, seed):
+    """Where the bucket path's scratch does not fit, the digit passes sort: on
+    first use (once refused, without asking again), after a reserve and
+    captured, and after other sorts' bucket scratch left too little.
+    fs_reserve with room again brings the bucket path back."""
+    L = forge_sort._load()
+    L.emu_test_stream_create.restype = ctypes.c_void_p
+    L.emu_test_memory_used.restype = L.emu_test_mallocs.restype = ctypes.c_size_t
+
+    def limit(b):
+        L.emu_test_memory_limit(ctypes.c_size_t(b))
+
+    everything = (1 << 64) - 1
+    probe = forge_sort.GpuSorter.new()
+    keys, vals = probe.alloc_sort_buffer(kind, 4 * n), probe.alloc_sort_buffer("u32", 4 * n)
+    ok = True
+    for op in (forge_sort.OP_SORT, forge_sort.OP_ARGSORT, forge_sort.OP_PAIRS):
+
+        def new(skip=True):
+            s = forge_sort.GpuSorter.new()
+            s.set_profiling(True)
+            L.emu_test_skip_launches(int(skip))
+            return s
+
+        def sort(s, m, stream=None):
+            s.profile_reset()
+            s.encode(op, kind, keys.device_ptr(), vals.device_ptr(), m, stream=stream)
+            return "buckets" if any("fs_split" in k for k, _ in s.profile()) else "digits"
+
+        def done(s):
+            s.close()
+            limit(everything)
+            L.emu_test_skip_launches(0)
+
+        def expect(what, got, want):
+            nonlocal ok
+            if got != want:
+                print(f"  op {op}, {what}: {got}, expected {want}", flush=True)
+                ok = False
+
+        s = new()
+        s.set_test_option(forge_sort.TEST_BUCKETS, forge_sort.BUCKETS_NEVER)
+        before = L.emu_test_memory_used()
+        sort(s, n)
+        need = L.emu_test_memory_used() - before
+        done(s)
+
+        s = new()
+        limit(L.emu_test_memory_used() + need)
+        expect("no room", sort(s, n), "digits")
+        calls = L.emu_test_mallocs()
+        expect("no room, again", sort(s, n), "digits")
+        expect("allocations", L.emu_test_mallocs(), calls)
+        limit(everything)
+        s.reserve(op, kind, n)
+        expect("room again", sort(s, n), "buckets")
+        done(s)
+
+        s = new()
+        limit(L.emu_test_memory_used() + need + (1 << 20))
+        s.reserve(op, kind, n)
+        stream = L.emu_test_stream_create()
+        L.emu_test_begin_capture(ctypes.c_void_p(stream))
+        expect("reserved, captured", sort(s, n, stream), "digits")
+        L.emu_test_end_capture(ctypes.c_void_p(stream))
+        done(s)
+
+        # a larger sort on the digit passes, with room for its scratch alone
+        s = new()
+        s.set_test_option(forge_sort.TEST_BUCKETS, forge_sort.BUCKETS_NEVER)
+        before = L.emu_test_memory_used()
+        sort(s, 4 * n)
+        need4 = L.emu_test_memory_used() - before
+        done(s)
+        s = new()
+        before = L.emu_test_memory_used()
+        expect("with room", sort(s, n), "buckets")
+        s.set_test_option(forge_sort.TEST_BUCKETS, forge_sort.BUCKETS_NEVER)
+        limit(before + need4)
+        expect("after the buckets", sort(s, 4 * n), "digits")
+        done(s)
+
+    # and exact
+    L.emu_test_skip_launches(0)
+    s = forge_sort.GpuSorter.new()
+    small = keys_for(kind, n // 10, "uniform", seed)
+    sorted_ok(s, kind, small[:2])                      # (the slice API's staging)
+    limit(L.emu_test_memory_used() + 8 * small.nbytes // 2)
+    ok &= sorted_ok(s, kind, small)
+    path, _ = s.last_bucket_info()
+    limit(everything)
+    if path != forge_sort.PATH_DIGITS:
+        print(f"  path {path} without room", flush=True)
+        ok = False
+    s.close()
+    keys.free()
+    vals.free()
+    probe.close()
+    return ok
+
+
 def check_no_alloc(sorter, kind, n, dist, seed):
     """fs_encode_no_alloc (static scratch) against fs_encode for every op,
     then the same with a smaller input (which finds the first call's contents
@@ -416,11 +517,13 @@ def check(sorter, op, kind, n, dist, seed):
         ok = check_no_alloc(sorter, kind, n, dist, seed)
         print(f"{'PASS' if ok else 'FAIL'} {op} {kind} n={n}", flush=True)
         return ok
-    if op in FAULTS or op in ("hold_timeout", "hold_exact", "capture", "small_s1", "reserve"):
+    if op in FAULTS or op in ("hold_timeout", "hold_exact", "capture", "small_s1", "reserve", "memory"):
         if op == "capture":
             ok = check_capture(sorter, kind, n, seed)
         elif op == "reserve":
             ok = check_reserve(kind, n, seed)
+        elif op == "memory":
+            ok = check_memory(kind, n, seed)
         elif op == "small_s1":
             ok = check_small_s1(sorter, kind, keys_for(kind, n, dist, seed))
         elif op.startswith("hold_"):

@@ -80,6 +80,14 @@ def test_reserve_holds_smaller_sorts(emulator, kind):  # noqa: F811
     run_cases("limits", [f"reserve:{kind}:4294967295:uniform:1"], env={"EMU_CUS": "256"})
 
 
+def test_buckets_without_memory(emulator):  # noqa: F811
+    """The bucket path needs more scratch than the digit passes: where that
+    much cannot be had they sort instead, by the product's limits (one level
+    for u32 and i64, two for f64)."""
+    run_cases("limits", ["memory:u32:590000:uniform:1", "memory:i64:990000:uniform:2", "memory:f64:1600000:uniform:3"],
+              env={"EMU_CUS": "256"}, parallel=3)
+
+
 def test_emulated_buckets_sanitizers(emulator):  # noqa: F811
     libasan = subprocess.run(["g++", "-print-file-name=libasan.so"], capture_output=True, text=True).stdout.strip()
     if not os.path.isabs(libasan):

@@ -45,7 +45,7 @@ const char* const kKernelNames[] = {
     "fs_local_k32", "fs_rescatter_k32", "fs_rescatter_k64", "fs_local_k64",
     "fs_local_deferred_k64", "fs_onesweep_loop_k64", "fs_local_deferred_k32", "fs_local_k32_w",
     "fs_local_deferred_k32_w", "fs_local_k64_w", "fs_local_deferred_k64_w", "fs_onesweep_k32_s",
-    "fs_onesweep_any_k32_s", "fs_onesweep_k32_vs", "fs_onesweep_k64_s", "fs_onesweep_any_k64_s", "fs_onesweep_k64_vs",
+    "fs_onesweep_any_k32_s", "fs_onesweep_k32_vs", "fs_onesweep_k64_vs",
     "fs_split_k32", "fs_split_k64", "fs_part_k32", "fs_part_k32_v", "fs_part_k64", "fs_part_k64_v", "fs_bucket_k32",
     "fs_bucket_k32_v", "fs_bucket_k64", "fs_bucket_k64_v", "fs_split2_k64", "fs_part1_k64", "fs_part1_k64_v",
     "fs_part2_k64", "fs_part2_k64_v", "fs_child_k64", "fs_child_k64_v", "fs_rest_k64", "fs_rest_k64_v",
@@ -54,14 +54,14 @@ const char* const kKernelNames[] = {
 enum {
     K_UP32, K_UP64, K_OS32, K_OS32V, K_OS64, K_OS64V, K_IOTA, K_ANY32, K_ANY64, K_SCRATCH_ADDR, K_FIRST32, K_FIRST64,
     K_SAMPLE32, K_SAMPLE64, K_LOCAL32, K_RESCATTER32, K_RESCATTER64, K_LOCAL64, K_DEFER64, K_LOOP64, K_DEFER32,
-    K_LOCAL32W, K_DEFER32W, K_LOCAL64W, K_DEFER64W, K_OS32S, K_ANY32S, K_OS32VS, K_OS64S, K_ANY64S, K_OS64VS,
+    K_LOCAL32W, K_DEFER32W, K_LOCAL64W, K_DEFER64W, K_OS32S, K_ANY32S, K_OS32VS, K_OS64VS,
     K_SPLIT32, K_SPLIT64, K_PART32, K_PART32V, K_PART64, K_PART64V, K_BUCKET32, K_BUCKET32V, K_BUCKET64, K_BUCKET64V,
     K_SPLIT2, K_PART1, K_PART1V, K_PART2, K_PART2V, K_CHILD, K_CHILDV, K_REST, K_RESTV, K_UP64C,
     K_COUNT
 };
 // the stable digit-pass kernel and the keys-only first-pass kernel of each variant (FS_VAR_*)
-const int kPassKernel[FS_VARIANTS] = {K_OS32, K_OS32V, K_OS64, K_OS64V, K_OS32S, K_OS32VS, K_OS64S, K_OS64VS};
-const int kAnyKernel[FS_VARIANTS] = {K_ANY32, -1, K_ANY64, -1, K_ANY32S, -1, K_ANY64S, -1};
+const int kPassKernel[FS_VARIANTS] = {K_OS32, K_OS32V, K_OS64, K_OS64V, K_OS32S, K_OS32VS, K_OS64VS};
+const int kAnyKernel[FS_VARIANTS] = {K_ANY32, -1, K_ANY64, -1, K_ANY32S, -1, -1};
 
 }  // namespace
 
@@ -482,14 +482,15 @@ static BucketShape bucket_shape(const fs_sorter* s, fs_op op, fs_key_type t, uin
 }
 
 // The digit-pass variant a sort runs: by key width and op, and its small
-// tiles (FS_VAR_K32S ... FS_VAR_K64VS) below FS_SMALL_TILE_KEYS (32-bit keys)
-// or FS_SMALL_TILE_KEYS64 (64-bit keys) keys on the LSD passes (the fused and
-// top-16 sequences and the static scratch keep the larger tiles).
+// tiles (FS_VAR_K32S, FS_VAR_K32VS, FS_VAR_K64VS) below FS_SMALL_TILE_KEYS
+// (32-bit keys) or FS_SMALL_TILE_KEYS64 (64-bit keys with values) keys on the
+// LSD passes (the fused and top-16 sequences and the static scratch keep the
+// larger tiles).
 static int sort_variant(const fs_sorter* s, fs_op op, fs_key_type t, uint64_t n, bool no_alloc) {
     const int v = variant_of(op, t);
-    if (no_alloc || n >= (key64(t) ? FS_SMALL_TILE_KEYS64 : FS_SMALL_TILE_KEYS)) return v;
+    if (no_alloc || v == FS_VAR_K64 || n >= (key64(t) ? FS_SMALL_TILE_KEYS64 : FS_SMALL_TILE_KEYS)) return v;
     if (op == FS_OP_SORT && (fused_path(s, op, t, n) || top16_path(s, op, t, n))) return v;
-    return v + (FS_VAR_K32S - FS_VAR_K32);    // the small variant of each (FS_VAR_* order)
+    return v == FS_VAR_K32 ? FS_VAR_K32S : v == FS_VAR_K32V ? FS_VAR_K32VS : FS_VAR_K64VS;
 }
 
 // The top-16 path's local sort runs on wide blocks (twice the keys) where

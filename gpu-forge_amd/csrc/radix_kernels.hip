@@ -3084,7 +3084,7 @@ extern "C" __global__ void __launch_bounds__(FS_K32_BLOCK) FS_OCC(FS_K32_WAVES_P
 extern "C" __global__ void __launch_bounds__(FS_K64_BLOCK) FS_OCC(FS_K64_WAVES_PER_EU) fs_onesweep_any_k64(FsArgs a, uint32_t slot) {
     onesweep_body<true, false, FS_K64_BLOCK, FS_K64_ITEMS, true>(a, slot, blockIdx.x);
 }
-// The small tiles of small sorts (FS_VAR_K32S ... FS_VAR_K64VS): the stable
+// The small tiles of small sorts (FS_VAR_K32S, FS_VAR_K32VS, FS_VAR_K64VS): the stable
 // passes, and for keys-only sorts digit 0's pass in any order.
 #ifndef FS_KS_WAVES_PER_EU
 #define FS_KS_WAVES_PER_EU 6
@@ -3097,12 +3097,6 @@ extern "C" __global__ void __launch_bounds__(FS_K32S_BLOCK) FS_OCC(FS_KS_WAVES_P
 }
 extern "C" __global__ void __launch_bounds__(FS_KS_BLOCK) FS_OCC(FS_KS_WAVES_PER_EU) fs_onesweep_k32_vs(FsArgs a, uint32_t slot) {
     onesweep_body<false, true, FS_KS_BLOCK, FS_K32VS_ITEMS>(a, slot, blockIdx.x);
-}
-extern "C" __global__ void __launch_bounds__(FS_KS_BLOCK) FS_OCC(FS_KS_WAVES_PER_EU) fs_onesweep_k64_s(FsArgs a, uint32_t slot) {
-    onesweep_body<true, false, FS_KS_BLOCK, FS_K64S_ITEMS>(a, slot, blockIdx.x);
-}
-extern "C" __global__ void __launch_bounds__(FS_KS_BLOCK) FS_OCC(FS_KS_WAVES_PER_EU) fs_onesweep_any_k64_s(FsArgs a, uint32_t slot) {
-    onesweep_body<true, false, FS_KS_BLOCK, FS_K64S_ITEMS, true>(a, slot, blockIdx.x);
 }
 extern "C" __global__ void __launch_bounds__(FS_KS_BLOCK) FS_OCC(FS_KS_WAVES_PER_EU) fs_onesweep_k64_vs(FsArgs a, uint32_t slot) {
     onesweep_body<true, true, FS_KS_BLOCK, FS_K64VS_ITEMS>(a, slot, blockIdx.x);
@@ -3228,7 +3222,7 @@ extern "C" __global__ void __launch_bounds__(FS_K64_BLOCK) FS_OCC(FS_K64_BLOCK /
 extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_tile_keys[FS_VARIANTS] = {
     FS_K32_BLOCK * FS_K32_ITEMS, FS_K32V_BLOCK * FS_K32V_ITEMS,
     FS_K64_BLOCK * FS_K64_ITEMS, FS_K64V_BLOCK * FS_K64V_ITEMS, FS_K32S_BLOCK * FS_K32S_ITEMS,
-    FS_KS_BLOCK * FS_K32VS_ITEMS, FS_KS_BLOCK * FS_K64S_ITEMS, FS_KS_BLOCK * FS_K64VS_ITEMS};
+    FS_KS_BLOCK * FS_K32VS_ITEMS, FS_KS_BLOCK * FS_K64VS_ITEMS};
 // Keys a block of the local sort holds, and its threads per block (32-bit
 // keys, then 64-bit keys); then the fewest segment bits whose 32-bit
 // segments the first launch sorts itself; then the same two pairs for the
@@ -3248,7 +3242,7 @@ extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_bucket_geometry
     FS_BC_BLOCK * FS_BC64_ITEMS, FS_BC_BLOCK * FS_BC64V_ITEMS, FS_BP_BLOCK * FS_BP2_64_ITEMS, FS_BP_BLOCK * FS_BP2_64V_ITEMS};
 // Threads per block of the same variants.
 extern "C" __constant__ __attribute__((used)) uint32_t fs_kernel_block_threads[FS_VARIANTS] = {
-    FS_K32_BLOCK, FS_K32V_BLOCK, FS_K64_BLOCK, FS_K64V_BLOCK, FS_K32S_BLOCK, FS_KS_BLOCK, FS_KS_BLOCK, FS_KS_BLOCK};
+    FS_K32_BLOCK, FS_K32V_BLOCK, FS_K64_BLOCK, FS_K64V_BLOCK, FS_K32S_BLOCK, FS_KS_BLOCK, FS_KS_BLOCK};
 
 // ---------------------------------------------------------------------------
 // fs_gather_elems: output[i] = source[indices[i]] for 4- or 8-byte elements

@@ -480,15 +480,17 @@ def check_first_pass(sorter, op, kind, n, dist, seed):
 
 def check(sorter, op, kind, n, dist, seed):
     # one_<op>: one block sorts everything; bk_<op>, bk<b>_<op>: the bucket
-    # path (2^b buckets), two_<op>: two levels of them; bkover_<op>, twoover_<op>,
+    # path (2^b buckets), two_<op>: two levels of them; size<p>_<op>: by size,
+    # which must be path p (fs_last_bucket_info); bkover_<op>, twoover_<op>,
     # twosecond_<op>: with a region (of the second level) that overflows (fault build)
-    bucket = re.fullmatch(r"(one|bk|bkover|two|twoover|twosecond)(\d*)_(sort|argsort|pairs|offset)", op)
+    bucket = re.fullmatch(r"(one|bk|bkover|two|twoover|twosecond|size)(\d*)_(sort|argsort|pairs|offset)", op)
     if bucket:
         one, b, rest = bucket.groups()
         sorter.set_test_option(forge_sort.TEST_BUCKETS,
-                               forge_sort.BUCKETS_ONE_BLOCK if one == "one"
+                               forge_sort.BUCKETS_BY_SIZE if one == "size"
+                               else forge_sort.BUCKETS_ONE_BLOCK if one == "one"
                                else (forge_sort.BUCKETS_TWO_LEVELS if one.startswith("two")
-                                     else forge_sort.BUCKETS_ALWAYS) + (int(b or 0) << 8))
+                                     else forge_sort.BUCKETS_ALWAYS) + (int(b or 0) << 8 if one != "size" else 0))
         fault = {"bkover": forge_sort.FAULT_SMALL_REGIONS, "twoover": forge_sort.FAULT_SMALL_REGIONS,
                  "twosecond": forge_sort.FAULT_SMALL_REGIONS2}.get(one)
         if fault:
@@ -496,8 +498,8 @@ def check(sorter, op, kind, n, dist, seed):
         try:
             ok = check(sorter, rest, kind, n, dist, seed)
             path, overflows = sorter.last_bucket_info()
-            want = {"one": forge_sort.PATH_ONE_BLOCK, "bk": forge_sort.PATH_BUCKETS, "bkover": forge_sort.PATH_BUCKETS}.get(
-                one, forge_sort.PATH_TWO_LEVELS)
+            want = int(b) if one == "size" else {"one": forge_sort.PATH_ONE_BLOCK, "bk": forge_sort.PATH_BUCKETS,
+                                                 "bkover": forge_sort.PATH_BUCKETS}.get(one, forge_sort.PATH_TWO_LEVELS)
             # (two levels: keys of few varying digits go to the digit passes)
             if path != want and not (want == forge_sort.PATH_TWO_LEVELS and path == forge_sort.PATH_DIGITS and not fault):
                 print(f"  path {path}, expected {want}", flush=True)

@@ -72,6 +72,15 @@ def test_emulated_buckets_overflow(emulator):  # noqa: F811
               env={"EMU_WORKERS": "1", "EMU_XCDS": "1"})   # (tiles in order: this build soon gives up a look-back wait)
 
 
+def test_emulated_paths_by_size(emulator):  # noqa: F811
+    """The product's limits: one block, one level of buckets, two (k / 255, whose
+    regions must hold), the digit passes beyond; capture and the static scratch."""
+    run_cases("limits", ["size1_sort:u32:8192:uniform:1", "size2_sort:u32:8193:few:2", "size1_pairs:i64:6144:few:3",
+                         "size2_argsort:f64:6145:uniform:4", "size2_pairs:f32:20001:uniform:5", "size0_sort:f32:190001:uniform:6",
+                         "size3_sort:f64:1600000:steps256:1", "capture:u32:20000:uniform:7", "capture:f64:20000:uniform:8",
+                         "noalloc:i32:9000:few:9", "noalloc:u64:6000:uniform:10"], parallel=4, env={"EMU_CUS": "8"})
+
+
 @pytest.mark.parametrize("kind", ["u32", "i32", "f32", "u64", "i64", "f64"])
 def test_reserve_holds_smaller_sorts(emulator, kind):  # noqa: F811
     """fs_reserve(n), then captured sorts of every smaller size, by the

@@ -130,6 +130,25 @@ def test_two_levels_by_size(sorter, kind, op, n, data):
     check(sorter, op, kind, keys_of(kind, n, data, seed=7300))
 
 
+@pytest.mark.parametrize("kind,op,n,values,lnb", [
+    ("f64", "sort", 1_600_000, 256, 0), ("f64", "argsort", 4_000_000, 190, 0), ("u64", "pairs", 12_000_000, 192, 0),
+    ("u32", "sort", 1_000_000, 400, 0), ("i64", "pairs", 900_001, 300, 0),
+    ("f64", "sort", 850_000, 384, 1), ("u64", "argsort", 850_000, 384, 1)])      # (two buckets of 192 values each)
+def test_repeated_values(sorter, kind, op, n, values, lnb):
+    """Evenly spaced values, every one in a group of the sample's own, so that
+    a bucket between two splitters can hold two: exact, and no region too small."""
+    from forge_sort import BUCKETS_BY_SIZE, BUCKETS_TWO_LEVELS, PATH_BUCKETS, PATH_TWO_LEVELS, TEST_BUCKETS
+    sorter.set_test_option(TEST_BUCKETS, BUCKETS_TWO_LEVELS + (lnb << 8) if lnb else BUCKETS_BY_SIZE)
+    try:
+        for seed in (1, 2, 3):
+            k = np.random.Generator(np.random.PCG64(seed)).integers(0, values, size=n, dtype=BITS[kind])
+            keys = k / (values - 1) if kind == "f64" else (k * (~BITS[kind](0) // BITS[kind](values))).view(NP[kind])
+            check(sorter, op, kind, keys)
+            assert sorter.last_bucket_info() == (PATH_TWO_LEVELS if lnb or n > 1_500_000 else PATH_BUCKETS, 0)
+    finally:
+        sorter.set_test_option(TEST_BUCKETS, BUCKETS_BY_SIZE)
+
+
 @pytest.mark.parametrize("kind,op", [("u32", "sort"), ("i32", "pairs"), ("f32", "argsort"), ("i64", "sort"),
                                      ("f64", "pairs")])
 @pytest.mark.parametrize("data", ["normal", "quantised", "specials", "clusters", "runs"])

@@ -33,6 +33,20 @@ def sorter():
     s.close()
 
 
+@pytest.fixture(params=["by size", "digit passes"])
+def either_path(sorter, request):
+    """The path that the size takes (buckets for small sorts), and the digit
+    passes, which take the same sizes where the bucket path's scratch does not
+    fit: at their own tiles' edges and on their own schedules."""
+    from forge_sort import BUCKETS_BY_SIZE, BUCKETS_NEVER, PATH_DIGITS, TEST_BUCKETS
+    digits = request.param == "digit passes"
+    sorter.set_test_option(TEST_BUCKETS, BUCKETS_NEVER if digits else BUCKETS_BY_SIZE)
+    yield
+    path, _ = sorter.last_bucket_info()
+    sorter.set_test_option(TEST_BUCKETS, BUCKETS_BY_SIZE)
+    assert not digits or path == PATH_DIGITS
+
+
 def bits_equal(a, b, kind):
     return np.array_equal(np.asarray(a).view(BITS[kind]), np.asarray(b).view(BITS[kind]))
 
@@ -168,6 +182,7 @@ SIZES = [2, 3, 100, 255, 4095, 4096, 4097, 65543, 1_000_000]
 
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("n", SIZES)
+@pytest.mark.usefixtures("either_path")
 def test_sort_sizes(sorter, kind, n):
     check_sort(sorter, kind, make_keys(kind, n, "uniform", seed=n))
 
@@ -175,6 +190,7 @@ def test_sort_sizes(sorter, kind, n):
 @pytest.mark.parametrize("kind", ["u32", "i32", "f32"])
 @pytest.mark.parametrize("n,dist", [((1 << 21) - 1, "uniform"), (1 << 21, "uniform"), ((1 << 21) - 1, "few"),
                                     (1_500_001, "byte1"), (6_144 * 7 + 5, "uniform")])
+@pytest.mark.usefixtures("either_path")
 def test_small_tile_boundary(sorter, kind, n, dist):
     """Keys-only 32-bit sorts take the digit pass's small tiles below 2^21
     keys (FS_SMALL_TILE_KEYS) and the stable tiles from there: exact against
@@ -186,10 +202,11 @@ def test_small_tile_boundary(sorter, kind, n, dist):
 
 
 @pytest.mark.parametrize("kind", ["u32", "f32", "u64", "i64", "f64"])
+@pytest.mark.usefixtures("either_path")
 def test_small_tile_boundary_values_and_64(sorter, kind):
-    """Argsort and pairs below and at FS_SMALL_TILE_KEYS (32-bit keys), and
-    64-bit sorts, argsort and pairs below and at FS_SMALL_TILE_KEYS64 (2^20):
-    exact against the oracle on both tile sizes."""
+    """Argsort and pairs below and at FS_SMALL_TILE_KEYS (32-bit keys) and
+    FS_SMALL_TILE_KEYS64 (2^20, 64-bit keys): exact against the oracle on both
+    tile sizes; 64-bit keys alone, which have one, at the same sizes."""
     limit = (1 << 20) if kind.endswith("64") else (1 << 21)
     for n in (limit - 1, limit):
         keys = make_keys(kind, n, "few" if n % 2 else "uniform", seed=150 + n % 89)
@@ -206,6 +223,7 @@ TILE_VARIANT = {("sort", False): "k32", ("sort", True): "k64", ("argsort", False
 
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("op", ["sort", "argsort", "pairs"])
+@pytest.mark.usefixtures("either_path")
 def test_tile_boundaries(sorter, kind, op):
     """Sizes at the edges of the kernel's own tile (read from the code object):
     one tile less one key, one tile, one tile plus one, two tiles plus one."""
@@ -222,18 +240,21 @@ def test_tile_boundaries(sorter, kind, op):
 
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("dist", ["zeros", "same", "sorted", "reverse", "few", "lowbits"])
+@pytest.mark.usefixtures("either_path")
 def test_sort_distributions(sorter, kind, dist):
     check_sort(sorter, kind, make_keys(kind, 100_003, dist, seed=7))
 
 
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("n", [2, 100, 4097, 65543, 1_000_000])
+@pytest.mark.usefixtures("either_path")
 def test_argsort_sizes(sorter, kind, n):
     check_argsort(sorter, kind, make_keys(kind, n, "uniform", seed=100 + n))
 
 
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("dist", ["same", "few", "lowbits", "reverse"])
+@pytest.mark.usefixtures("either_path")
 def test_argsort_ties(sorter, kind, dist):
     check_argsort(sorter, kind, make_keys(kind, 70_001, dist, seed=11))
 
@@ -241,6 +262,7 @@ def test_argsort_ties(sorter, kind, dist):
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("n", [2, 100, 4097, 1_000_000])
 @pytest.mark.parametrize("dist", ["uniform", "few"])
+@pytest.mark.usefixtures("either_path")
 def test_pairs(sorter, kind, n, dist):
     keys = make_keys(kind, n, dist, seed=200 + n)
     vals = np.random.Generator(np.random.PCG64(n)).integers(0, 1 << 32, size=n, dtype=np.uint32)
@@ -287,6 +309,7 @@ def test_deterministic(sorter):
 
 @pytest.mark.parametrize("dist", ["byte0", "byte1"])
 @pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.usefixtures("either_path")
 def test_single_pass_schedules(sorter, kind, dist):
     """Exactly one digit varies: the in-place sort runs one pass and moves the
     result to the caller's buffer through scratch (after the pass for the
@@ -303,6 +326,7 @@ def test_single_pass_schedules(sorter, kind, dist):
     check_buffer(sorter, kind, keys)
 
 
+@pytest.mark.usefixtures("either_path")
 def test_constant_digit_passes_skipped(sorter):
     keys = datagen.low20_u64(1_000_000, high=0x123456789AB)
     check_sort(sorter, "u64", keys)

@@ -511,7 +511,7 @@ DEV void bucket_pass_info(const FsArgs& a, uint64_t varying, uint32_t overs) {
 // ws: 2 * BLOCK / 64 words of LDS.  Every block reads the whole source, which
 // bounds it: 3 TB/s of a grid of 256 (8 keys per thread in flight: a tenth
 // faster).  With one region too small, us, against a sort without: u32, 1M keys
-// 1,420 / 54; f64, two levels, 2M 1,250 / 170, 16M 10,000 / 390, 128M 91,900 / 2,260.
+// 1,530 / 54; f64, two levels, 2M 1,260 / 170, 16M 10,100 / 380, 128M 91,800 / 2,120.
 template <bool K64, int BLOCK>
 DEV void gather_bucket(const FsArgs& a, uint64_t src_k, uint64_t src_v, bool fwd, uint32_t len, typename KeyT<K64>::type lo,
                        typename KeyT<K64>::type hi, bool last, uint64_t dst_k, uint64_t dst_v, uint32_t count, uint32_t* ws) {
@@ -1298,9 +1298,10 @@ DEV void sort_overflowed(const FsArgs& a, uint32_t start, uint32_t len, BlockSor
         if (last ? lo == ~(K)0 : hi - lo == (K)1) {      // one value: in order as it is
             const K v = xf_inv_apply<K64>(lo, xa, xb);
             for (uint32_t p = tid; p < len; p += BLOCK) gptr<K>(k2)[p] = v;
-        } else if (len <= (uint32_t)(BLOCK * ITEMS)) {
-            block_range_sort<K64, VALS, BLOCK, ITEMS>(a, k2, VALS ? v2 : 0u, false, len, k2, v2, L);
         } else {
+            // (also a bucket that LDS holds: the block sort, twice in the
+            // kernel, took registers from every other sort: u64 argsort 100,003
+            // keys 64.4 -> 65.9 us; here it saved 110 us of 1,530)
             slow_sort<K64, VALS, BLOCK, ITEMS>(a, k2, v2, false, k1, v1, k2, v2, k2, v2, len, L);
         }
     }

@@ -235,6 +235,7 @@ def launch_bytes(name, ksize, vbytes, n):
 
 FIRST_KINDS = ["histogram read", "fused first pass", "fused first pass, region overflow",
                "top-16 path", "top-16 path, region overflow (re-scatter)"]
+BUCKET_KINDS = [None, "one block", "buckets", "two levels of buckets"]
 
 
 def main():
@@ -310,6 +311,7 @@ def main():
     sorter.device_synchronize()
     t1 = time.perf_counter()
     first_kind = sorter.first_pass()             # how each sort began (same input every step)
+    bucket_kind = BUCKET_KINDS[sorter.last_bucket_info()[0]]
     log(f"bench: timed {K} sorts in {t1 - t0:.4f} s")
     # the last timed output (sorted, same multiset, stable for argsort and
     # pairs), checked below
@@ -383,9 +385,9 @@ def main():
         # constant digit's, or the re-scatter launch without an overflow)
         if b and e["avg_ms"] > 0 and b / (e["avg_ms"] / 1e3) / 1e9 <= HBM_PEAK_GBS:
             e["achieved_GBps"] = round(b / (e["avg_ms"] / 1e3) / 1e9, 1)
-    first_pass = {"kind": FIRST_KINDS[first_kind] if first_kind < len(FIRST_KINDS) else str(first_kind),
+    first_pass = {"kind": bucket_kind or (FIRST_KINDS[first_kind] if first_kind < len(FIRST_KINDS) else str(first_kind)),
                   "kernel": seq[0]["kernel"] if seq[0]["kernel"].startswith(("fs_first", "fs_upsweep"))
-                  else seq[1]["kernel"]}
+                  else seq[min(1, len(seq) - 1)]["kernel"]}
     sort_frac = sort_bytes * n / (ms_per_step / 1e3) / (HBM_PEAK_GBS * 1e9)
 
     # The slice API (sort_u32 on a host array: copy in, sort, copy out), reported

@@ -501,7 +501,7 @@ DEV void bucket_pass_info(const FsArgs& a, uint64_t varying, uint32_t overs) {
         }
     GLOBAL uint32_t* plan = gptr<uint32_t>(a.plan);
     st_agent(&plan[FS_PLAN_NPASSES], p);
-    st_agent(&plan[FS_PLAN_MASK], mask | FS_MASK_FUSED | FS_MASK_BUCKETS);
+    st_agent(&plan[FS_PLAN_MASK], mask | FS_MASK_BUCKETS);
     st_agent(&plan[FS_PLAN_RESCATTER], overs);
 }
 

@@ -799,8 +799,7 @@ static fs_status enqueue_buckets(fs_sorter* s, fs_op op, fs_key_type t, void* ke
     s->last_stream = st;
     s->pending = true;
     s->last_plan = (uint32_t*)(uintptr_t)sc.plan;
-    // (a sort of the fused range whose first pass scatters into regions)
-    s->last_fused = bp == BK_TWO_LEVELS && op == FS_OP_SORT && n >= FS_FUSED_MIN_KEYS;
+    s->last_fused = false;
     s->last_top16 = false;
     s->last_buckets = bp;
     return FS_OK;
@@ -835,14 +834,12 @@ static fs_status enqueue(fs_sorter* s, fs_op op, fs_key_type t, void* keys, uint
     fs_status r;
     BucketPath bp = bucket_path(s, op, t, n, no_alloc);
     if (bp == BK_BUCKETS || bp == BK_TWO_LEVELS) {
-        const std::string err = s->err;
+        std::string err;
+        err.swap(s->err);                                // (the last failing call's, unless this one fails)
         r = reserve_buckets(s, op, t, n, bp);
-        if (r == FS_ERR_OUT_OF_MEMORY || r == FS_ERR_INVALID_ARGUMENT) {
-            s->err = err;
-            bp = BK_NONE;
-        } else if (r != FS_OK) {
-            return r;
-        }
+        if (r == FS_ERR_OUT_OF_MEMORY || r == FS_ERR_INVALID_ARGUMENT) bp = BK_NONE;
+        else if (r != FS_OK) return r;
+        err.swap(s->err);
     }
     if (bp != BK_NONE) return enqueue_buckets(s, op, t, keys, vals, n, st, bp, no_alloc);
     const int var = sort_variant(s, op, t, n, no_alloc);

@@ -400,7 +400,8 @@ class GpuSorter:
         self._check(_load().fs_sorter_set_test_option(self._h, option, value))
 
     def first_pass(self):
-        """How the last sort began: FIRST_HISTOGRAM, FIRST_FUSED (the fused
+        """How the last sort began: FIRST_HISTOGRAM (also where buckets did it,
+        see last_bucket_info), FIRST_FUSED (the fused
         first pass, regions used), FIRST_FUSED_OVERFLOW (a region overflowed
         and the keys were re-scattered into exact regions, or every digit is
         constant), FIRST_TOP16 (the top-16

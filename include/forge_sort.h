@@ -293,13 +293,12 @@ fs_status fs_sorter_set_test_option(fs_sorter *s, fs_test_option opt, uint64_t v
 #define FS_TOP16_MIN_KEYS64 2097152u
 
 /* How the last completed sort began: 0 = the histogram read (argsort, pairs,
- * and keys-only sorts outside the fused range, also where buckets did them), 1 = the fused first pass of a
- * keys-only sort, its regions read by the next pass (or, f64, the partition
- * into buckets),
+ * and keys-only sorts outside the fused range), or no digit pass at all (see
+ * fs_last_bucket_info), 1 = the fused first pass of a keys-only sort, its
+ * regions read by the next pass,
  * 2 = the fused first pass after a region overflowed (the keys re-scattered
  * into exact regions by its second launch), or every digit constant (no
- * pass after it), or f64 keys of so few varying digits that the digit passes
- * sort them from the caller's buffer,
+ * pass after it),
  * 3 = the top-16 path (fused pass on the second-highest byte, its regions
  * read by the pass on the highest byte, then the local sort),
  * 4 = the top-16 path after a region of its fused pass overflowed (the keys

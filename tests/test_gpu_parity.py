@@ -519,12 +519,21 @@ def test_top16_sample_chooses(sorter, dist, expect):
 def test_top16_sample_chooses_64(sorter, kind, dist):
     """The same by size for 2^25 + 7 64-bit keys: u64/i64 uniform keys take
     the top-16 path, the others the LSD passes in the same launches (none
-    after the fused pass for equal keys); f64 keys always the fused LSD
-    passes (float keys do not take the top-16 launch sequence)."""
+    after the fused pass for equal keys); f64 keys two levels of buckets (the
+    digit passes where few digits vary) and, without buckets, always the fused
+    LSD passes (float keys do not take the top-16 launch sequence)."""
+    from forge_sort import BUCKETS_BY_SIZE, BUCKETS_NEVER, FIRST_HISTOGRAM, PATH_DIGITS, PATH_TWO_LEVELS, TEST_BUCKETS
     keys = make_keys(kind, (1 << 25) + 7, dist, seed=976)
     check_buffer(sorter, kind, keys)
     expect = {"uniform": (3,), "lowbits": (1,), "top8": (1,), "same": (2,)}[dist]
     if kind == "f64":
+        assert sorter.last_bucket_info() == (PATH_TWO_LEVELS if dist in ("uniform", "top8") else PATH_DIGITS, 0)
+        assert sorter.first_pass() == FIRST_HISTOGRAM
+        sorter.set_test_option(TEST_BUCKETS, BUCKETS_NEVER)
+        try:
+            check_buffer(sorter, kind, keys)
+        finally:
+            sorter.set_test_option(TEST_BUCKETS, BUCKETS_BY_SIZE)
         expect = (1, 2)
     assert sorter.first_pass() in expect
 

@@ -688,6 +688,14 @@ DEV void split_body(const FsArgs& a) {
     }
 
     const uint32_t stride = m / nb;
+    // Region of a bucket: room for its share of the samples plus six standard
+    // deviations, scaled to n.  budget: the keys that all of them can take.
+    auto region_keys = [&](uint32_t c) -> uint32_t {
+        const float room = (float)c + 6.0f * __builtin_sqrtf((float)c) + FS_BK_ROOM;
+        const uint32_t keys = ((uint32_t)(room * ((float)n / (float)m)) + 16u) & ~15u;
+        return keys > n ? (n + 15u) & ~15u : keys;
+    };
+    const uint32_t budget = L2 ? (uint32_t)(((uint64_t)n * a.bk2_room) >> 8) + 32u * nb : a.s1_keys;
     K least = 0, most = 0;
     block_fold<K64, false, BLOCK, ITEMS, false>(k, m, per, L, least, most);
     const K base = least;
@@ -724,14 +732,17 @@ DEV void split_body(const FsArgs& a) {
         __syncthreads();
         // A bucket's share of the samples: a quantile's where keys spread
         // within the splitters' groups, but up to all of both its splitters'
-        // groups where those are of a value each.  Where that is more, in any
-        // bucket, than a quantile's room holds but for once in 10^5, the
-        // samples are counted below.  (Counting them always took 1.6 us more:
-        // u32, 1M keys, 44.1 -> 45.8.)
+        // groups where those are of a value each.  A bucket for which that is
+        // more than a quantile's room holds, but for once in 10^5, is given
+        // all of it, and where the regions then take more than there is room
+        // for the samples are counted instead.  (Counted always: u32, 1M keys,
+        // 44.1 -> 45.8 us; wherever there was such a bucket: f64 pairs, normal,
+        // 1M keys, 72.1 -> 75.2.)
         if (tid < nb) {
             const uint32_t to = tid + 1u < nb ? L.starts[gi[tid + 1u] + 1u] : m;
-            if ((float)(to - L.starts[g]) > (float)stride + 2.0f * __builtin_sqrtf((float)stride) + 4.0f) L.flag = 1u;
-            share = stride;
+            share = to - L.starts[g];
+            if ((float)share > (float)stride + 2.0f * __builtin_sqrtf((float)stride) + 4.0f) L.flag = 1u;
+            else share = stride;
         }
         // The partition finds a key's bucket from its group: the splitters in
         // smaller groups, all below the key, then the few in its own.
@@ -754,7 +765,15 @@ DEV void split_body(const FsArgs& a) {
             tc[tid * TPT + j] = tx;
             tx += here;
         }
-        if (L.flag) {                                    // (uniform) count them, found as the partition finds its keys'
+        bool count = L.flag != 0u;                       // (uniform)
+        if (count) {
+            const uint32_t c16 = tid < nb ? region_keys(share) >> 4 : 0u;
+            const uint32_t before = block_exclusive_scan<BLOCK>(c16, L.wsum);
+            if (tid == nb - 1u) s_par[0] = before + c16;
+            __syncthreads();
+            count = s_par[0] > budget >> 4;
+        }
+        if (count) {                                     // found as the partition finds its keys'
             uint32_t* const sc = reinterpret_cast<uint32_t*>(&L.wcnt[0][0]);
             for (uint32_t i = tid; i < NB; i += BLOCK) sc[i] = 0u;
             __syncthreads();
@@ -845,24 +864,16 @@ DEV void split_body(const FsArgs& a) {
         }
     }
 
-    // Region of bucket j: room for its share of the sample plus six standard
-    // deviations, scaled to n.  (Should the regions not fit the S1 or S2 that
-    // the host sized for the largest layout, a bug, their buckets overflow:
-    // the sort stays exact.)
-    uint32_t cap = 0;
-    if (tid < nb) {
-        const float c = (float)share;
-        const float room = c + 6.0f * __builtin_sqrtf(c) + FS_BK_ROOM;
-        cap = ((uint32_t)(room * ((float)n / (float)m)) + 16u) & ~15u;
-        if (cap > n) cap = (n + 15u) & ~15u;
-    }
+    uint32_t cap = tid < nb ? region_keys(share) : 0u;
 #ifdef FS_FAULT_INJECTION
     if (a.fault == (L2 ? FS_FAULT_SMALL_REGIONS2 : FS_FAULT_SMALL_REGIONS) && tid == 1u) cap = 16u;
 #endif
-    const uint32_t rbase = block_exclusive_scan<BLOCK>(cap, L.wsum) + origin;
+    // (Should the regions not fit what the host sized for them, a bug, their
+    // buckets overflow: the sort stays exact.)
+    const uint32_t rbase = block_exclusive_scan<BLOCK>(cap, L.wsum);
     if (tid < nb) {
-        const bool fits = (uint64_t)rbase + cap <= (L2 ? a.s2_keys : a.s1_keys);
-        bases[tid] = fits ? rbase : 0u;
+        const bool fits = rbase + cap <= budget;
+        bases[tid] = fits ? origin + rbase : 0u;
         caps[tid] = fits ? cap : 0u;
         glb[tid] = lbs[tid];
     }

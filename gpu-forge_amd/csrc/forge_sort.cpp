@@ -468,9 +468,11 @@ static BucketShape bucket_shape(const fs_sorter* s, fs_op op, fs_key_type t, uin
     while ((1u << b.lm) > s->bk_samples) --b.lm;
     b.tile = (uint32_t)rows * s->bk_part_block;
     b.tiles = (uint32_t)((n + b.tile - 1) / b.tile);
+    // (one level: as for 4 samples a bucket, the most any smaller sort takes; two:
+    // a twentieth more, for buckets whose splitters lie in large groups)
     const double nb = (double)(1u << b.lnb);
-    b.s1_keys = (uint64_t)((double)n * bucket_room(nb, (double)(1u << b.lm)) + 32.0 * nb);
-    if (b.s1_keys < n) b.s1_keys = n;
+    const double room = two ? bucket_room(nb, (double)(1u << b.lm)) * 1.05 : bucket_room(1.0, 4.0);
+    b.s1_keys = (uint64_t)((double)n * room + 32.0 * nb);
     if (two) {
         const double nb2 = (double)(1u << b.lnb2);
         b.room2 = (uint32_t)(bucket_room(nb2, (double)(1u << b.lm2)) * 256.0) + 2u;
@@ -540,7 +542,8 @@ static fs_status reserve_buckets(fs_sorter* s, fs_op op, fs_key_type t, uint64_t
     const size_t kb = key_bytes(t);
     const BucketShape b = bucket_shape(s, op, t, n, two);
     const double nb = (double)(1u << b.lnb);
-    uint64_t s1 = b.s1_keys, s2 = n;
+    const uint64_t s1 = b.s1_keys;
+    uint64_t s2 = n;
     uint64_t tiles = b.tiles > (uint32_t)s->num_cus + 2u ? b.tiles : (uint32_t)s->num_cus + 2u;
     uint64_t lb = ((tiles + tiles / FS_LB_GROUP + 1) << b.lnb) * 4, digit_lb = 0;
     if (two) {
@@ -552,10 +555,8 @@ static fs_status reserve_buckets(fs_sorter* s, fs_op op, fs_key_type t, uint64_t
         digit_lb = lookback_bytes(s, op, t, n);                   // or the digit passes
         if (lb2 > lb) lb = lb2;
         if (digit_lb > lb) lb = digit_lb;
-    } else {
-        const uint64_t all = (uint64_t)((double)n * bucket_room(1.0, 4.0) + 32.0 * nb);
-        if (all > s1) s1 = all;
-        if (op == FS_OP_SORT) lb = 0;
+    } else if (op == FS_OP_SORT) {
+        lb = 0;
     }
     const bool v = op != FS_OP_SORT;
     const struct {

@@ -190,7 +190,7 @@ fs_status fs_encode_no_alloc(fs_sorter *s, fs_op op, fs_key_type type, void *dev
  * (the grow-only ensure_buffers*, lib.rs:1120-1289, done ahead of time), e.g.
  * before capturing a sort into a HIP graph.  Synchronous.
  * Bucket sorts need more scratch than the digit passes (f64, 128M keys:
- * 6.8 GB against 3.1): a sort whose bucket scratch cannot be allocated, or may not grow
+ * 7.0 GB against 3.1): a sort whose bucket scratch cannot be allocated, or may not grow
  * after a capture, takes the digit passes instead, and so do later ones that
  * need as much, until fs_reserve asks for it again. */
 fs_status fs_reserve(fs_sorter *s, fs_op op, fs_key_type type, uint64_t n);

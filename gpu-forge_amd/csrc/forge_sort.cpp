@@ -390,11 +390,11 @@ struct BucketLimit {
 };
 static BucketLimit bucket_limit(fs_op op, fs_key_type t) {
     const bool v = op != FS_OP_SORT;
-    // f64: always; with values, u64 and i64 keys from FS_BK2_MIN_64V on (alone
-    // they have the top-16 path)
+    // f64: always (with values from FS_BK2_MIN_F64V on); with values, u64 and i64
+    // keys from FS_BK2_MIN_64V on (alone they have the top-16 path)
     const bool f64 = t == FS_KEY_F64;
     if (key64(t))
-        return v ? BucketLimit{FS_BK_ONE_64V, FS_BK_MAX_64V, f64 ? 0u : FS_BK2_MIN_64V, FS_BK2_MAX_64V}
+        return v ? BucketLimit{FS_BK_ONE_64V, FS_BK_MAX_64V, f64 ? FS_BK2_MIN_F64V : FS_BK2_MIN_64V, FS_BK2_MAX_64V}
                  : BucketLimit{FS_BK_ONE_64, FS_BK_MAX_64, 0, f64 ? FS_BK2_MAX_64 : 0u};
     const bool f32 = t == FS_KEY_F32;
     return v ? BucketLimit{FS_BK_ONE_32V, f32 ? FS_BK_MAX_F32 : FS_BK_MAX_32V, 0, 0}

@@ -409,14 +409,16 @@
 // levels of buckets do (64-bit keys), by key width and values (V).  Where the
 // digit passes are as fast (us, buckets against passes, keys in place):
 // f32 keys with zeros, infinities, NaN and subnormals, which crowd the sample
-// and one bucket, 0.1M: 45 / 52, 0.22M: 61 / 53 (without them 1.1M: 48 / 67);
-// 32-bit integers, uniform, 1.1M: 46 / 66, of few values 41 / 45; with values
-// u32 argsort, 20 varying bits, 0.7M: 52 / 51 (0.5M: 42 / 49); 64-bit keys with
-// values of 20 bits, 1M: 64 / 66 (uniform 68 / 136).  Two levels: f64 from
-// there on (3M: sort 170 / 190, argsort 163 / 184; 128M: 2,496 / 4,567), but
-// u64 and i64 with values from FS_BK2_MIN_64V: those of few varying digits,
-// which go back to the passes, pay 8 to 10 us for the launches that find
-// nothing to do (12M pairs: 329 / 321 for 20 bits, 420 / 671 uniform).  The
+// and one bucket, 0.19M: 51 / 54, 0.22M: 64 / 54 (without them 1.1M: 48 / 67);
+// 32-bit integers, uniform, 1.1M: 46 / 66, of 20 bits 45 / 55; with values
+// u32 argsort, 20 varying bits, 0.7M: 53 / 53 (0.5M: 46 / 53); 64-bit keys with
+// values of 20 bits, 1M: 69 / 72 (uniform 68 / 142).  Two levels: f64 from
+// there on (1.51M: sort 153 / 159; 3M: sort 171 / 184, argsort 177 / 186; 128M:
+// 2,227 / 4,319), with values from FS_BK2_MIN_F64V, where the digit passes' small
+// tiles end (1.01M: argsort 142 to 152 / 138, pairs 146 / 143; 1.25M: argsort 147
+// / 153, pairs 150 / 160), but u64 and i64 with values from FS_BK2_MIN_64V: those of few
+// varying digits, which go back to the passes, pay 8 to 10 us for the launches
+// that find nothing to do (12M pairs: 273 / 265 for 20 bits, 385 / 625 uniform).  The
 // largest: 65,536 children of 3,072 keys (2,048 with values) each have room
 // for 1.4 times (1.7) their mean; those that need more are sorted by fs_rest_*.
 #ifndef FS_BK_ONE_32
@@ -435,6 +437,7 @@
 #ifndef FS_BK2_MIN_64V
 #define FS_BK2_MIN_64V 12000000u
 #endif
+#define FS_BK2_MIN_F64V FS_SMALL_TILE_KEYS64
 #ifndef FS_BK_MEAN
 #define FS_BK_MEAN 2048u
 #endif

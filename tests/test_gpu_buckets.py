@@ -123,11 +123,18 @@ def test_two_levels(sorter, op, kind, lnb, n):
         sorter.set_test_option(TEST_BUCKETS, BUCKETS_BY_SIZE)
 
 
-@pytest.mark.parametrize("kind,op,n", [("f64", "sort", 1_500_001), ("f64", "argsort", 1_000_001), ("i64", "pairs", 12_000_000)])
+@pytest.mark.parametrize("kind,op,n", [("f64", "sort", 1_500_001), ("f64", "argsort", 1_000_001), ("f64", "argsort", 1 << 20),
+                                       ("f64", "pairs", 1 << 20), ("i64", "pairs", 12_000_000)])
 @pytest.mark.parametrize("data", ["normal", "quantised", "narrow", "lone"])
 def test_two_levels_by_size(sorter, kind, op, n, data):
-    """The least sizes that take two levels by size."""
+    """The least sizes that take two levels by size, and one below (f64 with
+    values between the one level's largest and 2^20 keys)."""
+    from forge_sort import PATH_DIGITS, PATH_TWO_LEVELS
     check(sorter, op, kind, keys_of(kind, n, data, seed=7300))
+    if n == 1_000_001:
+        assert sorter.last_bucket_info()[0] == PATH_DIGITS
+    elif data == "normal":
+        assert sorter.last_bucket_info() == (PATH_TWO_LEVELS, 0)
 
 
 @pytest.mark.parametrize("kind,op,n,values,lnb", [

@@ -28,9 +28,9 @@
 //     fs_rest_*     children larger than a block and buckets of an overflowed
 //                   child, from a list, on a small grid
 //   The digit passes run before these and sort keys of few varying digits
-//   (FS_BK2_FEW_DIGITS); f64, 128M keys: 4,567 -> 2,496 us (part1 623, part2
-//   554, child 648, rest 96), u64 pairs, 16M: 906 -> 542 (143, 107, 143, 20).
-//   The partitions move 1 GB of reads and 1 GB of scattered writes of
+//   (FS_BK2_FEW_DIGITS); f64, 128M keys in place: 4,319 -> 2,227 us (part1 659,
+//   part2 574, child 677, rest 156), u64 pairs, 16M: 830 -> 471 (146, 106, 149,
+//   18).  The partitions move 1 GB of reads and 1 GB of scattered writes of
 //   f64 128M at 3.3 and 3.7 TB/s (a copy here: 4.75), the children's blocks
 //   are bound by their LDS passes.
 //

@@ -805,8 +805,13 @@ DEV void split_body(const FsArgs& a) {
         // Keys crowded in parts of the range, or many copies of some: the
         // sample sorted, by groups where those hold copies of one key each,
         // else by stable passes.  64-bit keys take the top FS_BK_SAMPLE_BITS
-        // bits of their range first (enough to order most samples), all of
-        // them when two neighbours are then out of order.
+        // bits of their range first.  Where two neighbours are then out of
+        // order, the quantiles' top bits alone are the splitters (in order, and
+        // below them exactly the samples of smaller top bits), unless two
+        // quantiles share them: then the rest is sorted too.  (u64 argsort,
+        // 995,000 keys, file and offset, most in few files: sorted twice, the
+        // sample took 93 of 146 us.)
+        K down = ~(K)0;                                  // the bits of a quantile that make a splitter
         bool done = a.xform == FS_XF_FLOAT &&
                     group_sort<K64, false, BLOCK, ITEMS>(k, m, group_map<K64>(least, most, true), per, L);
         if (!done) done = group_sort<K64, false, BLOCK, ITEMS>(k, m, group_map<K64>(least, most, false), per, L);
@@ -818,11 +823,15 @@ DEV void split_body(const FsArgs& a) {
             if (lo) {
                 bool bad = false;
                 for (uint32_t i = tid; i + 1u < m; i += BLOCK) bad |= L.keys[i] > L.keys[i + 1u];
-                if (tid == 0) L.flag = 0u;
+                const bool shared = tid >= 1u && tid < nb &&
+                                    L.keys[tid * stride] >> lo == L.keys[(tid - 1u) * stride] >> lo;
+                if (tid < 2u) s_par[tid] = 0u;
                 __syncthreads();
-                if (bad) L.flag = 1u;
+                if (bad) s_par[0] = 1u;
+                if (shared) s_par[1] = 1u;
                 __syncthreads();
-                const bool again = L.flag != 0u;
+                const bool again = s_par[0] && s_par[1];
+                if (s_par[0] && !again) down <<= lo;
                 __syncthreads();
                 if (again) {
 #pragma unroll
@@ -840,9 +849,9 @@ DEV void split_body(const FsArgs& a) {
         K q = 0;
         uint32_t emit = 0;
         if (tid >= 1u && tid < nb) {
-            q = L.keys[tid * stride];
-            const bool rep = tid > 1u && q == L.keys[(tid - 1u) * stride];
-            const bool dup = tid + 1u < nb && q == L.keys[(tid + 1u) * stride] && (K)(q + base) != ~(K)0;
+            q = L.keys[tid * stride] & down;
+            const bool rep = tid > 1u && q == (L.keys[(tid - 1u) * stride] & down);
+            const bool dup = tid + 1u < nb && q == (L.keys[(tid + 1u) * stride] & down) && (K)(q + base) != ~(K)0;
             emit = rep ? 0u : dup ? 2u : 1u;
         }
         for (uint32_t i = tid; i < NB; i += BLOCK) lbs[i] = i ? ~(K)0 : (K)0;

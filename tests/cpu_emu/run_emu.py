@@ -43,6 +43,11 @@ def keys_for(kind, n, dist, seed, tile=None):
         v = int(dist[5:])
         k = g.integers(0, v, size=n, dtype=BITS[kind])
         b = (k / (v - 1)).view(np.uint64) if kind == "f64" else k * BITS[kind](~BITS[kind](0) // BITS[kind](v))
+    elif dist == "records":         # (file index << 32 | offset), most keys in few files
+        files = np.minimum(g.random(n) ** (-1 / 0.3), 2e5).astype(np.uint64) - 1
+        b = (files << np.uint64(32)) | g.integers(0, 1 << 24, size=n, dtype=np.uint64)
+    elif dist == "cluster":         # half of the keys in a range that two quantiles' top bits share
+        b = np.where(g.random(n) < 0.5, g.integers(0, 1 << 10, size=n), g.integers(0, 1 << 50, size=n)).astype(np.uint64)
     elif dist.startswith("tenths"):  # f64: multiples of 0.1
         b = (g.integers(0, int(dist[6:]), size=n) * 0.1).view(np.uint64)
     elif dist == "same":

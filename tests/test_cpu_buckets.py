@@ -50,6 +50,19 @@ def test_emulated_buckets_of_repeated_values(emulator):  # noqa: F811
                        "bk_sort:u32:200000:steps400:1", "bk_pairs:u64:200000:steps300:2"], parallel=4, env={"EMU_CUS": "8"})
 
 
+SAMPLES = ["bk_sort:u64:3000:records:1", "bk_argsort:u64:3000:records:2", "bk_pairs:i64:3000:cluster:3",
+           "two_sort:u64:9000:records:4", "two_pairs:u64:6000:cluster:5", "bk2_sort:u64:4000:cluster:6"]
+
+
+def test_emulated_crowded_samples(emulator):  # noqa: F811
+    """Samples of 64-bit keys that their top bits do not order: splitters from
+    the top bits alone, or, where quantiles share them, from all bits."""
+    run_cases("small", SAMPLES, parallel=2)
+    run_cases("small", SAMPLES, env={"EMU_SCHED": "wave"}, parallel=2)
+    run_cases("prod", ["bk_argsort:u64:60000:records:1", "bk_sort:u64:60000:cluster:2", "two_pairs:u64:100000:records:3",
+                       "two_sort:u64:100000:cluster:4"], parallel=4, env={"EMU_CUS": "8"})
+
+
 @pytest.mark.parametrize("order", ["wave", "wave_rev"])
 def test_emulated_buckets_wave_serial(emulator, order):  # noqa: F811
     run_cases("small", CASES + TWO, timeout=900, env={"EMU_SCHED": order}, parallel=4)

@@ -49,6 +49,10 @@ def keys_of(kind, n, data, seed):
         b[n // 3 + 1] = ~u(0)
     elif data == "runs":                          # random keys, each five times in a row
         b = np.repeat(g.integers(0, 1 << (64 if wide else 32), size=n // 5 + 1, dtype=u, endpoint=False), 5)[:n]
+    elif data == "records":                       # (file index << 32 | offset), most keys in few files
+        b = (np.minimum(g.random(n) ** (-1 / 0.3), 2e5).astype(np.uint64) - u(1)) << u(32) | g.integers(0, 1 << 24, size=n, dtype=u)
+    elif data == "cluster":                       # half of them in a range that quantiles' top bits share
+        b = np.where(g.random(n) < 0.5, g.integers(0, 1 << 10, size=n), g.integers(0, 1 << 50, size=n)).astype(u)
     elif data == "sorted":
         b = np.sort(g.integers(0, 1 << (64 if wide else 32), size=n, dtype=u, endpoint=False))
     else:
@@ -154,6 +158,14 @@ def test_repeated_values(sorter, kind, op, n, values, lnb):
             assert sorter.last_bucket_info() == (PATH_TWO_LEVELS if lnb or n > 1_500_000 else PATH_BUCKETS, 0)
     finally:
         sorter.set_test_option(TEST_BUCKETS, BUCKETS_BY_SIZE)
+
+
+@pytest.mark.parametrize("op,n", [("sort", 1_500_000), ("argsort", 1_000_000), ("pairs", 8_193), ("pairs", 13_000_001)])
+@pytest.mark.parametrize("data", ["records", "cluster"])
+def test_crowded_samples(sorter, op, n, data):
+    """64-bit samples that their top bits do not order."""
+    check(sorter, op, "u64", keys_of("u64", n, data, seed=7600))
+    assert sorter.last_bucket_info()[1] == 0
 
 
 @pytest.mark.parametrize("kind,op", [("u32", "sort"), ("i32", "pairs"), ("f32", "argsort"), ("i64", "sort"),

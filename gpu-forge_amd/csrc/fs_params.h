@@ -412,7 +412,11 @@
 // and one bucket, 0.19M: 51 / 54, 0.22M: 64 / 54 (without them 1.1M: 48 / 67);
 // 32-bit integers, uniform, 1.1M: 46 / 66, of 20 bits 45 / 55; with values
 // u32 argsort, 20 varying bits, 0.7M: 53 / 53 (0.5M: 46 / 53); 64-bit keys with
-// values of 20 bits, 1M: 69 / 72 (uniform 68 / 142).  Two levels: f64 from
+// values of 20 bits, 1M: 69 / 72 (uniform 68 / 142).  Slower than the passes
+// near the limits where skewed integers crowd the sample, which its block then
+// sorts by stable passes: u32 Zipf ranks 0.8M 62 / 54, 1.1M 66 / 58, argsort
+// 0.6M 60 / 54 (uniform 44 / 61); u64 (file, offset) keys with values 1.0M
+// 120 / 109 (0.8M 94 / 100; alone 1.5M 124 / 124).  Two levels: f64 from
 // there on (1.51M: sort 153 / 159; 3M: sort 171 / 184, argsort 177 / 186; 128M:
 // 2,227 / 4,319), with values from FS_BK2_MIN_F64V, where the digit passes' small
 // tiles end (1.01M: argsort 142 to 152 / 138, pairs 146 / 143; 1.25M: argsort 147
